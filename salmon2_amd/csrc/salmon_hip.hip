@@ -15,6 +15,8 @@
 //                     the sum of taylor.f90:53-114
 //   k_nl_scatter      the KB scatter of zpseudo (nonlocal_potential.f90:370-378) as a
 //                     deterministic per-point gather over a point->(atom, j) inverse map
+//   k_taylor_small    a whole orbital per block for small grids: the Taylor step (or H psi) from LDS;
+//   k_current_small   its current (small_grid.h)
 //   k_density_*       calc_density (density_matrix.f90:150-230)
 //   k_current_*       stencil_current + calc_current (density_matrix.f90:240-530)
 //   k_dipole_part/_sum calc_dip (src/rt/dip.f90:114-225)
@@ -29,6 +31,7 @@
 #include <algorithm>
 #include <atomic>
 #include <climits>
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -1967,22 +1970,24 @@ __device__ __forceinline__ void current_orb_body(const CurFinArgs &a, int bx, in
 
 __global__ __launch_bounds__(kBlock) void k_current_orb(CurFinArgs a, int ispin) { current_orb_body(a, blockIdx.x, ispin); }
 
-// Sum of the orbital contributions in (ik, io) order, divided by N_grid
-// (contributions staged through LDS in chunks so the serial sum reads LDS).
+// Sum of the orbital contributions divided by N_grid: one wave per component, lanes on every 64th
+// orbital with 8 loads in flight, combined over the lanes in a fixed tree.
 __device__ __forceinline__ void current_sum_body(const CurFinArgs &a, int ispin) {
-  __shared__ double sh[3 * 1024];
   const int M = a.no * a.nk;
-  const double *cs = a.contrib + 3 * (size_t)M * ispin;  // this spin's contributions
-  double w4 = 0.0;
-  for (int m0 = 0; m0 < M; m0 += 1024) {
-    const int n = min(1024, M - m0);
-    for (int i = threadIdx.x; i < 3 * n; i += kBlock) sh[i] = cs[3 * (size_t)m0 + i];
-    __syncthreads();
-    if (threadIdx.x < 3)
-      for (int mm = 0; mm < n; ++mm) w4 = w4 + sh[3 * mm + threadIdx.x];
-    __syncthreads();
+  const int d = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  if (d >= 3) return;
+  const double *cs = a.contrib + 3 * (size_t)M * ispin + d;  // this spin's contributions
+  double acc = 0.0;
+  for (int m0 = lane; m0 < M; m0 += 64 * 8) {
+    double v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = m0 + 64 * u < M ? cs[3 * (size_t)(m0 + 64 * u)] : 0.0;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) acc += v[u];
   }
-  if (threadIdx.x < 3) a.curr[3 * ispin + threadIdx.x] = w4 * a.inv_ngrid;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+  if (lane == 0) a.curr[3 * ispin + d] = acc * a.inv_ngrid;
 }
 
 __global__ __launch_bounds__(kBlock) void k_current_sum(CurFinArgs a, int ispin) { current_sum_body(a, ispin); }
@@ -2057,6 +2062,8 @@ __device__ __forceinline__ void dipole_sum_body(const DipArgs &a) {
 }
 
 __global__ __launch_bounds__(256) void k_dipole_sum(DipArgs a) { dipole_sum_body(a); }
+
+#include "small_grid.h"
 
 // ---------------------------------------------------------------------------
 // Hartree potential: poisson_ft (src/poisson/poisson_periodic.f90:23-242) as six
@@ -2386,6 +2393,7 @@ struct salmon_hip_ctx {
   // (whole plane when it fits 256 threads), 0 = y tiles, 1 = whole plane; mid_nzt 0 = rule
   int tile_plane = -1, mid_nzt = 0;
   bool tile8 = true;  // stencil_tile8 for the mixed middle terms where the shape allows it
+  bool small_grid = true;  // k_taylor_small where the grid fits (salmon_hip_set_launch_shape turns it off)
   bool tilez = true;  // stencil_tilez for the FP64 ones and the mixed first term (before stencil_tile8)
   // salmon_hip_set_skip: device flag read by the launches of hpsi/taylor, density and the
   // potential update (they do nothing while it is set); null = none
@@ -3210,6 +3218,147 @@ static int launch_hpsi(salmon_hip_t c, int kind, const void *in, void *hout, boo
   return 0;
 }
 
+}  // extern "C"
+
+// ---------------------------------------------------------------------------
+// Whole-orbital launches for small grids (small_grid.h)
+// ---------------------------------------------------------------------------
+constexpr size_t kSmallLds = 156 * 1024;  // of the CU's 160 KB
+
+// The launch of k_taylor_small for a handle's grid: template class (largest block, waves per SIMD that
+// the registers allow), planes per thread, z chunks per column, threads, waves per atom.
+struct SmallShape {
+  int cls = -1, ppt = 0, zchunks = 0, bs = 0, nsub = 1;
+  size_t lds = 0;
+};
+
+// Classes with the most planes per thread that each one's registers hold (more spill).
+struct SmallClass {
+  int bsmax, minw, pptmax;
+};
+constexpr SmallClass kSmallClass[] = {{512, 2, 8}, {512, 4, 4}, {768, 3, 10}, {1024, 4, 4}};
+
+// The fewest wave-planes (waves x planes per thread, idle lanes included: the stencil is bound by the
+// CU's LDS reads), weighted by what the launch needs beside: with up to two orbitals per CU the
+// block's own latency counts, and the class with 256 registers issues its table loads ahead of their
+// use; with more, blocks that share a CU hide each other's barriers and loads.  Measured (one Taylor
+// step of order 4, 8 atoms): 16^3, 16 orbitals: 51.6 us as {512, 2} with 8 planes, 56.7 as {768, 3},
+// 73.8 as {512, 4}; 12^3, 1024 orbitals: 94 us as {512, 4} with 4 planes, 117 as {768, 3} with 3,
+// 126 as {512, 2} with 4.
+static SmallShape small_shape(const salmon_hip_ctx *c) {
+  SmallShape best;
+  const int ncol = c->nx * c->ny;
+  double low = 0.0;
+  for (int k = 0; k < 4; ++k) {
+    const SmallClass &K = kSmallClass[k];
+    for (int ppt = 2; ppt <= K.pptmax; ++ppt) {
+      SmallShape s;
+      s.cls = k;
+      s.ppt = ppt;
+      s.zchunks = (c->nz + ppt - 1) / ppt;
+      if ((size_t)ncol * s.zchunks > (size_t)K.bsmax) continue;
+      // at least one wave for each of the first eight atoms
+      const int waves = std::max((ncol * s.zchunks + 63) / 64, std::min(c->natom, 8));
+      s.bs = 64 * waves;
+      if (c->natom > 0) s.nsub = std::max(1, waves / c->natom);
+      s.lds = sizeof(double2) * (c->osz + 2 * (size_t)c->nlma * s.nsub + 2 * (size_t)c->ntp_shared);
+      if (s.lds > kSmallLds) continue;
+      double cost = (double)waves * ppt;
+      if (c->norb <= 512) {
+        cost *= K.minw == 2 ? 1.0 : 1.15;
+      } else {
+        const int blocks = std::min(std::max(1, 4 * K.minw / waves), (int)std::max<size_t>(1, (160 * 1024) / s.lds));
+        cost *= std::sqrt(16.0 / std::min(16, blocks * waves));
+      }
+      if (best.cls < 0 || cost < low) {
+        best = s;
+        low = cost;
+      }
+    }
+  }
+  return best;
+}
+
+// FP64 handles whose orbital block fits one CU's LDS; a launch shape set by hand
+// (salmon_hip_set_launch_shape) and the overlapped projections select the per-term kernels.
+static bool small_fits(const salmon_hip_ctx *c) {
+  if (!c->small_grid || c->overlap || c->prec != SALMON_HIP_PREC_FP64) return false;
+  if (c->osz * sizeof(double2) > kSmallLds || (size_t)c->nx * c->ly * sizeof(double2) > 65536 || c->ntp_shared > 65534)
+    return false;
+  return small_shape(c).cls >= 0;
+}
+
+static SmallArgs small_args(salmon_hip_t c, const void *psi, void *out, void *h1) {
+  SmallArgs a;
+  memset(&a, 0, sizeof(a));
+  a.psi = (const double2 *)psi;
+  a.out = (double2 *)out;
+  a.h1 = (double2 *)h1;
+  a.V = c->d_V;
+  a.kpar = c->d_kpar;
+  a.zekr = c->d_zekr;
+  a.zent = c->d_zent;
+  a.jidx = c->d_jidx;
+  a.mps = c->d_mps;
+  a.atom_lma = c->d_atom_lma;
+  a.jexcl = c->d_jexcl;
+  a.tp_shared = c->d_tp_shared;
+  a.pt_lma = c->d_pt_lma;
+  a.rinv = c->d_rinv;
+  for (int i = 0; i < 12; ++i) a.lap[i] = -0.5 * c->coef_lap[i];
+  a.osz = c->osz;
+  a.nx = c->nx; a.ny = c->ny; a.nz = c->nz; a.ly = c->ly;
+  a.nspin = c->nspin; a.nb = c->nb; a.nk = c->nk;
+  a.nterm = a.first = 1;
+  a.natom = c->natom; a.nps = c->nps; a.nlma = c->nlma;
+  a.nent = c->nent; a.cmax = c->cmax; a.ntp_shared = c->ntp_shared;
+  a.skip = c->d_skip;
+  return a;
+}
+
+template <int PPT, int BSMAX, int MINW>
+static int launch_taylor_small_t(salmon_hip_ctx *c, const SmallShape &s, const SmallArgs &a, hipEvent_t e0, hipEvent_t e1) {
+  static std::atomic<unsigned long long> attr_dev{0};
+  if (int rc = lds_attr((const void *)k_taylor_small<PPT, BSMAX, MINW>, attr_dev, kSmallLds)) return rc;
+  hipExtLaunchKernelGGL((k_taylor_small<PPT, BSMAX, MINW>), dim3((unsigned)c->norb), dim3(s.bs), s.lds, c->stream, e0, e1, 0,
+                        a);
+  LAUNCHCHK("k_taylor_small");
+  return 0;
+}
+
+template <int K>
+static int launch_taylor_small_c(salmon_hip_ctx *c, const SmallShape &s, const SmallArgs &a, hipEvent_t e0, hipEvent_t e1) {
+  constexpr int BSMAX = kSmallClass[K].bsmax, MINW = kSmallClass[K].minw, PM = kSmallClass[K].pptmax;
+  switch (s.ppt) {
+    case 2: return launch_taylor_small_t<2, BSMAX, MINW>(c, s, a, e0, e1);
+    case 3: return launch_taylor_small_t<3, BSMAX, MINW>(c, s, a, e0, e1);
+    case 4: return launch_taylor_small_t<4, BSMAX, MINW>(c, s, a, e0, e1);
+    case 5: return launch_taylor_small_t<std::min(5, PM), BSMAX, MINW>(c, s, a, e0, e1);
+    case 6: return launch_taylor_small_t<std::min(6, PM), BSMAX, MINW>(c, s, a, e0, e1);
+    case 7: return launch_taylor_small_t<std::min(7, PM), BSMAX, MINW>(c, s, a, e0, e1);
+    case 8: return launch_taylor_small_t<std::min(8, PM), BSMAX, MINW>(c, s, a, e0, e1);
+    case 9: return launch_taylor_small_t<std::min(9, PM), BSMAX, MINW>(c, s, a, e0, e1);
+    default: return launch_taylor_small_t<std::min(10, PM), BSMAX, MINW>(c, s, a, e0, e1);
+  }
+}
+
+static int launch_taylor_small(salmon_hip_ctx *c, int kind, SmallArgs &a) {
+  const SmallShape s = small_shape(c);
+  a.zchunks = s.zchunks;
+  a.nsub = s.nsub;
+  c->pre_state = 0;
+  hipEvent_t e0, e1;
+  prof_events(c, kind, &e0, &e1);
+  switch (s.cls) {
+    case 0: return launch_taylor_small_c<0>(c, s, a, e0, e1);
+    case 1: return launch_taylor_small_c<1>(c, s, a, e0, e1);
+    case 2: return launch_taylor_small_c<2>(c, s, a, e0, e1);
+    default: return launch_taylor_small_c<3>(c, s, a, e0, e1);
+  }
+}
+
+extern "C" {
+
 static int ready(salmon_hip_t c) {
   if (!c->have_V) return fail(SALMON_HIP_ESTATE, "V_local not set");
   if (!c->have_k) return fail(SALMON_HIP_ESTATE, "update_kvector (vec_Ac) not set");
@@ -3220,6 +3369,13 @@ int salmon_hip_hpsi(salmon_hip_t c, const void *tpsi, void *htpsi) {
   if (int rc = check(c)) return rc;
   if (!tpsi || !htpsi || tpsi == htpsi) return fail(SALMON_HIP_EINVAL, "tpsi/htpsi invalid or aliased");
   if (int rc = ready(c)) return rc;
+  // one application alone: the per-term kernels' three launches are worth their cost above about a
+  // thousand orbitals (16^3, 1024 orbitals: 93 us in one launch, 112 per term; 15x17x14, 1600
+  // orbitals: 150 and 126; 12x12x24, 2048 orbitals: 171 and 158)
+  if (c->norb <= 1024 && small_fits(c)) {
+    SmallArgs a = small_args(c, tpsi, nullptr, htpsi);
+    return launch_taylor_small(c, SALMON_HIP_KERNEL_HPSI0, a);
+  }
   if (c->natom > 0)
     if (int rc = launch_proj(c, tpsi, 1)) return rc;
   return launch_hpsi(c, SALMON_HIP_KERNEL_HPSI0, tpsi, htpsi, false, nullptr, 0, nullptr);
@@ -3264,9 +3420,32 @@ int salmon_hip_set_precision(salmon_hip_t c, int mode) {
   return 0;
 }
 
-// first = 1: the whole chain; first = 2: h_1 = sshtpsi is already current
+// h_1 += dv psi (salmon_hip_taylor_reuse)
+}  // extern "C"
+template <typename TH>
+static int launch_vshift(salmon_hip_ctx *c, void *h1, const void *psi, const double *dv) {
+  const size_t ntot = c->osz * c->norb;
+  const dim3 grid((unsigned)((ntot + kBlock - 1) / kBlock));
+  hipLaunchKernelGGL(k_vshift<TH>, grid, dim3(kBlock), 0, c->stream, (TH *)h1, (const double2 *)psi, dv, c->osz, c->nx,
+                     c->ny, c->ly, c->nz, c->nspin, ntot, c->d_skip);
+  LAUNCHCHK("k_vshift");
+  return 0;
+}
+extern "C" {
+
+// first = 1: the whole chain; first = 2: h_1 = sshtpsi is H psi of a previous call, to be shifted by dv
 static int taylor_fp64(salmon_hip_t c, const double *zc, int n_hamil, void *tspsi_in, void *tspsi_out, void *sshtpsi,
-                       int first) {
+                       int first, const double *dv = nullptr) {
+  if (small_fits(c)) {
+    SmallArgs a = small_args(c, tspsi_in, tspsi_out, n_hamil >= 2 ? sshtpsi : nullptr);
+    for (int n = 0; n < n_hamil; ++n) a.zc[n] = make_double2(zc[2 * n], zc[2 * n + 1]);
+    a.nterm = n_hamil;
+    a.first = first;
+    a.dv = dv;
+    return launch_taylor_small(c, SALMON_HIP_KERNEL_HPSI_TAYLOR_LAST, a);
+  }
+  if (dv)
+    if (int rc = launch_vshift<double2>(c, sshtpsi, tspsi_in, dv)) return rc;
   // h_1 = H psi -> sshtpsi, h_2 .. h_{N-1} -> internal scratch
   const int nscr = std::max(0, n_hamil - 2);
   while ((int)c->tscr.size() < nscr) {
@@ -3316,17 +3495,11 @@ int salmon_hip_taylor_reuse(salmon_hip_t c, const double *zc, int n_hamil, void 
   void *h1 = mixed ? (c->tscr32.empty() ? nullptr : (void *)c->tscr32[0]) : sshtpsi;
   if (!h1 || (!mixed && (sshtpsi == tspsi_in || sshtpsi == tspsi_out)))
     return fail(SALMON_HIP_ESTATE, "taylor_reuse needs H psi of a previous taylor call (sshtpsi, or the FP32 chain)");
-  const size_t ntot = c->osz * c->norb;
-  const dim3 grid((unsigned)((ntot + kBlock - 1) / kBlock));
-  if (mixed)
-    hipLaunchKernelGGL(k_vshift<float2>, grid, dim3(kBlock), 0, c->stream, (float2 *)h1, (const double2 *)tspsi_in,
-                       dv_dev, c->osz, c->nx, c->ny, c->ly, c->nz, c->nspin, ntot, c->d_skip);
-  else
-    hipLaunchKernelGGL(k_vshift<double2>, grid, dim3(kBlock), 0, c->stream, (double2 *)h1, (const double2 *)tspsi_in,
-                       dv_dev, c->osz, c->nx, c->ny, c->ly, c->nz, c->nspin, ntot, c->d_skip);
-  LAUNCHCHK("k_vshift");
-  if (mixed) return taylor_mixed(c, zc, n_hamil, tspsi_in, tspsi_out, 2);
-  return taylor_fp64(c, zc, n_hamil, tspsi_in, tspsi_out, sshtpsi, 2);
+  if (mixed) {
+    if (int rc = launch_vshift<float2>(c, h1, tspsi_in, dv_dev)) return rc;
+    return taylor_mixed(c, zc, n_hamil, tspsi_in, tspsi_out, 2);
+  }
+  return taylor_fp64(c, zc, n_hamil, tspsi_in, tspsi_out, sshtpsi, 2, dv_dev);
 }
 
 
@@ -3405,6 +3578,7 @@ int salmon_hip_set_launch_shape(salmon_hip_t c, int whole_plane, int z_chunks) {
   if (whole_plane < -1 || whole_plane > 1 || z_chunks < 0) return fail(SALMON_HIP_EINVAL, "launch shape");
   c->tile_plane = whole_plane;
   c->mid_nzt = z_chunks;
+  c->small_grid = whole_plane == -1 && z_chunks == 0;
   return 0;
 }
 
@@ -3496,8 +3670,51 @@ static CurFinArgs curfin_args(salmon_hip_t c, const double *vec_Ac, const double
   return f;
 }
 
+static size_t small_current_lds(const salmon_hip_ctx *c, int nsub) {
+  return sizeof(double2) * c->osz + sizeof(double) * (8 * (size_t)c->nlma * nsub + 4 * (kSmallCurBs / 64));
+}
+
+// Whole-orbital current of a small grid; false where its moments do not fit the LDS beside the orbital.
+static bool small_current_args(salmon_hip_t c, const void *psi, const CurFinArgs &f, SmallCurArgs &a) {
+  a.f = f;
+  a.psi = (const double2 *)psi;
+  a.zekr = c->d_zekr;
+  a.rxyz = c->d_rxyz;
+  a.jidx = c->d_jidx;
+  a.mps = c->d_mps;
+  a.atom_lma = c->d_atom_lma;
+  memcpy(a.coef_nab, c->coef_nab, sizeof(a.coef_nab));
+  a.osz = c->osz;
+  a.nx = c->nx; a.ny = c->ny; a.nz = c->nz; a.ly = c->ly;
+  a.natom = c->natom; a.nps = c->nps; a.nlma = c->nlma;
+  a.nsub = c->natom > 0 ? std::max(1, kSmallCurBs / 64 / c->natom) : 1;
+  return small_current_lds(c, a.nsub) <= kSmallLds;
+}
+
+static int launch_current_small(salmon_hip_t c, const SmallCurArgs &a) {
+  static std::atomic<unsigned long long> attr_dev{0};
+  if (int rc = lds_attr((const void *)k_current_small, attr_dev, kSmallLds)) return rc;
+  hipEvent_t e0, e1;
+  prof_events(c, SALMON_HIP_KERNEL_PROJ_CURRENT, &e0, &e1);
+  hipExtLaunchKernelGGL(k_current_small, dim3((unsigned)c->norb), dim3(kSmallCurBs), small_current_lds(c, a.nsub), c->stream,
+                        e0, e1, 0, a);
+  LAUNCHCHK("k_current_small");
+  return 0;
+}
+
 static int current_impl(salmon_hip_t c, const double *vec_Ac, const double *actab, const int *itt, const void *psi,
                         double *curr_dev, int tmax = 0, bool next = false) {
+  if (!actab && small_fits(c)) {
+    SmallCurArgs a;
+    if (small_current_args(c, psi, curfin_args(c, vec_Ac, actab, itt, curr_dev, tmax), a)) {
+      if (int rc = launch_current_small(c, a)) return rc;
+      for (int is = 0; is < c->nspin; ++is) {
+        hipLaunchKernelGGL(k_current_sum, dim3(1), dim3(kBlock), 0, c->stream, a.f, is);
+        LAUNCHCHK("k_current_sum");
+      }
+      return 0;
+    }
+  }
   const CurArgs a = cur_args(c, psi);
   // the projector moments run on the side stream, overlapping the local part
   if (c->natom > 0)
@@ -3555,9 +3772,11 @@ int salmon_hip_current_next(salmon_hip_t c, const double *vec_Ac, const void *ps
   LAUNCHCHK("k_update_kvector");
   c->staged = true;
   memcpy(c->staged_A, vec_Ac_next, sizeof(c->staged_A));
-  if (int rc = current_impl(c, vec_Ac, nullptr, nullptr, psi, curr_dev, 0, true)) return rc;
-  c->pre_state = 1;
-  c->pre_psi = psi;
+  // (the whole-orbital current of a small grid leaves the projection to the whole-orbital Taylor step)
+  const void *pre = small_fits(c) ? nullptr : psi;
+  if (int rc = current_impl(c, vec_Ac, nullptr, nullptr, psi, curr_dev, 0, pre != nullptr)) return rc;
+  c->pre_state = pre ? 1 : 0;
+  c->pre_psi = pre;
   return 0;
 }
 
