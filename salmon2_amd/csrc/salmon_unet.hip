@@ -97,7 +97,12 @@ struct ConvArgs {
 // SK = false: each wave takes its own 16 points and the whole K; SK = true (coarse levels, few
 // points): the four waves of a block share 16 points and take every fourth K step each, and wave
 // 0 adds the four partial sums in a fixed order (deterministic).
-template <int NT, bool SK>
+//
+// CI = input channels / 16.  Bound by the latency of the operand loads (a wave has 2 (1 + NT) KB of
+// operands per K step and 14 to 81 steps): U steps' loads are issued together, the next group's while the
+// MFMAs of a group run, and the channel count is a constant so that a step's addresses cost no division.
+// With one step ahead and runtime divisions a 16 -> 16 layer took 12.7 us at 32^3, now 6.2.
+template <int NT, bool SK, int CI>
 __global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int p0 = (SK ? blockIdx.x : blockIdx.x * 4 + wave) * 16;
@@ -108,8 +113,7 @@ __global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
   const int pp = pv ? p : 0;
   const int nx = a.nx, ny = a.ny, nz = a.nz;
   const int x = pp % nx, y = (pp / nx) % ny, z = pp / (nx * ny);
-  const int ci = a.c1 + a.c2;
-  const int K = 27 * ci;
+  constexpr int ci = 16 * CI, K = 27 * ci;
   f4v acc[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) acc[t] = f4v{0.f, 0.f, 0.f, 0.f};
@@ -117,35 +121,50 @@ __global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
   // (branch-free: what lies outside the point range or past K is read from a zero buffer, so
   // every lane issues the same loads and each wait can sit at the MFMA that uses the data)
   auto load = [&](int f0, s8v &av, s8v (&bv)[NT]) __attribute__((always_inline)) {
-    const int f = f0 + 8 * kq;
+    const unsigned f = f0 + 8 * kq;
     const bool fv = f < K;
-    const int fc = fv ? f : 0;
+    const unsigned fc = fv ? f : 0;
     const int tap = fc / ci, c = fc - tap * ci;
     const int dz = tap / 9 - 1, dy = (tap / 3) % 3 - 1, dx = tap % 3 - 1;
-    const int xn = (x + dx + nx) % nx, yn = (y + dy + ny) % ny, zn = (z + dz + nz) % nz;
-    const size_t pn = (size_t)xn + (size_t)nx * ((size_t)yn + (size_t)ny * zn);
-    const size_t ph = a.up1 ? (size_t)(xn >> 1) + (size_t)(nx >> 1) * ((size_t)(yn >> 1) + (size_t)(ny >> 1) * (zn >> 1))
-                            : pn;
-    const bf16_t *src = c < a.c1 ? a.src1 + ph * a.c1 + c : a.src2 + pn * a.c2 + (c - a.c1);
+    int xn = x + dx, yn = y + dy, zn = z + dz;
+    xn += xn < 0 ? nx : 0;
+    xn -= xn >= nx ? nx : 0;
+    yn += yn < 0 ? ny : 0;
+    yn -= yn >= ny ? ny : 0;
+    zn += zn < 0 ? nz : 0;
+    zn -= zn >= nz ? nz : 0;
+    const int pn = xn + nx * (yn + ny * zn);
+    const int ph = a.up1 ? (xn >> 1) + (nx >> 1) * ((yn >> 1) + (ny >> 1) * (zn >> 1)) : pn;
+    const bf16_t *src = c < a.c1 ? a.src1 + (size_t)ph * a.c1 + c : a.src2 + (size_t)pn * a.c2 + (c - a.c1);
     av = *(const s8v *)((fv && pv) ? src : a.zero);
-    const bf16_t *wt = fv ? a.w + (size_t)tap * a.co * ci + c : a.zero;
+    const bf16_t *wt = fv ? a.w + (size_t)(tap * a.co) * ci + c : a.zero;
 #pragma unroll
-    for (int t = 0; t < NT; ++t) bv[t] = *(const s8v *)(wt + (size_t)(t * 16 + row) * ci);
+    for (int t = 0; t < NT; ++t) bv[t] = *(const s8v *)(wt + (t * 16 + row) * ci);
   };
-  // two operand sets: the loads of step f0 + 32 are in flight while the MFMAs of step f0 run
-  // (the accumulation order over f0 is unchanged)
-  constexpr int kst = SK ? 4 * 32 : 32;  // this wave's K steps: fs, fs + kst, ...
+  // this wave's K steps fs, fs + kst, ... in two sets of U operands (steps past the end multiply zeros
+  // and are left out); the accumulation order is that of the steps
+  constexpr int kst = SK ? 4 * 32 : 32;
+  constexpr int U = NT == 1 ? 7 : NT == 2 ? 5 : NT == 3 ? 4 : NT == 4 ? 3 : 2;
   const int fs = SK ? 32 * wave : 0;
-  s8v avA, avB, bvA[NT], bvB[NT];
-  load(fs, avA, bvA);
-  for (int f0 = fs; f0 < K; f0 += 2 * kst) {
-    if (f0 + kst < K) load(f0 + kst, avB, bvB);
+  s8v av[2][U], bv[2][U][NT];
+  auto load_group = [&](int f0, s8v (&A)[U], s8v (&B)[U][NT]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int t = 0; t < NT; ++t) acc[t] = mfma32(avA, bvA[t], acc[t]);
-    if (f0 + kst >= K) break;
-    if (f0 + 2 * kst < K) load(f0 + 2 * kst, avA, bvA);
+    for (int u = 0; u < U; ++u) load(f0 + kst * u, A[u], B[u]);
+  };
+  auto mfma_group = [&](int f0, s8v (&A)[U], s8v (&B)[U][NT]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int t = 0; t < NT; ++t) acc[t] = mfma32(avB, bvB[t], acc[t]);
+    for (int u = 0; u < U; ++u)
+      if (f0 + kst * u < K)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[t] = mfma32(A[u], B[u][t], acc[t]);
+  };
+  load_group(fs, av[0], bv[0]);
+  for (int f0 = fs; f0 < K; f0 += 2 * U * kst) {
+    if (f0 + U * kst < K) load_group(f0 + U * kst, av[1], bv[1]);
+    mfma_group(f0, av[0], bv[0]);
+    if (f0 + U * kst >= K) break;
+    if (f0 + 2 * U * kst < K) load_group(f0 + 2 * U * kst, av[0], bv[0]);
+    mfma_group(f0 + U * kst, av[1], bv[1]);
   }
   if constexpr (SK) {
     __shared__ f4v red[3][NT][64];
@@ -563,18 +582,25 @@ int launch_conv(salmon_unet *u, const bf16_t *s1, int c1, int up1, const bf16_t 
   // fewer 64-point blocks than CUs: split K over the four waves of 16-point blocks
   const bool sk = (a.npts + 63) / 64 < 256;
   const unsigned nb = (unsigned)(sk ? (a.npts + 15) / 16 : (a.npts + 63) / 64);
-#define CONV_LAUNCH(NTv)                                                                   \
-  do {                                                                                     \
-    if (sk) hipLaunchKernelGGL((k_conv<NTv, true>), dim3(nb), dim3(256), 0, u->stream, a); \
-    else hipLaunchKernelGGL((k_conv<NTv, false>), dim3(nb), dim3(256), 0, u->stream, a);   \
-  } while (0)
-  switch (co / 16) {
-    case 1: CONV_LAUNCH(1); break;
-    case 2: CONV_LAUNCH(2); break;
-    case 3: CONV_LAUNCH(3); break;
-    case 4: CONV_LAUNCH(4); break;
-    case 6: CONV_LAUNCH(6); break;
-    default: return ufail(SALMON_HIP_EUNSUPPORTED, "conv with %d output channels", co);
+#define CONV_LAUNCH(NTv, CIv)                                                                   \
+  case 16 * NTv + CIv:                                                                          \
+    if (sk) hipLaunchKernelGGL((k_conv<NTv, true, CIv>), dim3(nb), dim3(256), 0, u->stream, a); \
+    else hipLaunchKernelGGL((k_conv<NTv, false, CIv>), dim3(nb), dim3(256), 0, u->stream, a);   \
+    break
+  // output and input tiles of the layers, forward and (transposed) backward
+  switch (c1 % 16 == 0 && c2 % 16 == 0 && co % 16 == 0 ? co + (c1 + c2) / 16 : 0) {
+    CONV_LAUNCH(1, 1);
+    CONV_LAUNCH(1, 2);
+    CONV_LAUNCH(1, 3);
+    CONV_LAUNCH(2, 1);
+    CONV_LAUNCH(2, 2);
+    CONV_LAUNCH(2, 4);
+    CONV_LAUNCH(2, 6);
+    CONV_LAUNCH(3, 1);
+    CONV_LAUNCH(4, 2);
+    CONV_LAUNCH(4, 4);
+    CONV_LAUNCH(6, 2);
+    default: return ufail(SALMON_HIP_EUNSUPPORTED, "conv %d -> %d channels", c1 + c2, co);
   }
 #undef CONV_LAUNCH
   ULAUNCH("k_conv");
