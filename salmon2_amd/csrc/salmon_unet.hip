@@ -20,11 +20,12 @@
 //                  points per wave, N = NT x 16 output channels, K = 32 of the flattened
 //                  (tap, input channel) index (two taps per instruction at 16 channels);
 //                  also the data gradient (flipped, transposed weights, FP32 output)
-//   k_wgrad        weight gradient per (tap, co tile, ci tile) as MFMA over point chunks
-//                  (M = co, N = ci, K = 32 points), FP32 partials reduced in fixed order
+//   k_wg_pack, k_wgrad, k_wg_reduce  weight and bias gradient as MFMA over points (M = co, N = ci, K = 32
+//                  points of channel-major copies), FP32 partials reduced in fixed order
 //   small kernels  pooling, gradient routing (mask, down-sum, pool-back), head, MSE, Adam
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -195,85 +196,210 @@ __global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Weight gradient dW[tap][co][ci] = sum_p dy[p][co] x[p + d(tap)][ci] over one chunk of
-// points per grid row y; wave = (tap, co tile, ci tile); A = dy^T (M = co, K = points),
-// B = shifted input (K = points, N = ci), 32 points per MFMA (lane group q takes points
-// pb + 8q .. pb + 8q + 7).  part[(chunk*27 + tap)*co + co_][ci_].
+// Weight and bias gradient of a convolution: dW[tap][co][ci] = sum_p dy[p][co] x[p + d(tap)][ci],
+// db[co] = sum_p dy[p][co].  The MFMAs' K runs over points, so an operand is 8 consecutive points of
+// one channel per lane: k_wg_pack first lays both tensors out channel-major, the input three times,
+// shifted by -1, 0 and 1 along x with its periodic neighbour.  A wave then takes one (dz, dy) of the
+// kernel, 16 input channels, one or two tiles of 16 output channels and 1024 points: an 8-point block is
+// one 16-byte load where rows are whole blocks (8 / G loads of G points where only G divides the row
+// length: a group of G never spans two rows, so its neighbour rows are contiguous too), and each block of
+// dy serves the three dx taps.  Points are summed in the order of their index, 32 per MFMA, the 1024-point
+// shares in ascending order (k_wg_reduce).
+//
+// A wave per (tap, co tile, ci tile) gathering single 2-byte elements, three divisions each, took 91 us
+// per layer on average at 32^3 where the three kernels here take 20 (4 + 11 + 5); bound now by the
+// latency of the loads (288 waves at the finest level's 16 x 16 channels), not by the matrix cores.
 // ---------------------------------------------------------------------------
+constexpr int kWgChunk = 1024;  // points per partial sum
+
 struct WgArgs {
-  const bf16_t *dy;
+  const bf16_t *dy;            // [npts][co]
   int co;
-  const bf16_t *src1, *src2;
+  const bf16_t *src1, *src2;   // input [up(src1), src2], channels-last
   int c1, c2, up1;
-  float *part;
-  int nx, ny, nz, npts, chunk;
+  bf16_t *xt;                  // [3][ci][npad]
+  bf16_t *gt;                  // [co][npad]
+  float *part;                 // [chunks][27][co][ci]
+  float *grad;                 // [27 co ci weights][co biases]
+  int nx, ny, nz, npts, npad;  // npad: npts rounded up to whole 32-point steps (zeros past npts)
 };
 
-__global__ __launch_bounds__(256) void k_wgrad(WgArgs a) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+// one thread per (point, 8 channels): the input's threads, then dy's
+__global__ __launch_bounds__(256) void k_wg_pack(WgArgs a) {
   const int ci = a.c1 + a.c2;
-  const int nco = a.co / 16, nci = ci / 16;
-  const int task = blockIdx.x * 4 + wave;
-  if (task >= 27 * nco * nci) return;
-  const int cit = task % nci, cot = (task / nci) % nco, tap = task / (nci * nco);
-  const int dz = tap / 9 - 1, dy = (tap / 3) % 3 - 1, dx = tap % 3 - 1;
-  const int row = lane & 15, kq = lane >> 4;
-  const int nx = a.nx, ny = a.ny, nz = a.nz;
-  const int pbeg = blockIdx.y * a.chunk, pend = min(pbeg + a.chunk, a.npts);
-  const int cc = cit * 16 + row;
-  const bool first = cit * 16 < a.c1;
-  f4v acc = f4v{0.f, 0.f, 0.f, 0.f};
-  for (int pb = pbeg; pb < pend; pb += 32) {
-    s8v av, bv;
+  const size_t nxi = (size_t)a.npad * (ci / 8);
+  size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  const s8v zero = {0, 0, 0, 0, 0, 0, 0, 0};
+  if (i < nxi) {
+    const int p = i % a.npad, c = 8 * (int)(i / a.npad);
+    const size_t plane = (size_t)ci * a.npad;
+    const int x = p % a.nx, r = p / a.nx;
+    const int y = r % a.ny, z = r / a.ny;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int pk = pb + 8 * kq + e;
-      short va = 0, vb = 0;
-      if (pk < pend) {
-        va = (short)a.dy[(size_t)pk * a.co + cot * 16 + row];
-        const int x = pk % nx, y = (pk / nx) % ny, z = pk / (nx * ny);
-        const int xn = (x + dx + nx) % nx, yn = (y + dy + ny) % ny, zn = (z + dz + nz) % nz;
-        if (first) {
-          const size_t ph = a.up1 ? (size_t)(xn >> 1) + (size_t)(nx >> 1) * ((size_t)(yn >> 1) + (size_t)(ny >> 1) * (zn >> 1))
-                                  : (size_t)xn + (size_t)nx * ((size_t)yn + (size_t)ny * zn);
-          vb = (short)a.src1[ph * a.c1 + cc];
+    for (int d = 0; d < 3; ++d) {
+      int xn = x + d - 1;
+      xn += xn < 0 ? a.nx : 0;
+      xn -= xn >= a.nx ? a.nx : 0;
+      s8v v = zero;
+      if (p < a.npts) {
+        if (c < a.c1) {
+          const size_t q = a.up1 ? (size_t)(xn >> 1) + (size_t)(a.nx >> 1) * ((size_t)(y >> 1) + (size_t)(a.ny >> 1) * (z >> 1))
+                                 : (size_t)xn + (size_t)a.nx * r;
+          v = *(const s8v *)(a.src1 + q * a.c1 + c);
         } else {
-          const size_t pn = (size_t)xn + (size_t)nx * ((size_t)yn + (size_t)ny * zn);
-          vb = (short)a.src2[pn * a.c2 + (cc - a.c1)];
+          v = *(const s8v *)(a.src2 + ((size_t)xn + (size_t)a.nx * r) * a.c2 + (c - a.c1));
         }
       }
-      av[e] = va;
-      bv[e] = vb;
-    }
-    acc = mfma32(av, bv, acc);
-  }
 #pragma unroll
-  for (int r = 0; r < 4; ++r)
-    a.part[((size_t)(blockIdx.y * 27 + tap) * a.co + cot * 16 + 4 * kq + r) * ci + cc] = acc[r];
+      for (int e = 0; e < 8; ++e) a.xt[d * plane + (size_t)(c + e) * a.npad + p] = (bf16_t)v[e];
+    }
+    return;
+  }
+  i -= nxi;
+  if (i >= (size_t)a.npad * (a.co / 8)) return;
+  const int p = i % a.npad, c = 8 * (int)(i / a.npad);
+  const s8v v = p < a.npts ? *(const s8v *)(a.dy + (size_t)p * a.co + c) : zero;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) a.gt[(size_t)(c + e) * a.npad + p] = (bf16_t)v[e];
 }
 
-// grad[i] += sum_k part[k][i], k ascending
-__global__ __launch_bounds__(256) void k_reduce_add(const float *part, int nk, size_t n, float *grad) {
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  float s = 0.f;
-  for (int k = 0; k < nk; ++k) s += part[(size_t)k * n + i];
-  grad[i] += s;
+template <int G> struct WgGroup;
+template <> struct WgGroup<8> { typedef s8v T; };
+template <> struct WgGroup<4> { typedef short T __attribute__((ext_vector_type(4))); };
+template <> struct WgGroup<2> { typedef short T __attribute__((ext_vector_type(2))); };
+template <> struct WgGroup<1> { typedef short T; };
+
+// NCO: output tiles per wave; G: points per load of the input (a divisor of nx)
+template <int NCO, int G>
+__global__ __launch_bounds__(64) void k_wgrad(WgArgs a) {
+  const int lane = threadIdx.x;
+  const int row = lane & 15, kq = lane >> 4;
+  const int ci = a.c1 + a.c2;
+  const int nci = ci / 16, nct = a.co / 16 / NCO;
+  int t = blockIdx.x;
+  const int cit = t % nci;
+  t /= nci;
+  const int cot = NCO * (t % nct), g = t / nct;
+  const int dz = g / 3 - 1, dyy = g % 3 - 1;
+  const int pbeg = blockIdx.y * kWgChunk, pend = min(pbeg + kWgChunk, a.npts);
+  f4v acc[3][NCO];
+#pragma unroll
+  for (int d = 0; d < 3; ++d)
+#pragma unroll
+    for (int k = 0; k < NCO; ++k) acc[d][k] = f4v{0.f, 0.f, 0.f, 0.f};
+  const size_t plane = (size_t)ci * a.npad;
+  const bf16_t *xr = a.xt + (size_t)(cit * 16 + row) * a.npad;
+  const bf16_t *gr = a.gt + (size_t)(cot * 16 + row) * a.npad;
+  // p / nx by a reciprocal multiply with one correction step
+  const float rnx = 1.f / (float)a.nx, rny = 1.f / (float)a.ny;
+  auto divide = [](int p, int n, float rn) __attribute__((always_inline)) {
+    int q = (int)((float)p * rn);
+    q += (q + 1) * n <= p ? 1 : 0;
+    q -= q * n > p ? 1 : 0;
+    return q;
+  };
+  typedef typename WgGroup<G>::T T;
+  auto load = [&](int pb, s8v (&av)[NCO], s8v (&bv)[3]) __attribute__((always_inline)) {
+    const int p0 = min(pb + 8 * kq, a.npad - 8);  // the lane's 8 points (dy is zero past npts)
+#pragma unroll
+    for (int k = 0; k < NCO; ++k) av[k] = *(const s8v *)(gr + (size_t)(16 * k) * a.npad + p0);
+#pragma unroll
+    for (int h = 0; h < 8 / G; ++h) {
+      const int p = min(p0 + G * h, a.npts - G);
+      const int r = divide(p, a.nx, rnx);
+      const int x = p - r * a.nx;
+      const int z = divide(r, a.ny, rny);
+      int yn = r - z * a.ny + dyy, zn = z + dz;
+      yn += yn < 0 ? a.ny : 0;
+      yn -= yn >= a.ny ? a.ny : 0;
+      zn += zn < 0 ? a.nz : 0;
+      zn -= zn >= a.nz ? a.nz : 0;
+      const bf16_t *xp = xr + (size_t)(zn * a.ny + yn) * a.nx + x;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        if constexpr (G == 8) {
+          bv[d] = *(const s8v *)(xp + d * plane);
+        } else if constexpr (G == 1) {
+          bv[d][h] = (short)xp[d * plane];
+        } else {
+          const T v = *(const T *)(xp + d * plane);
+#pragma unroll
+          for (int e = 0; e < G; ++e) bv[d][G * h + e] = v[e];
+        }
+      }
+    }
+  };
+  // two sets of U steps: the next set's loads are in flight while a set's MFMAs run
+  constexpr int U = NCO == 1 ? 6 : 5;
+  s8v av[2][U][NCO], bv[2][U][3];
+  auto load_group = [&](int pb, s8v (&A)[U][NCO], s8v (&B)[U][3]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) load(pb + 32 * u, A[u], B[u]);
+  };
+  auto mfma_group = [&](int pb, s8v (&A)[U][NCO], s8v (&B)[U][3]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (pb + 32 * u < pend)
+#pragma unroll
+        for (int k = 0; k < NCO; ++k)
+#pragma unroll
+          for (int d = 0; d < 3; ++d) acc[d][k] = mfma32(A[u][k], B[u][d], acc[d][k]);
+  };
+  load_group(pbeg, av[0], bv[0]);
+  for (int pb = pbeg; pb < pend; pb += 64 * U) {
+    if (pb + 32 * U < pend) load_group(pb + 32 * U, av[1], bv[1]);
+    mfma_group(pb, av[0], bv[0]);
+    if (pb + 32 * U >= pend) break;
+    if (pb + 64 * U < pend) load_group(pb + 64 * U, av[0], bv[0]);
+    mfma_group(pb + 32 * U, av[1], bv[1]);
+  }
+  float *part = a.part + (size_t)blockIdx.y * 27 * a.co * ci;
+#pragma unroll
+  for (int k = 0; k < NCO; ++k)
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        part[((size_t)(3 * g + d) * a.co + (cot + k) * 16 + 4 * kq + e) * ci + cit * 16 + row] = acc[d][k][e];
 }
 
-// grad[c] += sum_p g[p][c] (bias gradient), one block per channel, fixed-order tree
-__global__ __launch_bounds__(256) void k_colsum(const bf16_t *g, int npts, int C, float *grad) {
+// grad[i] += sum_k part[k][i], k ascending, 8 loads in flight (the first nwb blocks), and the biases:
+// grad[nw + c] += sum_p dy[p][c], one block per channel, fixed-order tree
+__global__ __launch_bounds__(256) void k_wg_reduce(WgArgs a, int nk, size_t nw, unsigned nwb) {
   __shared__ float sh[256];
-  const int c = blockIdx.x;
+  if (blockIdx.x < nwb) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= nw) return;
+    float s = 0.f;
+    for (int k = 0; k < nk; k += 8) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = a.part[(size_t)min(k + u, nk - 1) * nw + i];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (k + u < nk) s += v[u];
+    }
+    a.grad[i] += s;
+    return;
+  }
+  const int c = blockIdx.x - nwb;
+  const bf16_t *g = a.gt + (size_t)c * a.npad;
   float s = 0.f;
-  for (int p = threadIdx.x; p < npts; p += 256) s += bf2f(g[(size_t)p * C + c]);
+  for (int p0 = threadIdx.x; p0 < a.npts; p0 += 256 * 16) {
+    bf16_t v[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) v[u] = g[min(p0 + 256 * u, a.npts - 1)];
+#pragma unroll
+    for (int u = 0; u < 16; ++u)
+      if (p0 + 256 * u < a.npts) s += bf2f(v[u]);
+  }
   sh[threadIdx.x] = s;
   __syncthreads();
   for (int k = 128; k > 0; k >>= 1) {
     if ((int)threadIdx.x < k) sh[threadIdx.x] += sh[threadIdx.x + k];
     __syncthreads();
   }
-  if (threadIdx.x == 0) grad[c] += sh[0];
+  if (threadIdx.x == 0) a.grad[nw + c] += sh[0];
 }
 
 // 2x2x2 average pool: out (hx, hy, hz) = mean of its 8 children
@@ -388,19 +514,33 @@ __global__ __launch_bounds__(256) void k_loss(const float *part, int nb, size_t 
   if (threadIdx.x == 0) *loss = sh[0] / (float)n;
 }
 
-// head gradients: block c < 16: grad[c] += sum_p dout[p] x[p][c]; block 16: grad[16] += sum dout
+// head gradients: block b < 4: grad[c] += sum_p dout[p] x[p][c] for its four channels; block 4: grad[16]
+// += sum dout.  A thread takes every 256th point, one 8-byte load for its channels, 8 points in flight;
+// fixed-order tree.  (One block and one 2-byte load per channel: 42 us at 32^3, 14 us here.)
 __global__ __launch_bounds__(256) void k_head_grad(const float *dout, const bf16_t *x, size_t npts, float *grad) {
-  __shared__ float sh[256];
-  const int c = blockIdx.x;
-  float s = 0.f;
-  for (size_t p = threadIdx.x; p < npts; p += 256) s += dout[p] * (c < 16 ? bf2f(x[p * 16 + c]) : 1.f);
-  sh[threadIdx.x] = s;
+  __shared__ float sh[4][256];
+  typedef short s4v __attribute__((ext_vector_type(4)));
+  const bool ones = blockIdx.x == 4;
+  const int c0 = ones ? 0 : 4 * blockIdx.x;
+  float s[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+  for (size_t p = threadIdx.x; p < npts; p += 256) {
+    const float d = dout[p];
+    const s4v v = *(const s4v *)(x + p * 16 + c0);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) s[c] += d * (ones ? 1.f : bf2f((bf16_t)v[c]));
+  }
+#pragma unroll
+  for (int c = 0; c < 4; ++c) sh[c][threadIdx.x] = s[c];
   __syncthreads();
   for (int k = 128; k > 0; k >>= 1) {
-    if ((int)threadIdx.x < k) sh[threadIdx.x] += sh[threadIdx.x + k];
+    if ((int)threadIdx.x < k)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) sh[c][threadIdx.x] += sh[c][threadIdx.x + k];
     __syncthreads();
   }
-  if (threadIdx.x == 0) grad[c] += sh[0];
+  if (ones && threadIdx.x == 0) grad[16] += sh[0][0];
+  if (!ones && threadIdx.x < 4) grad[c0 + threadIdx.x] += sh[threadIdx.x][0];
 }
 
 // g[p][c] = bf16(dout[p] wh[c] (act[p][c] > 0))
@@ -550,8 +690,8 @@ struct salmon_unet {
   // backward work
   float *d_out = nullptr, *d_dout = nullptr, *d_part = nullptr, *d_fx = nullptr, *d_fy = nullptr, *d_wpart = nullptr;
   bf16_t *g_a = nullptr, *g_b = nullptr;
-  size_t wpart_n = 0, fx_n = 0;
-  int chunk = 1024;
+  bf16_t *d_xt = nullptr, *d_gt = nullptr;  // channel-major operands of the weight gradient
+  size_t fx_n = 0;
   double *d_rpart = nullptr;  // residual partial maxima
   std::vector<void *> allocs;
 };
@@ -654,25 +794,39 @@ int forward(salmon_unet *u, const float *in, float *out) {
   return 0;
 }
 
+template <int NCO>
+void launch_wgrad(hipStream_t st, const dim3 &grid, const WgArgs &a) {
+  if (a.nx % 8 == 0) hipLaunchKernelGGL((k_wgrad<NCO, 8>), grid, dim3(64), 0, st, a);
+  else if (a.nx % 4 == 0) hipLaunchKernelGGL((k_wgrad<NCO, 4>), grid, dim3(64), 0, st, a);
+  else if (a.nx % 2 == 0) hipLaunchKernelGGL((k_wgrad<NCO, 2>), grid, dim3(64), 0, st, a);
+  else hipLaunchKernelGGL((k_wgrad<NCO, 1>), grid, dim3(64), 0, st, a);
+}
+
+size_t wg_pad(size_t npts) { return (npts + 31) / 32 * 32; }
+
 // weight and bias gradient of conv layer l (act index i) from its pre-activation gradient g
 int layer_wgrad(salmon_unet *u, int i, const Layer &l, const bf16_t *g) {
   const int ci = l.c1 + l.c2;
   WgArgs a;
   a.dy = g; a.co = l.co;
   a.src1 = layer_src1(u, i); a.src2 = layer_src2(u, i); a.c1 = l.c1; a.c2 = l.c2; a.up1 = l.up1;
+  a.xt = u->d_xt; a.gt = u->d_gt;
   a.part = u->d_wpart;
+  a.grad = u->d_g + l.woff;  // the layer's weights and biases lie side by side
   a.nx = u->n[l.level][0]; a.ny = u->n[l.level][1]; a.nz = u->n[l.level][2];
   a.npts = (int)u->np[l.level];
-  a.chunk = u->chunk;
-  const int nchunk = (a.npts + a.chunk - 1) / a.chunk;
-  const int ntask = 27 * (l.co / 16) * (ci / 16);
-  hipLaunchKernelGGL(k_wgrad, dim3((ntask + 3) / 4, nchunk), dim3(256), 0, u->stream, a);
+  a.npad = (int)wg_pad(a.npts);
+  hipLaunchKernelGGL(k_wg_pack, dim3(blocks((size_t)a.npad * (ci + l.co) / 8)), dim3(256), 0, u->stream, a);
+  ULAUNCH("k_wg_pack");
+  const int nchunk = (a.npts + kWgChunk - 1) / kWgChunk;
+  // two output tiles per wave share the input's loads where that leaves a wave for every CU
+  const int tasks = 9 * (ci / 16) * (l.co / 16);
+  if (l.co % 32 == 0 && tasks * nchunk / 2 >= 256) launch_wgrad<2>(u->stream, dim3(tasks / 2, nchunk), a);
+  else launch_wgrad<1>(u->stream, dim3(tasks, nchunk), a);
   ULAUNCH("k_wgrad");
   const size_t nw = (size_t)27 * l.co * ci;
-  hipLaunchKernelGGL(k_reduce_add, dim3(blocks(nw)), dim3(256), 0, u->stream, u->d_wpart, nchunk, nw, u->d_g + l.woff);
-  ULAUNCH("k_reduce_add");
-  hipLaunchKernelGGL(k_colsum, dim3(l.co), dim3(256), 0, u->stream, g, a.npts, l.co, u->d_g + l.boff);
-  ULAUNCH("k_colsum");
+  hipLaunchKernelGGL(k_wg_reduce, dim3(blocks(nw) + l.co), dim3(256), 0, u->stream, a, nchunk, nw, blocks(nw));
+  ULAUNCH("k_wg_reduce");
   return 0;
 }
 
@@ -691,7 +845,7 @@ int backward(salmon_unet *u, const float *target, float *loss) {
     hipLaunchKernelGGL(k_loss, dim3(1), dim3(256), 0, u->stream, u->d_part, (int)nb0, n0, loss);
     ULAUNCH("k_loss");
   }
-  hipLaunchKernelGGL(k_head_grad, dim3(17), dim3(256), 0, u->stream, u->d_dout, u->act[D1B], n0, u->d_g + u->head_off);
+  hipLaunchKernelGGL(k_head_grad, dim3(5), dim3(256), 0, u->stream, u->d_dout, u->act[D1B], n0, u->d_g + u->head_off);
   ULAUNCH("k_head_grad");
   bf16_t *g = u->g_a, *gn = u->g_b;
   hipLaunchKernelGGL(k_head_back, dim3(blocks(n0 * 16)), dim3(256), 0, u->stream, u->d_dout, u->d_w + u->head_off,
@@ -801,15 +955,17 @@ int salmon_unet_create(int nx, int ny, int nz, unsigned long long seed, salmon_u
     if ((rc = ualloc(u, &u->act[i], act_n[i]))) return bail(rc);
   // d_fx: data gradient (max np * ci) followed by the two kept skip gradients (n0 x 48, n1 x 96)
   u->fx_n = std::max({n0 * 48, n1 * 96, n2 * 64, n1 * 32, n0 * 16});
-  size_t wp = 0;
+  size_t wp = 0, xt = 0, gt = 0;
   for (Layer &l : u->L) {
-    const size_t nch = (u->np[l.level] + u->chunk - 1) / u->chunk;
-    wp = std::max(wp, nch * 27 * l.co * (l.c1 + l.c2));
+    const size_t ci = l.c1 + l.c2, np = u->np[l.level];
+    wp = std::max(wp, (np + kWgChunk - 1) / kWgChunk * 27 * l.co * ci);
+    xt = std::max(xt, 3 * ci * wg_pad(np));
+    gt = std::max(gt, l.co * wg_pad(np));
   }
-  u->wpart_n = wp;
   if ((rc = ualloc(u, &u->d_out, n0)) || (rc = ualloc(u, &u->d_dout, n0)) || (rc = ualloc(u, &u->d_part, blocks(n0))) ||
       (rc = ualloc(u, &u->d_fx, u->fx_n + n0 * 48 + n1 * 96)) || (rc = ualloc(u, &u->d_fy, n1 * 64)) ||
-      (rc = ualloc(u, &u->d_wpart, wp)) || (rc = ualloc(u, &u->g_a, n0 * 64)) || (rc = ualloc(u, &u->g_b, n0 * 64)) ||
+      (rc = ualloc(u, &u->d_wpart, wp)) || (rc = ualloc(u, &u->d_xt, xt)) || (rc = ualloc(u, &u->d_gt, gt)) ||
+      (rc = ualloc(u, &u->g_a, n0 * 64)) || (rc = ualloc(u, &u->g_b, n0 * 64)) ||
       (rc = ualloc(u, &u->d_rpart, 1024)))
     return bail(rc);
   // He-normal weights, zero biases; head: small normal weights, zero bias
