@@ -254,7 +254,7 @@ int salmon_hip_set_poisson(salmon_hip_t h, const double *al);
 /*
  * Hartree potential Vh(nx,ny,nz) of the total density rho(nx,ny,nz), both DEVICE
  * arrays (hartree -> poisson_ft, src/poisson/hartree.f90, poisson_periodic.f90:23-242):
- * separable forward DFT z, y, x with 1/N, multiply by coef, inverse DFT, real part.
+ * separable forward DFT z, y, x with 1/N, multiply by coef, inverse DFT (the real density's half spectrum).
  */
 int salmon_hip_hartree(salmon_hip_t h, const double *rho_dev, double *vh_dev);
 
@@ -291,7 +291,7 @@ int salmon_hip_vlocal_extrapolate(salmon_hip_t h, double *vold1_dev, double *vol
  * rho_s(nx,ny,nz,nspin) as calc_density returns it, as time_evolution_step.f90:160-207
  * does every step with yn_fix_func = 'n': Vh of the total density (rho_s(1) + rho_s(2)
  * for nspin = 2, summed in the first DFT pass), Vxc of the channel densities formed in
- * the update kernel, Vh kept in handle scratch.  vmix, vout (nx,ny,nz,nspin) as above.
+ * the last transform pass, where Vh is complete point by point.  vmix, vout (nx,ny,nz,nspin) as above.
  */
 int salmon_hip_update_potential(salmon_hip_t h, const double *rho_dev, const double *vpsl_dev,
                                 const double *vmix_dev, double *vout_dev);

@@ -20,7 +20,7 @@
 //   k_density_*       calc_density (density_matrix.f90:150-230)
 //   k_current_*       stencil_current + calc_current (density_matrix.f90:240-530)
 //   k_dipole_part/_sum calc_dip (src/rt/dip.f90:114-225)
-//   k_dft_axis        Hartree potential (poisson_ft, src/poisson/poisson_periodic.f90:23-242)
+//   k_dft_*           Hartree potential (poisson_ft, src/poisson/poisson_periodic.f90:23-242)
 //   k_xc_pz           PZ81 LDA (src/xc/builtin_pz.f90:23-83) and its spin-polarised form
 //                     (src/xc/builtin_pz_sp.f90:23-98)
 //   k_update_vlocal   update_vlocal (src/common/hamiltonian.f90:813-843) with the
@@ -2065,93 +2065,6 @@ __global__ __launch_bounds__(256) void k_dipole_sum(DipArgs a) { dipole_sum_body
 
 #include "small_grid.h"
 
-// ---------------------------------------------------------------------------
-// Hartree potential: poisson_ft (src/poisson/poisson_periodic.f90:23-242) as six
-// separable DFT passes (forward z, y, x with conj twiddles, 1/N and the 4 pi/|G|^2
-// table folded into the x pass; inverse z, y, x, real part out).  Per pass the grid
-// is viewed as (outer, n, inner), inner = stride of the transformed axis; a block
-// owns `cols` consecutive columns c = (o, i), stages the [n][cols] tile in LDS and
-// forms out(k) = sum_j tw(k, j) in(j) with the n x n table tw = exp(i 2 pi j k / n)
-// (src/common/initialization.f90:761-784).  Reads and writes are unit-stride along
-// c for the y and z passes and along j for the x pass.
-// ---------------------------------------------------------------------------
-constexpr int kDftMaxN = 256;
-
-struct DftArgs {
-  const double2 *in;  // complex input, or null with rin
-  const double *rin;  // real input (first forward pass)
-  const double *rin2; // with rin: a second real input added to it (the other spin channel), or null
-  double2 *out;       // complex output, or null with rout
-  double *rout;       // real part output (last inverse pass)
-  const double2 *tw;  // n x n, tw[k * n + j]
-  const double *coef; // per-point multiplier after the pass (x forward pass), or null
-  double nrm;         // divisor applied before coef
-  long long ncols;    // outer * inner
-  int n, inner, cols;
-  double sg;          // -1: conj(tw) (forward), +1: tw (inverse)
-  const int *skip;    // device flag: the launch does nothing when it is set (null: never)
-};
-
-__global__ __launch_bounds__(256) void k_dft_axis(DftArgs a) {
-  extern __shared__ double2 dft_tile[];  // [n][cols]
-  if (a.skip && *a.skip) return;  // a device-side gate switched this launch off
-  const int n = a.n, inner = a.inner, cols = a.cols;
-  const long long c0 = (long long)blockIdx.x * cols;
-  const int ncl = (int)min((long long)cols, a.ncols - c0);
-  const int tot = n * cols;
-  for (int t = threadIdx.x; t < tot; t += blockDim.x) {
-    int j, cl;
-    if (inner == 1) { cl = t / n; j = t - cl * n; } else { j = t / cols; cl = t - j * cols; }
-    double2 v = make_double2(0.0, 0.0);
-    if (cl < ncl) {
-      const long long c = c0 + cl;
-      const long long o = c / inner, i = c - o * inner;
-      const size_t g = ((size_t)o * n + j) * inner + i;
-      v = a.rin ? make_double2(a.rin2 ? a.rin[g] + a.rin2[g] : a.rin[g], 0.0) : a.in[g];
-    }
-    dft_tile[j * cols + cl] = v;
-  }
-  __syncthreads();
-  for (int t = threadIdx.x; t < tot; t += blockDim.x) {
-    int k, cl;
-    if (inner == 1) { cl = t / n; k = t - cl * n; } else { k = t / cols; cl = t - k * cols; }
-    if (cl >= ncl) continue;
-    const double2 *w = a.tw + (size_t)k * n;
-    double sr = 0.0, si = 0.0;
-    int j = 0;
-    // 8 twiddle loads in flight ahead of the in-order sum
-    for (; j + 8 <= n; j += 8) {
-      double2 e[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) e[u] = w[j + u];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const double2 x = dft_tile[(j + u) * cols + cl];
-        const double ei = a.sg * e[u].y;
-        sr = sr + (e[u].x * x.x - ei * x.y);
-        si = si + (e[u].x * x.y + ei * x.x);
-      }
-    }
-    for (; j < n; ++j) {
-      const double2 e = w[j];
-      const double2 x = dft_tile[j * cols + cl];
-      const double ei = a.sg * e.y;
-      sr = sr + (e.x * x.x - ei * x.y);
-      si = si + (e.x * x.y + ei * x.x);
-    }
-    const long long c = c0 + cl;
-    const long long o = c / inner, i = c - o * inner;
-    const size_t g = ((size_t)o * n + k) * inner + i;
-    if (a.coef) {
-      const double cf = a.coef[g];
-      sr = cf * (sr / a.nrm);
-      si = cf * (si / a.nrm);
-    }
-    if (a.rout) a.rout[g] = sr;
-    else a.out[g] = make_double2(sr, si);
-  }
-}
-
 // PZ81 LDA, unpolarised (exc_cor_pz / PZxc, src/xc/builtin_pz.f90:23-83), trho = rho.
 __device__ __forceinline__ void pz_point(double rho, double &vxc, double &exc) {
   const double Pi = 3.141592653589793;
@@ -2250,10 +2163,8 @@ struct VlocArgs {
   const int *skip;    // device flag: the launch does nothing when it is set (null: never)
 };
 
-__global__ __launch_bounds__(256) void k_update_vlocal(VlocArgs a) {
-  if (a.skip && *a.skip) return;  // a device-side gate switched this launch off
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= a.n) return;
+// V_local of point i from its Hartree potential
+__device__ __forceinline__ void vlocal_point(const VlocArgs &a, size_t i, double vh) {
   double vx[2];
   if (a.rho) {
     double e;
@@ -2263,13 +2174,223 @@ __global__ __launch_bounds__(256) void k_update_vlocal(VlocArgs a) {
     vx[0] = a.vxc[i];
     if (a.nspin == 2) vx[1] = a.vxc[a.n + i];
   }
-  const double base = a.vpsl[i] + a.vh[i];
+  const double base = a.vpsl[i] + vh;
   for (int is = 0; is < a.nspin; ++is) {
     const size_t j = (size_t)is * a.n + i;
     double v = base + vx[is];
     if (a.vmix) v = 0.5 * (a.vmix[j] + v);
     a.V[j] = v;
     if (a.vout) a.vout[j] = v;
+  }
+}
+
+__global__ __launch_bounds__(256) void k_update_vlocal(VlocArgs a) {
+  if (a.skip && *a.skip) return;  // a device-side gate switched this launch off
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < a.n) vlocal_point(a, i, a.vh[i]);
+}
+
+// ---------------------------------------------------------------------------
+// Hartree potential: poisson_ft (src/poisson/poisson_periodic.f90:23-242) as separable DFT passes in
+// five launches: forward z, forward y, along x forward, times 4 pi/|G|^2/N and back in one, inverse y,
+// inverse z.  The density is real, so only kz = 0 .. nz/2 is kept (the others are the conjugates), and
+// the last pass can finish with V_local of its points instead of storing Vh.  A pass views the grid as
+// columns of the transformed axis; a block stages COLS of them in LDS and folds them, u_j = x_j +
+// x_{n-j} and v_j = x_j - x_{n-j}: with A = sum_j u_j cos(2 pi jk/n) and B = sum_j v_j sin(2 pi jk/n)
+// over half the points, one thread has both X_k = A + i sg B and X_{n-k} = A - i sg B, a quarter of the
+// plain sum's operations.  The n values exp(2 pi i m/n) are in LDS too, read at m = jk mod n.
+//
+// Bound by launch and LDS latency (a few thousand operations per thread's pair at most).  Measured, per
+// potential update: seven launches with n x n twiddle tables gathered from memory took 75 us at
+// 56x50x42 and 31 us at 12^3, these 29 us and 20 us.  256 threads (32 output pairs of 8 columns) beat
+// 128 by a quarter at 56x50x42 (29 against 38 us): one round of pairs instead of two.
+// ---------------------------------------------------------------------------
+constexpr int kDftMaxN = 256;
+
+struct DftArgs {
+  const double *rho, *rho2;  // density, and the other spin channel's to be added (or null)
+  const double2 *in;
+  double2 *out;
+  const double2 *tw;  // exp(2 pi i m / n), m = 0 .. n-1
+  const double *coef;  // 4 pi/|G|^2 (nx, ny, nz)
+  double *vh;          // Hartree potential, or null: finish with V_local (v)
+  VlocArgs v;
+  double rn;           // 1 / N_grid
+  double sg;           // -1 forward, +1 inverse
+  int n, inner, ncols; // transformed extent, its stride, columns
+  const int *skip;     // device flag: the launch does nothing when it is set (null: never)
+};
+
+__device__ __forceinline__ double2 operator+(const double2 &a, const double2 &b) { return make_double2(a.x + b.x, a.y + b.y); }
+__device__ __forceinline__ double2 operator-(const double2 &a, const double2 &b) { return make_double2(a.x - b.x, a.y - b.y); }
+__device__ __forceinline__ double2 operator*(double a, const double2 &b) { return make_double2(a * b.x, a * b.y); }
+
+// Columns of [n][COLS] in place: u_j at j, v_j at n - j (j = 1 .. (n-1)/2); ends with a barrier.
+template <int COLS, int BS, typename T>
+__device__ __forceinline__ void dft_fold(T *x, int n) {
+  const int h = (n - 1) / 2;
+  for (int t = threadIdx.x; t < h * COLS; t += BS) {
+    const int j = 1 + t / COLS, cl = t % COLS;
+    const T a = x[j * COLS + cl], b = x[(n - j) * COLS + cl];
+    x[j * COLS + cl] = a + b;
+    x[(n - j) * COLS + cl] = a - b;
+  }
+  __syncthreads();
+}
+
+// A and B of output pair k of folded column cl
+template <int COLS, typename T>
+__device__ __forceinline__ void dft_pair(const T *x, const double2 *tw, int n, int k, int cl, T &A, T &B) {
+  const int h = (n - 1) / 2;
+  A = x[cl];
+  if (n % 2 == 0) A = k % 2 ? A - x[(n / 2) * COLS + cl] : A + x[(n / 2) * COLS + cl];
+  B = 0.0 * x[cl];
+  int m = 0;
+#pragma unroll 4
+  for (int j = 1; j <= h; ++j) {
+    m += k;
+    m -= m >= n ? n : 0;
+    const double2 w = tw[m];
+    A = A + w.x * x[j * COLS + cl];
+    B = B + w.y * x[(n - j) * COLS + cl];
+  }
+}
+
+__device__ __forceinline__ double2 times_i(double s, const double2 &b) { return make_double2(-s * b.y, s * b.x); }
+
+// forward z of the real density: out[kz][column], kz = 0 .. n/2
+__global__ __launch_bounds__(256) void k_dft_zr(DftArgs a) {
+  constexpr int COLS = 16, BS = 256;
+  extern __shared__ double2 lds[];
+  if (a.skip && *a.skip) return;  // a device-side gate switched this launch off
+  double2 *tw = lds;
+  double *x = (double *)(lds + a.n);  // [n][COLS]
+  const int c0 = blockIdx.x * COLS;
+  for (int t = threadIdx.x; t < a.n; t += BS) tw[t] = a.tw[t];
+  for (int t = threadIdx.x; t < a.n * COLS; t += BS) {
+    const int j = t / COLS, c = c0 + t % COLS;
+    const size_t g = (size_t)j * a.inner + c;
+    x[t] = c >= a.ncols ? 0.0 : a.rho2 ? a.rho[g] + a.rho2[g] : a.rho[g];
+  }
+  __syncthreads();
+  dft_fold<COLS, BS>(x, a.n);
+  const int cl = threadIdx.x % COLS;
+  if (c0 + cl >= a.ncols) return;
+  for (int k = threadIdx.x / COLS; k <= a.n / 2; k += BS / COLS) {
+    double A, B;
+    dft_pair<COLS>(x, tw, a.n, k, cl, A, B);
+    a.out[(size_t)k * a.inner + c0 + cl] = make_double2(A, a.sg * B);
+  }
+}
+
+// y pass: columns (kz, x)
+template <int COLS>
+__global__ __launch_bounds__(256) void k_dft_y(DftArgs a) {
+  constexpr int BS = 256;
+  extern __shared__ double2 lds[];
+  if (a.skip && *a.skip) return;  // a device-side gate switched this launch off
+  const int n = a.n;
+  double2 *tw = lds, *x = lds + n;  // [n][COLS]
+  const int cl = threadIdx.x % COLS, c = blockIdx.x * COLS + cl;
+  const bool on = c < a.ncols;
+  const int o = on ? c / a.inner : 0;
+  const size_t g0 = (size_t)o * n * a.inner + (on ? c - o * a.inner : 0);
+  for (int t = threadIdx.x; t < n; t += BS) tw[t] = a.tw[t];
+  for (int j = threadIdx.x / COLS; j < n; j += BS / COLS) x[j * COLS + cl] = a.in[g0 + (size_t)j * a.inner];
+  __syncthreads();
+  dft_fold<COLS, BS>(x, n);
+  if (!on) return;
+  for (int k = threadIdx.x / COLS; k <= n / 2; k += BS / COLS) {
+    double2 A, B;
+    dft_pair<COLS>(x, tw, n, k, cl, A, B);
+    const double2 iB = times_i(a.sg, B);
+    a.out[g0 + (size_t)k * a.inner] = A + iB;
+    if (k > 0 && 2 * k < n) a.out[g0 + (size_t)(n - k) * a.inner] = A - iB;
+  }
+}
+
+// along x: forward, times coef / N, inverse, in place; columns are rows (ky, kz) of n points
+template <int COLS>
+__global__ __launch_bounds__(256) void k_dft_x(DftArgs a) {
+  constexpr int BS = 256;
+  extern __shared__ double2 lds[];
+  if (a.skip && *a.skip) return;  // a device-side gate switched this launch off
+  const int n = a.n;
+  double2 *tw = lds, *x = lds + n, *y = x + n * COLS;  // [n][COLS] each
+  const int c0 = blockIdx.x * COLS, ncl = min(COLS, a.ncols - c0);
+  for (int t = threadIdx.x; t < n; t += BS) tw[t] = a.tw[t];
+  for (int t = threadIdx.x; t < n * COLS; t += BS) {
+    const int r = t / n, j = t - r * n;
+    x[j * COLS + r] = r < ncl ? a.in[(size_t)(c0 + r) * n + j] : make_double2(0.0, 0.0);
+  }
+  __syncthreads();
+  dft_fold<COLS, BS>(x, n);
+  const int cl = threadIdx.x % COLS;
+  const bool on = cl < ncl;
+  const double *cf = a.coef + (size_t)(c0 + (on ? cl : 0)) * n;
+  for (int k = threadIdx.x / COLS; k <= n / 2; k += BS / COLS) {
+    const int kk = k > 0 && 2 * k < n ? n - k : k;
+    const double f0 = a.rn * cf[k], f1 = a.rn * cf[kk];
+    double2 A, B;
+    dft_pair<COLS>(x, tw, n, k, cl, A, B);
+    const double2 iB = times_i(-1.0, B);
+    y[k * COLS + cl] = f0 * (A + iB);
+    if (kk != k) y[kk * COLS + cl] = f1 * (A - iB);
+  }
+  __syncthreads();
+  dft_fold<COLS, BS>(y, n);
+  for (int k = threadIdx.x / COLS; k <= n / 2; k += BS / COLS) {
+    double2 A, B;
+    dft_pair<COLS>(y, tw, n, k, cl, A, B);
+    const double2 iB = times_i(1.0, B);
+    x[k * COLS + cl] = A + iB;
+    if (k > 0 && 2 * k < n) x[(n - k) * COLS + cl] = A - iB;
+  }
+  __syncthreads();
+  for (int t = threadIdx.x; t < n * ncl; t += BS) {
+    const int r = t / n, j = t - r * n;
+    a.out[(size_t)(c0 + r) * n + j] = x[j * COLS + r];
+  }
+}
+
+// inverse z from kz = 0 .. n/2 to real values at z and n - z, which are Vh or end in V_local
+template <int COLS>
+__global__ __launch_bounds__(256) void k_dft_zi(DftArgs a) {
+  constexpr int BS = 256;
+  extern __shared__ double2 lds[];
+  if (a.skip && *a.skip) return;  // a device-side gate switched this launch off
+  const int n = a.n, h = (n - 1) / 2;
+  double2 *tw = lds, *x = lds + n;  // [n/2 + 1][COLS]
+  const int cl = threadIdx.x % COLS, c = blockIdx.x * COLS + cl;
+  const bool on = c < a.ncols;
+  for (int t = threadIdx.x; t < n; t += BS) tw[t] = a.tw[t];
+  for (int k = threadIdx.x / COLS; k <= n / 2; k += BS / COLS)
+    x[k * COLS + cl] = on ? a.in[(size_t)k * a.inner + c] : make_double2(0.0, 0.0);
+  __syncthreads();
+  if (!on) return;
+  for (int z = threadIdx.x / COLS; z <= n / 2; z += BS / COLS) {
+    double A = 0.0, B = 0.0;
+    int m = 0;
+#pragma unroll 4
+    for (int k = 1; k <= h; ++k) {
+      m += z;
+      m -= m >= n ? n : 0;
+      const double2 w = tw[m], v = x[k * COLS + cl];
+      A += w.x * v.x;
+      B += w.y * v.y;
+    }
+    A = x[cl].x + 2.0 * A;
+    B = 2.0 * B;
+    if (n % 2 == 0) A += z % 2 ? -x[(n / 2) * COLS + cl].x : x[(n / 2) * COLS + cl].x;
+    const size_t g = (size_t)z * a.inner + c, gm = (size_t)(n - z) * a.inner + c;
+    const bool two = z > 0 && 2 * z < n;
+    if (a.vh) {
+      a.vh[g] = A - B;
+      if (two) a.vh[gm] = A + B;
+    } else {
+      vlocal_point(a.v, g, A - B);
+      if (two) vlocal_point(a.v, gm, A + B);
+    }
   }
 }
 
@@ -2382,10 +2503,10 @@ struct salmon_hip_ctx {
   double *d_scratch = nullptr;  // this device's copy of `scratch` (salmon_hip_density_noalloc)
   double *d_dippart = nullptr;  // dipole block partials (4 x kDipBlocks)
   int dens_ngrp = 1;
-  // Hartree (salmon_hip_set_poisson): twiddle tables per axis, 4 pi/|G|^2 table, work
+  // Hartree (salmon_hip_set_poisson): exp(2 pi i m/n) per axis, 4 pi/|G|^2 table, half-spectrum work grids
   bool have_cell = false;
   double2 *d_tw[3] = {nullptr, nullptr, nullptr};
-  double *d_gcoef = nullptr, *d_vh = nullptr;
+  double *d_gcoef = nullptr;
   double2 *d_fft[2] = {nullptr, nullptr};
   // stencil launch shape
   int TY = 1, TZ = 1, nyt = 1, nzt = 1;
@@ -2527,7 +2648,7 @@ int salmon_hip_destroy(salmon_hip_t c) {
   dfree(c->d_tp_info); dfree(c->d_sink);
   dfree(c->d_curpart); dfree(c->d_contrib); dfree(c->d_denspart); dfree(c->d_dippart);
   for (int d = 0; d < 3; ++d) dfree(c->d_tw[d]);
-  dfree(c->d_gcoef); dfree(c->d_vh); dfree(c->d_fft[0]); dfree(c->d_fft[1]);
+  dfree(c->d_gcoef); dfree(c->d_fft[0]); dfree(c->d_fft[1]);
   for (double2 *&p : c->tscr) dfree(p);
   for (float2 *&p : c->tscr32) dfree(p);
   for (hipEvent_t e : c->ev) (void)hipEventDestroy(e);
@@ -3241,7 +3362,8 @@ constexpr SmallClass kSmallClass[] = {{512, 2, 8}, {512, 4, 4}, {768, 3, 10}, {1
 // The fewest wave-planes (waves x planes per thread, idle lanes included: the stencil is bound by the
 // CU's LDS reads), weighted by what the launch needs beside: with up to two orbitals per CU the
 // block's own latency counts, and the class with 256 registers issues its table loads ahead of their
-// use; with more, blocks that share a CU hide each other's barriers and loads.  Measured (one Taylor
+// use; with more, blocks that share a CU hide each other's barriers and loads (few resident waves, or one
+// block alone, cost as measured at 12^3).  Measured (one Taylor
 // step of order 4, 8 atoms): 16^3, 16 orbitals: 51.6 us as {512, 2} with 8 planes, 56.7 as {768, 3},
 // 73.8 as {512, 4}; 12^3, 1024 orbitals: 94 us as {512, 4} with 4 planes, 117 as {768, 3} with 3,
 // 126 as {512, 2} with 4.
@@ -3268,7 +3390,7 @@ static SmallShape small_shape(const salmon_hip_ctx *c) {
         cost *= K.minw == 2 ? 1.0 : 1.15;
       } else {
         const int blocks = std::min(std::max(1, 4 * K.minw / waves), (int)std::max<size_t>(1, (160 * 1024) / s.lds));
-        cost *= std::sqrt(16.0 / std::min(16, blocks * waves));
+        cost *= std::sqrt(16.0 / std::min(16, blocks * waves)) * (blocks == 1 ? 1.2 : 1.0);
       }
       if (best.cls < 0 || cost < low) {
         best = s;
@@ -3802,12 +3924,11 @@ int salmon_hip_set_poisson(salmon_hip_t c, const double *al) {
   const double pi = 3.141592653589793238462643383279502884;
   int rc = 0;
   for (int d = 0; d < 3; ++d) {
-    std::vector<double2> tw((size_t)n[d] * n[d]);
-    for (int j = 0; j < n[d]; ++j)
-      for (int k = 0; k < n[d]; ++k) {
-        const double ang = 2.0 * pi * (double)((long)j * k) / (double)n[d];
-        tw[(size_t)k * n[d] + j] = make_double2(cos(ang), sin(ang));
-      }
+    std::vector<double2> tw(n[d]);
+    for (int m = 0; m < n[d]; ++m) {
+      const double ang = 2.0 * pi * (double)m / (double)n[d];
+      tw[m] = make_double2(cos(ang), sin(ang));
+    }
     if (!c->d_tw[d] && (rc = dalloc(&c->d_tw[d], tw.size()))) return rc;
     HIPCHK(hipMemcpy(c->d_tw[d], tw.data(), sizeof(double2) * tw.size(), hipMemcpyHostToDevice));
   }
@@ -3828,56 +3949,90 @@ int salmon_hip_set_poisson(salmon_hip_t c, const double *al) {
       }
   if (!c->d_gcoef && (rc = dalloc(&c->d_gcoef, c->ngrid))) return rc;
   HIPCHK(hipMemcpy(c->d_gcoef, coef.data(), sizeof(double) * c->ngrid, hipMemcpyHostToDevice));
-  if (!c->d_fft[0] && (rc = dalloc(&c->d_fft[0], c->ngrid))) return rc;
-  if (!c->d_fft[1] && (rc = dalloc(&c->d_fft[1], c->ngrid))) return rc;
-  if (!c->d_vh && (rc = dalloc(&c->d_vh, c->ngrid))) return rc;
+  const size_t half = (size_t)c->nx * c->ny * (c->nz / 2 + 1);
+  for (double2 *&p : c->d_fft)
+    if (!p && (rc = dalloc(&p, half))) return rc;
   c->have_cell = true;
   return 0;
 }
 
-static int launch_dft(salmon_hip_t c, int axis, double sg, const double *rin, const double2 *in, double2 *out,
-                      double *rout, const double *coef, const double *rin2 = nullptr) {
-  const int n[3] = {c->nx, c->ny, c->nz};
-  const int inner = axis == 0 ? 1 : (axis == 1 ? c->nx : c->nx * c->ny);
-  DftArgs a;
-  a.in = in; a.rin = rin; a.rin2 = rin2; a.out = out; a.rout = rout;
-  a.tw = c->d_tw[axis];
-  a.coef = coef;
-  a.nrm = (double)c->ngrid;
-  a.n = n[axis];
-  a.inner = inner;
-  a.ncols = (long long)(c->ngrid / (size_t)n[axis]);
-  a.sg = sg;
+}  // extern "C"
+
+// Columns per block of the complex passes: 8 (whole 128-byte lines) while their tile fits, else 4.
+static int dft_cols(int n) { return n <= 128 ? 8 : 4; }
+
+template <typename F8, typename F4>
+static void launch_dft(hipStream_t st, const DftArgs &a, int tiles, F8 f8, F4 f4) {
+  const int cols = dft_cols(a.n);
+  const size_t shm = sizeof(double2) * (size_t)a.n * (1 + tiles * cols);
+  const dim3 grid((unsigned)((a.ncols + cols - 1) / cols));
+  if (cols == 8) hipLaunchKernelGGL(f8, grid, dim3(256), shm, st, a);
+  else hipLaunchKernelGGL(f4, grid, dim3(256), shm, st, a);
+}
+
+static VlocArgs vloc_args(salmon_hip_t c, const double *vpsl, const double *vh, const double *vxc, const double *rho,
+                          const double *vmix, double *vout) {
+  VlocArgs a;
+  a.vpsl = vpsl; a.vh = vh; a.vxc = vxc; a.rho = rho; a.vmix = vmix;
+  a.V = c->d_V;
+  a.vout = vout;
+  a.n = c->ngrid;
+  a.nspin = c->nspin;
   a.skip = c->d_skip;
-  // about one output per thread; columns per block a power of two in [1, 32]
-  int cols = 1;
-  while (cols < 32 && 2 * cols * a.n <= 256) cols *= 2;
-  a.cols = cols;
-  const unsigned nblk = (unsigned)((a.ncols + cols - 1) / cols);
-  const size_t shm = sizeof(double2) * (size_t)a.n * cols;
-  hipLaunchKernelGGL(k_dft_axis, dim3(nblk), dim3(256), shm, c->stream, a);
-  LAUNCHCHK("k_dft_axis");
-  return 0;
+  return a;
 }
 
 // Hartree potential of rho (+ rho2 when not null: the total density of two spin channels,
-// rho_s(1) + rho_s(2), src/rt/time_evolution_step.f90:166-169, formed in the first pass)
-static int hartree_impl(salmon_hip_t c, const double *rho_dev, const double *rho2_dev, double *vh_dev) {
-  double2 *b0 = c->d_fft[0], *b1 = c->d_fft[1];
-  int rc;
-  if ((rc = launch_dft(c, 2, -1.0, rho_dev, nullptr, b0, nullptr, nullptr, rho2_dev))) return rc;
-  if ((rc = launch_dft(c, 1, -1.0, nullptr, b0, b1, nullptr, nullptr))) return rc;
-  if ((rc = launch_dft(c, 0, -1.0, nullptr, b1, b0, nullptr, c->d_gcoef))) return rc;
-  if ((rc = launch_dft(c, 2, 1.0, nullptr, b0, b1, nullptr, nullptr))) return rc;
-  if ((rc = launch_dft(c, 1, 1.0, nullptr, b1, b0, nullptr, nullptr))) return rc;
-  return launch_dft(c, 0, 1.0, nullptr, b0, nullptr, vh_dev, nullptr);
+// rho_s(1) + rho_s(2), src/rt/time_evolution_step.f90:166-169, formed in the first pass) into vh_dev, or
+// where that is null straight into the local potential (v)
+static int hartree_impl(salmon_hip_t c, const double *rho_dev, const double *rho2_dev, double *vh_dev, const VlocArgs *v) {
+  const int plane = c->nx * c->ny, nkz = c->nz / 2 + 1;
+  DftArgs a;
+  memset(&a, 0, sizeof(a));
+  a.skip = c->d_skip;
+  a.coef = c->d_gcoef;
+  a.rn = 1.0 / (double)c->ngrid;
+  a.sg = -1.0;
+  a.rho = rho_dev;
+  a.rho2 = rho2_dev;
+  a.out = c->d_fft[0];
+  a.tw = c->d_tw[2];
+  a.n = c->nz; a.inner = plane; a.ncols = plane;
+  hipLaunchKernelGGL(k_dft_zr, dim3((unsigned)((plane + 15) / 16)), dim3(256), sizeof(double2) * c->nz * 9, c->stream, a);
+  LAUNCHCHK("k_dft_zr");
+  a.in = c->d_fft[0]; a.out = c->d_fft[1];
+  a.tw = c->d_tw[1];
+  a.n = c->ny; a.inner = c->nx; a.ncols = nkz * c->nx;
+  launch_dft(c->stream, a, 1, k_dft_y<8>, k_dft_y<4>);
+  LAUNCHCHK("k_dft_y");
+  a.in = a.out = c->d_fft[1];
+  a.tw = c->d_tw[0];
+  a.n = c->nx; a.inner = 1; a.ncols = nkz * c->ny;
+  launch_dft(c->stream, a, 2, k_dft_x<8>, k_dft_x<4>);
+  LAUNCHCHK("k_dft_x");
+  a.sg = 1.0;
+  a.in = c->d_fft[1]; a.out = c->d_fft[0];
+  a.tw = c->d_tw[1];
+  a.n = c->ny; a.inner = c->nx; a.ncols = nkz * c->nx;
+  launch_dft(c->stream, a, 1, k_dft_y<8>, k_dft_y<4>);
+  LAUNCHCHK("k_dft_y");
+  a.in = c->d_fft[0]; a.out = nullptr;
+  a.tw = c->d_tw[2];
+  a.n = c->nz; a.inner = plane; a.ncols = plane;
+  a.vh = vh_dev;
+  if (!vh_dev) a.v = *v;
+  launch_dft(c->stream, a, 1, k_dft_zi<8>, k_dft_zi<4>);
+  LAUNCHCHK("k_dft_zi");
+  return 0;
 }
+
+extern "C" {
 
 int salmon_hip_hartree(salmon_hip_t c, const double *rho_dev, double *vh_dev) {
   if (int rc = check(c)) return rc;
   if (!rho_dev || !vh_dev) return fail(SALMON_HIP_EINVAL, "null pointer");
   if (!c->have_cell) return fail(SALMON_HIP_ESTATE, "set_poisson not called");
-  return hartree_impl(c, rho_dev, nullptr, vh_dev);
+  return hartree_impl(c, rho_dev, nullptr, vh_dev, nullptr);
 }
 
 int salmon_hip_xc_pz(salmon_hip_t c, const double *rho_dev, double *vxc_dev, double *exc_dev) {
@@ -3889,26 +4044,15 @@ int salmon_hip_xc_pz(salmon_hip_t c, const double *rho_dev, double *vxc_dev, dou
   return 0;
 }
 
-static int launch_vlocal(salmon_hip_t c, const double *vpsl, const double *vh, const double *vxc,
-                         const double *rho, const double *vmix, double *vout) {
-  VlocArgs a;
-  a.vpsl = vpsl; a.vh = vh; a.vxc = vxc; a.rho = rho; a.vmix = vmix;
-  a.V = c->d_V;
-  a.vout = vout;
-  a.n = c->ngrid;
-  a.nspin = c->nspin;
-  a.skip = c->d_skip;
-  hipLaunchKernelGGL(k_update_vlocal, dim3((unsigned)((c->ngrid + 255) / 256)), dim3(256), 0, c->stream, a);
-  LAUNCHCHK("k_update_vlocal");
-  c->have_V = true;
-  return 0;
-}
-
 int salmon_hip_update_vlocal(salmon_hip_t c, const double *vpsl_dev, const double *vh_dev, const double *vxc_dev,
                              const double *vmix_dev, double *vout_dev) {
   if (int rc = check(c)) return rc;
   if (!vpsl_dev || !vh_dev || !vxc_dev) return fail(SALMON_HIP_EINVAL, "null pointer");
-  return launch_vlocal(c, vpsl_dev, vh_dev, vxc_dev, nullptr, vmix_dev, vout_dev);
+  const VlocArgs a = vloc_args(c, vpsl_dev, vh_dev, vxc_dev, nullptr, vmix_dev, vout_dev);
+  hipLaunchKernelGGL(k_update_vlocal, dim3((unsigned)((c->ngrid + 255) / 256)), dim3(256), 0, c->stream, a);
+  LAUNCHCHK("k_update_vlocal");
+  c->have_V = true;
+  return 0;
 }
 
 int salmon_hip_vlocal_extrapolate(salmon_hip_t c, double *vold1_dev, double *vold2_dev, double *vout_dev) {
@@ -3927,8 +4071,10 @@ int salmon_hip_update_potential(salmon_hip_t c, const double *rho_dev, const dou
   if (int rc = check(c)) return rc;
   if (!rho_dev || !vpsl_dev) return fail(SALMON_HIP_EINVAL, "null pointer");
   if (!c->have_cell) return fail(SALMON_HIP_ESTATE, "set_poisson not called");
-  if (int rc = hartree_impl(c, rho_dev, c->nspin == 2 ? rho_dev + c->ngrid : nullptr, c->d_vh)) return rc;
-  return launch_vlocal(c, vpsl_dev, c->d_vh, nullptr, rho_dev, vmix_dev, vout_dev);
+  const VlocArgs v = vloc_args(c, vpsl_dev, nullptr, nullptr, rho_dev, vmix_dev, vout_dev);
+  if (int rc = hartree_impl(c, rho_dev, c->nspin == 2 ? rho_dev + c->ngrid : nullptr, nullptr, &v)) return rc;
+  c->have_V = true;
+  return 0;
 }
 
 // ---------------------------------------------------------------------------
