@@ -646,6 +646,7 @@ struct StencilArgs {
   size_t osz;
   int nx, ny, nz, ly, nspin, nb, nk;
   int TY, TZ, nyt, nzt, nblk;
+  int TX, nxt;            // x tiles (stencil_tilez with XT; else one tile of nx)
   const int *skip;        // device flag: the launch does nothing when it is set (null: never)
 };
 
@@ -1277,14 +1278,20 @@ __device__ __forceinline__ void stencil_tile8(const StencilArgs &a, int bid, dou
 // the slot (kept in a 4-deep register queue), pushes p's own value into a 9-deep queue of own
 // values (planes p-8 .. p) and completes plane p-4 with its z part.  The centre, x/y and z
 // partial sums are added in that order (hh = ((V t + klap0 t) - v_xy/2 + i w_xy) - v_z/2 + i w_z),
-// a regrouping of stencil_tile's sum.  Needs TZ % 4 == 0; the z loop runs TZ + 4 planes,
-// unrolled by 4 so that slot and queue indices are compile-time.  A slot holds NCK chunks of 64
-// elements (8: rows of up to 32 points; 10: 13 rows of 48 points, so that the 48-point rows keep
+// a regrouping of stencil_tile's sum.  Any number of planes: the z loop runs TZ + 4 planes
+// (rounded up to 4), unrolled by 4 so that slot and queue indices are compile-time (a break per
+// plane instead of the rounding cost 1% at 32^3).  A slot holds NCK chunks of 64 elements (8: rows of up to 32 points; 10: 13 rows of 48 points, so that the 48-point rows keep
 // three blocks per CU; 12: up to 64 points); chunk c is moved by wave c % 4, and a wave with no
 // chunk left for its last DMA of a plane moves its previous chunk again (the same data to the
 // same place), so that every wave issues the same number of operations per plane.
 // ---------------------------------------------------------------------------
-template <typename TI, typename R, typename TO, int NCK>
+// XT: tiles of TX x TY points with a halo on x too, for rows above 64 points (full rows would leave two
+// or three of them per tile beside 8 halo rows).  HBM-bound; 96 x 14 x 12, 512 orbitals: 188 us with full
+// rows (stencil_tile), 100 us so; the last term 244 and 174 us.
+// NC >= 0 (FP64): the last term with the Taylor sum over NC earlier terms.  Their values at plane p - 4
+// come two planes ahead through per-lane LDS slots (a wave reads only what it moved itself: no barrier).
+// 32^3, 1024 orbitals: 593 us, 80 bytes a point at 4.5 TB/s (620 us in stencil_tile, one plane ahead).
+template <typename TI, typename R, typename TO, int NCK, bool XT = false, int NC = -1>
 __device__ __forceinline__ void stencil_tilez(const StencilArgs &a, int bid, double2 *lds) {
   using CH = typename Cx<R>::T;
   constexpr int BS = kTile;
@@ -1292,10 +1299,15 @@ __device__ __forceinline__ void stencil_tilez(const StencilArgs &a, int bid, dou
   constexpr unsigned EB = sizeof(TI);
   constexpr int SLOT = 64 * NCK;              // elements per slot: (TY + 8) * nx <= 64 NCK
   constexpr int NW = (NCK + 3) / 4;           // tile DMA chunks per wave and plane
-  constexpr int kOps = NW * WI + 2 + 1;
+  constexpr int NCB = NC > 0 ? NC : 0;
+  static_assert(NC < 0 || std::is_same<TI, double2>::value, "the Taylor sum here is FP64");
+  constexpr int kOps = NCB + NW * WI + 2 + 1;
   TI *tileR = (TI *)lds;                      // 4 x SLOT
   double *vR = (double *)(tileR + 4 * SLOT);  // 4 x BS
+  double2 *combR = (double2 *)(vR + 4 * BS);  // 2 x NC x BS
 
+  const int xtile = XT ? bid % a.nxt : 0;
+  if (XT) bid /= a.nxt;
   const int ytile = bid % a.nyt;
   const int zt = (bid / a.nyt) % a.nzt;
   const int b = bid / (a.nyt * a.nzt);
@@ -1308,21 +1320,25 @@ __device__ __forceinline__ void stencil_tilez(const StencilArgs &a, int bid, dou
   const int z1 = min(z0 + a.TZ, nz);
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
-  const int ntile = TY * nx;
+  const int TX = XT ? a.TX : nx;           // points of a tile row
+  const int SW = XT ? TX + 8 : nx;         // elements of a slot row
+  const int x0 = xtile * TX;
+  const int ntile = TY * TX;
   const bool active = tid < ntile;
   const int te = active ? tid : 0;
-  const int tx = te % nx, ty = te / nx;
+  const int tx = te % TX, ty = te / TX;
   const int y = y0 + ty;
-  const bool outY = active && y < ny;
+  const bool outY = active && y < ny && (!XT || x0 + tx < nx);
   const size_t zs = (size_t)nx * ly;
   const size_t orbOff = (size_t)b * a.osz;
   const TI *in = (const TI *)a.in + orbOff;
-  const size_t colOff = (size_t)tx + (size_t)nx * wrapi(y, ny);
+  const size_t colOff = (size_t)(XT ? wrapi(x0 + tx, nx) : tx) + (size_t)nx * wrapi(y, ny);
   const size_t gplane = (size_t)nx * ny;
-  const int nslot = (TY + 8) * nx;
+  const int nslot = (TY + 8) * SW;
   auto sofs = [&](int e) {
     const int ec = e < nslot ? e : 0;
-    return (size_t)(ec % nx) + (size_t)nx * wrapi(y0 - 4 + ec / nx, ny);
+    const int ex = XT ? wrapi(x0 - 4 + ec % SW, nx) : ec % SW;
+    return (size_t)ex + (size_t)nx * wrapi(y0 - 4 + ec / SW, ny);
   };
   size_t toff[NW][2];
   unsigned kofs[NW];  // slot offset (elements) of the chunk of this wave's k-th DMA, wave-uniform
@@ -1339,7 +1355,8 @@ __device__ __forceinline__ void stencil_tilez(const StencilArgs &a, int bid, dou
   for (int kk = 0; kk < 2; ++kk) {
     const int e = 64 * wave + 32 * kk + (lane >> 1);
     const int ec = e < ntile ? e : 0;
-    voff[kk] = 2 * ((size_t)(ec % nx) + (size_t)nx * wrapi(y0 + ec / nx, ny)) + (lane & 1);
+    const int ex = XT ? wrapi(x0 + ec % TX, nx) : ec % TX;
+    voff[kk] = 2 * ((size_t)ex + (size_t)nx * wrapi(y0 + ec / TX, ny)) + (lane & 1);
   }
   const double *Vb = a.V + (size_t)ispin * gplane * nz;
   const unsigned tileA = __builtin_amdgcn_readfirstlane(lds_addr(tileR) + EB * 64u * wave);
@@ -1354,14 +1371,20 @@ __device__ __forceinline__ void stencil_tilez(const StencilArgs &a, int bid, dou
     dma4(vb + voff[0], vA + 8u * BS * slot);
     dma4(vb + voff[1], vA + 8u * BS * slot + 256u);
   };
-  const int own = (ty + 4) * nx + tx;
+  const unsigned combA = __builtin_amdgcn_readfirstlane(lds_addr(combR) + 16u * 64u * wave);
+  auto dma_comb = [&](int plane, int slot) {
+    const size_t at = orbOff + colOff + zs * plane;
+#pragma unroll
+    for (int n = 0; n < NCB; ++n) dma16((const double2 *)a.comb[n] + at, combA + 16u * BS * (NCB * slot + n));
+  };
+  const int own = (ty + 4) * SW + tx + (XT ? 4 : 0);
   int xo[8], yo[8];
 #pragma unroll
   for (int n = 1; n <= 4; ++n) {
-    xo[n - 1] = (ty + 4) * nx + wrapi(tx + n, nx);
-    xo[3 + n] = (ty + 4) * nx + wrapi(tx - n, nx);
-    yo[n - 1] = (ty + 4 + n) * nx + tx;
-    yo[3 + n] = (ty + 4 - n) * nx + tx;
+    xo[n - 1] = XT ? own + n : (ty + 4) * nx + wrapi(tx + n, nx);
+    xo[3 + n] = XT ? own - n : (ty + 4) * nx + wrapi(tx - n, nx);
+    yo[n - 1] = own + n * SW;
+    yo[3 + n] = own - n * SW;
   }
   const double *kp = a.kpar + 16 * ik;
   const R klap0 = (R)kp[0];
@@ -1377,7 +1400,7 @@ __device__ __forceinline__ void stencil_tilez(const StencilArgs &a, int bid, dou
   // (periodic z), whose own values are kept from the first pass: the tail needs only those
   // (no x/y part is formed there), so it fetches nothing from HBM (its slot DMAs re-read the
   // last plane, an L2 hit, to keep the per-plane memory-op count fixed).
-  const bool wrapkeep = a.nzt == 1;
+  const bool wrapkeep = a.nzt == 1 && nz % 4 == 0;  // the slot of a tail plane is then its own index
   CH keep[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -1396,14 +1419,23 @@ __device__ __forceinline__ void stencil_tilez(const StencilArgs &a, int bid, dou
 
   auto body = [&](int p, auto ph) {
     constexpr int P = decltype(ph)::v;
-    wait_vm<2 * kOps>();
+    wait_vm<2 * kOps - NCB>();
     __syncthreads();
+    // the sum's values of plane p - 4, then its slot's next ones (plane p - 2)
+    double2 cc[NCB > 0 ? NCB : 1];
+    if constexpr (NCB > 0) {
+#pragma unroll
+      for (int n = 0; n < NCB; ++n) cc[n] = combR[BS * (NCB * (P & 1) + n) + tid];
+#pragma unroll
+      for (int n = 0; n < NCB; ++n) asm volatile("" : "+v"(cc[n].x), "+v"(cc[n].y)::"memory");
+      dma_comb(min(max(p - 2, z0), z1 - 1), P & 1);
+    }
     dma_tile(p + 3 < z1 ? p + 3 : (wrapkeep ? z1 - 1 : min(p + 3, z1 + 3)), (P + 3) & 3);
     dma_v(min(p + 3, z1 - 1), (P + 3) & 3);
     const TI *T = tileR + SLOT * P;
 #pragma unroll
     for (int i = 0; i < 8; ++i) q[i] = q[i + 1];
-    // in the tail of a whole-column chunk p = z1 + P wraps to plane P (z0 = 0, TZ % 4 == 0)
+    // in the tail of a whole-column chunk p = z1 + P wraps to plane P (z0 = 0, nz % 4 == 0)
     q[8] = (wrapkeep && p >= z1) ? keep[P] : cvt2<CH>(T[own]);
     if (p < z0 + 4) keep[P] = q[8];
     const CH hp = hq[P];  // plane p - 4
@@ -1440,10 +1472,22 @@ __device__ __forceinline__ void stencil_tilez(const StencilArgs &a, int bid, dou
     CH hh;
     hh.x = hp.x - (R)0.5 * v.x + w.y;
     hh.y = hp.y - (R)0.5 * v.y - w.x;
-    // every lane stores every plane (the vm count per plane is fixed): the first four planes
-    // of the chunk and lanes without a point store into the sink
-    const bool outP = outY && p >= z0 + 4;
+    // every lane stores every plane (the vm count per plane is fixed): the first four planes of
+    // the chunk, what the loop runs past its last one and lanes without a point go to the sink
+    const bool outP = outY && (unsigned)(p - z0 - 4) < (unsigned)(z1 - z0);
     TO *dst = outP ? (TO *)a.hout + orbOff + colOff + zs * (p - 4) : (TO *)a.sink + tid;
+    if constexpr (NC >= 0) {
+      auto add = [](double2 &o, double2 zc, double2 v) {
+        o.x = o.x + (zc.x * v.x - zc.y * v.y);
+        o.y = o.y + (zc.x * v.y + zc.y * v.x);
+      };
+      double2 od = NC > 0 ? cc[0] : q[4];
+#pragma unroll
+      for (int n = 1; n < NC; ++n) add(od, a.zc[n - 1], cc[n]);
+      if (NC > 0) add(od, a.zc[NC > 0 ? NC - 1 : 0], q[4]);
+      add(od, a.zc[NC >= 0 ? NC : 0], hh);
+      hh = od;
+    }
     *dst = cvt2<TO>(hh);
   };
   for (int p = z0; p < z1 + 4; p += 4) {
@@ -1455,32 +1499,28 @@ __device__ __forceinline__ void stencil_tilez(const StencilArgs &a, int bid, dou
   wait_vm<0>();
 }
 
-template <typename TI, typename R, typename TO, int NCK>
+template <typename TI, typename R, typename TO, int NCK, bool XT, int NC>
 __global__ __launch_bounds__(kTile) void k_stencilz(StencilArgs a) {
   extern __shared__ double2 lds[];
   if (a.skip && *a.skip) return;  // a device-side gate switched this launch off
   int bid = blockIdx.x;
   const int nfull = (a.nblk / 8) * 8;
   if (bid < nfull) bid = (bid % 8) * (a.nblk / 8) + bid / 8;  // XCD-aware tile order
-  stencil_tilez<TI, R, TO, NCK>(a, bid, lds);
+  stencil_tilez<TI, R, TO, NCK, XT, NC>(a, bid, lds);
 }
 
-// Persistent form over many systems (the batched step's terms without the Taylor sum): block b
-// takes tiles b, b + grid, ... of `tiles` = (system index, tile index).  stencil_tilez returns
-// with its DMAs drained (vmcnt 0); the barrier keeps the next tile's DMAs off slots that other
-// waves still read.
-template <typename TI, typename R, typename TO, int NCK>
+// Over many systems (the batched step): block b takes tile `tiles[b]` = (system index, tile index).  One
+// tile per block: a persistent loop over tiles keeps 10 more registers live and its blocks end
+// unevenly (8 systems, 12 to 36 points an axis: 94 us a term and 119 us the last, 85 and 110 us so).
+template <typename TI, typename R, typename TO, int NCK, int NC>
 __global__ __launch_bounds__(kTile) void k_stencilz_packed(const StencilArgs *__restrict__ sys,
-                                                           const int2 *__restrict__ tiles, int ntiles) {
+                                                           const int2 *__restrict__ tiles) {
   extern __shared__ double2 lds[];
-  for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
-    const int2 tr = tiles[t];
-    const int si = __builtin_amdgcn_readfirstlane(tr.x);
-    const int bid = __builtin_amdgcn_readfirstlane(tr.y);
-    const StencilArgs a = sys[si];
-    stencil_tilez<TI, R, TO, NCK>(a, bid, lds);
-    __syncthreads();
-  }
+  const int2 tr = tiles[blockIdx.x];
+  const int si = __builtin_amdgcn_readfirstlane(tr.x);
+  const int bid = __builtin_amdgcn_readfirstlane(tr.y);
+  const StencilArgs a = sys[si];
+  stencil_tilez<TI, R, TO, NCK, false, NC>(a, bid, lds);
 }
 
 template <typename TI, typename R, typename TO, int NCH, bool PR>
@@ -2515,7 +2555,6 @@ struct salmon_hip_ctx {
   int tile_plane = -1, mid_nzt = 0;
   bool tile8 = true;  // stencil_tile8 for the mixed middle terms where the shape allows it
   bool small_grid = true;  // k_taylor_small where the grid fits (salmon_hip_set_launch_shape turns it off)
-  bool tilez = true;  // stencil_tilez for the FP64 ones and the mixed first term (before stencil_tile8)
   // salmon_hip_set_skip: device flag read by the launches of hpsi/taylor, density and the
   // potential update (they do nothing while it is set); null = none
   const int *d_skip = nullptr;
@@ -3089,21 +3128,32 @@ static bool tile8_fits(const salmon_hip_ctx *c, int stage, int nc, const Stencil
 // the paired dwordx4 DMAs need rows of even length and 16-byte aligned orbital blocks
 static bool tile8_pairs(const StencilArgs &a) { return a.nx % 2 == 0 && a.osz % 2 == 0; }
 
-// y tiles with the delayed z part (stencil_tilez): the FP64 terms without the Taylor sum and the
-// mixed first term (FP64 input), z chunks of 4k planes; a plane's tile and halo rows fill a slot
-// of 8, 10 or 12 64-element chunks (rows of up to 32 points; 48-point rows take 5 tile rows,
-// 13 x 48 = 624 elements in 10 chunks; up to 64 points).
-static bool tilez_fits(const salmon_hip_ctx *c, int stage, int nc, const StencilArgs &a) {
-  return ((stage == kStagePlain && nc < 0) || stage == kStageMixedFirst) && a.nx <= 64 &&
-         (a.TY + 8) * a.nx <= 3 * kTile && a.TY * a.nx <= kTile && a.TZ % 4 == 0 && a.nz % 4 == 0 && c->tilez;
+// Taylor sums over up to 3 earlier terms (order 4): the slots of 4 or 5 would leave one block of
+// stencil_tilez per CU (88 KB and more) where stencil_tile's shorter rings leave two.
+constexpr int kTilezComb = 3;
+
+// y tiles with the delayed z part (stencil_tilez): the FP64 terms on rows of up to 64 points and any
+// number of planes; the mixed first term (FP64 input) on z chunks of 4k planes, elsewhere it keeps
+// stencil_tile's order of the FP32 sum.  A plane's tile and halo rows fill a slot of 8, 10 or 12
+// 64-element chunks (rows of up to 32 points; 48-point rows take 5 tile rows, 13 x 48 = 624
+// elements in 10 chunks; up to 64 points).
+static bool tilez_fits(int stage, int nc, const StencilArgs &a) {
+  const bool fp64 = stage == kStagePlain && nc <= kTilezComb;
+  return (fp64 || (stage == kStageMixedFirst && a.TZ % 4 == 0 && a.nz % 4 == 0)) && a.nx <= 64 &&
+         (a.TY + 8) * a.nx <= 3 * kTile && a.TY * a.nx <= kTile;
 }
 
-template <typename TI, typename R, typename TO, int NCK>
+template <typename TI, int NCK, int NC>
+static constexpr size_t tilez_lds() {
+  return sizeof(TI) * 4 * 64 * NCK + sizeof(double) * 4 * kTile + sizeof(double2) * 2 * (NC > 0 ? NC : 0) * kTile;
+}
+
+template <typename TI, typename R, typename TO, int NCK, bool XT, int NC>
 static int launch_tilez_n(salmon_hip_ctx *c, dim3 grid, hipEvent_t e0, hipEvent_t e1, const StencilArgs &a) {
-  const size_t shmem = sizeof(TI) * 4 * 64 * NCK + sizeof(double) * 4 * kTile;
+  const size_t shmem = tilez_lds<TI, NCK, NC>();
   static std::atomic<unsigned long long> attr_dev{0};
-  if (int rc = lds_attr((const void *)k_stencilz<TI, R, TO, NCK>, attr_dev, shmem)) return rc;
-  hipExtLaunchKernelGGL((k_stencilz<TI, R, TO, NCK>), grid, dim3(kTile), shmem, c->stream, e0, e1, 0, a);
+  if (int rc = lds_attr((const void *)k_stencilz<TI, R, TO, NCK, XT, NC>, attr_dev, shmem)) return rc;
+  hipExtLaunchKernelGGL((k_stencilz<TI, R, TO, NCK, XT, NC>), grid, dim3(kTile), shmem, c->stream, e0, e1, 0, a);
   return 0;
 }
 
@@ -3113,13 +3163,47 @@ static int tilez_chunks(int TY, int nx) {
   return need <= 8 * 64 ? 8 : (need <= 10 * 64 ? 10 : 12);
 }
 
-template <typename TI, typename R, typename TO>
+template <typename TI, typename R, typename TO, bool XT = false, int NC = -1>
 static int launch_tilez_t(salmon_hip_ctx *c, dim3 grid, hipEvent_t e0, hipEvent_t e1, const StencilArgs &a) {
-  switch (tilez_chunks(a.TY, a.nx)) {
-    case 8: return launch_tilez_n<TI, R, TO, 8>(c, grid, e0, e1, a);
-    case 10: return launch_tilez_n<TI, R, TO, 10>(c, grid, e0, e1, a);
-    default: return launch_tilez_n<TI, R, TO, 12>(c, grid, e0, e1, a);
+  switch (tilez_chunks(a.TY, XT ? a.TX + 8 : a.nx)) {
+    case 8: return launch_tilez_n<TI, R, TO, 8, XT, NC>(c, grid, e0, e1, a);
+    case 10: return launch_tilez_n<TI, R, TO, 10, XT, NC>(c, grid, e0, e1, a);
+    default: return launch_tilez_n<TI, R, TO, 12, XT, NC>(c, grid, e0, e1, a);
   }
+}
+
+template <bool XT>
+static int launch_tilez_fp64(salmon_hip_ctx *c, int nc, dim3 grid, hipEvent_t e0, hipEvent_t e1, const StencilArgs &a) {
+  switch (nc) {
+    case -1: return launch_tilez_t<double2, double, double2, XT>(c, grid, e0, e1, a);
+    case 0: return launch_tilez_t<double2, double, double2, XT, 0>(c, grid, e0, e1, a);
+    case 1: return launch_tilez_t<double2, double, double2, XT, 1>(c, grid, e0, e1, a);
+    case 2: return launch_tilez_t<double2, double, double2, XT, 2>(c, grid, e0, e1, a);
+    default: return launch_tilez_t<double2, double, double2, XT, 3>(c, grid, e0, e1, a);
+  }
+}
+
+// Tiles of at most 256 points with a halo on x and y for rows above 64 points: the split of the plane
+// that moves the fewest slot chunks.
+static void tilez_xtiles(StencilArgs &a) {
+  int best = INT_MAX;
+  for (int nxt = 2; nxt <= 16; ++nxt) {
+    const int TX = (a.nx + nxt - 1) / nxt;
+    for (int nyt = 1; nyt <= a.ny; ++nyt) {
+      const int TY = (a.ny + nyt - 1) / nyt;
+      if (TX * TY > kTile || (TX + 8) * (TY + 8) > 12 * 64) continue;
+      const int cost = ((a.nx + TX - 1) / TX) * ((a.ny + TY - 1) / TY) * tilez_chunks(TY, TX + 8);
+      if (cost < best) {
+        best = cost;
+        a.TX = TX;
+        a.TY = TY;
+      }
+      break;
+    }
+  }
+  a.nxt = (a.nx + a.TX - 1) / a.TX;
+  a.nyt = (a.ny + a.TY - 1) / a.TY;
+  a.nblk = a.nk * a.nb * a.nxt * a.nyt * a.nzt;
 }
 
 template <typename TI, typename R, typename TO, int NCH, bool PR>
@@ -3153,15 +3237,8 @@ static int launch_stencil_hc(salmon_hip_ctx *c, int stage, int nc, dim3 grid, hi
       default: return launch_stencil_t<float2, float, double2, HC, 5>(c, grid, e0, e1, a);
     }
   }
-  switch (nc) {
-    case -1: return launch_stencil_t<double2, double, double2, HC, -1>(c, grid, e0, e1, a);
-    case 0: return launch_stencil_t<double2, double, double2, HC, 0>(c, grid, e0, e1, a);
-    case 1: return launch_stencil_t<double2, double, double2, HC, 1>(c, grid, e0, e1, a);
-    case 2: return launch_stencil_t<double2, double, double2, HC, 2>(c, grid, e0, e1, a);
-    case 3: return launch_stencil_t<double2, double, double2, HC, 3>(c, grid, e0, e1, a);
-    case 4: return launch_stencil_t<double2, double, double2, HC, 4>(c, grid, e0, e1, a);
-    default: return launch_stencil_t<double2, double, double2, HC, 5>(c, grid, e0, e1, a);
-  }
+  if (nc == 4) return launch_stencil_t<double2, double, double2, HC, 4>(c, grid, e0, e1, a);
+  return launch_stencil_t<double2, double, double2, HC, 5>(c, grid, e0, e1, a);
 }
 
 extern "C" {
@@ -3285,6 +3362,7 @@ static StencilArgs stencil_args(salmon_hip_t c, const void *in, void *hout, bool
   a.nx = c->nx; a.ny = c->ny; a.nz = c->nz; a.ly = c->ly;
   a.nspin = c->nspin; a.nb = c->nb; a.nk = c->nk;
   a.TY = c->TY; a.TZ = c->TZ; a.nyt = c->nyt; a.nzt = c->nzt;
+  a.TX = c->nx; a.nxt = 1;
   // terms without the Taylor sum use whole xy-plane tiles when a plane fits one block
   const int plane = c->nx * c->ny;
   // rule (tile_plane = -1): whole planes only up to 256 points (one 256-thread block); the
@@ -3321,10 +3399,14 @@ static int launch_hpsi(salmon_hip_t c, int kind, const void *in, void *hout, boo
   if (bs == 256) rc = launch_stencil_plane<256>(c, stage, grid, e0, e1, a);
   else if (bs == 512) rc = launch_stencil_wp<1>(c, stage, grid, e0, e1, a);
   else if (bs == 1024) rc = launch_stencil_wp<2>(c, stage, grid, e0, e1, a);
-  else if (tilez_fits(c, stage, nc, a))
-    rc = stage == kStagePlain ? launch_tilez_t<double2, double, double2>(c, grid, e0, e1, a)
+  else if (tilez_fits(stage, nc, a))
+    rc = stage == kStagePlain ? launch_tilez_fp64<false>(c, nc, grid, e0, e1, a)
                               : launch_tilez_t<double2, float, float2>(c, grid, e0, e1, a);
   else if (tile8_fits(c, stage, nc, a)) rc = launch_tile8_t<float2, float, float2>(c, grid, e0, e1, a);
+  else if (stage == kStagePlain && nc <= kTilezComb && a.nx > 64) {
+    tilez_xtiles(a);
+    rc = launch_tilez_fp64<true>(c, nc, dim3((unsigned)a.nblk), e0, e1, a);
+  }
   else if (hc <= 1) rc = launch_stencil_hc<1>(c, stage, nc, grid, e0, e1, a);
   else if (hc <= 2) rc = launch_stencil_hc<2>(c, stage, nc, grid, e0, e1, a);
   else if (hc <= 4) rc = launch_stencil_hc<4>(c, stage, nc, grid, e0, e1, a);
@@ -4113,15 +4195,17 @@ int launch_packed_t(hipStream_t st, const StencilArgs *sys, const int2 *tiles, i
 
 template <int HC>
 int launch_packed_hc(hipStream_t st, int nc, const StencilArgs *sys, const int2 *tiles, int ntiles, int grid) {
-  switch (nc) {
-    case -1: return launch_packed_t<HC, -1>(st, sys, tiles, ntiles, grid);
-    case 0: return launch_packed_t<HC, 0>(st, sys, tiles, ntiles, grid);
-    case 1: return launch_packed_t<HC, 1>(st, sys, tiles, ntiles, grid);
-    case 2: return launch_packed_t<HC, 2>(st, sys, tiles, ntiles, grid);
-    case 3: return launch_packed_t<HC, 3>(st, sys, tiles, ntiles, grid);
-    case 4: return launch_packed_t<HC, 4>(st, sys, tiles, ntiles, grid);
-    default: return launch_packed_t<HC, 5>(st, sys, tiles, ntiles, grid);
+  if (nc == 4) return launch_packed_t<HC, 4>(st, sys, tiles, ntiles, grid);
+  if (nc == 5) return launch_packed_t<HC, 5>(st, sys, tiles, ntiles, grid);
+  if constexpr (HC > 2) {  // rows of up to 64 points take the delayed-z tiles there
+    switch (nc) {
+      case -1: return launch_packed_t<HC, -1>(st, sys, tiles, ntiles, grid);
+      case 1: return launch_packed_t<HC, 1>(st, sys, tiles, ntiles, grid);
+      case 2: return launch_packed_t<HC, 2>(st, sys, tiles, ntiles, grid);
+      case 3: return launch_packed_t<HC, 3>(st, sys, tiles, ntiles, grid);
+    }
   }
+  return fail(SALMON_HIP_EINVAL, "batch stencil form");
 }
 
 int launch_packed(hipStream_t st, int hc, int nc, const StencilArgs *sys, const int2 *tiles, int ntiles, int grid) {
@@ -4131,24 +4215,34 @@ int launch_packed(hipStream_t st, int hc, int nc, const StencilArgs *sys, const 
   return launch_packed_hc<8>(st, nc, sys, tiles, ntiles, grid);
 }
 
-template <int NCK>
-int launch_packed_z_t(hipStream_t st, const StencilArgs *sys, const int2 *tiles, int ntiles, int grid) {
-  const size_t shmem = sizeof(double2) * 4 * 64 * NCK + sizeof(double) * 4 * kTile;
+template <int NCK, int NC>
+int launch_packed_z_t(hipStream_t st, const StencilArgs *sys, const int2 *tiles, int ntiles) {
+  const size_t shmem = tilez_lds<double2, NCK, NC>();
   static std::atomic<unsigned long long> attr_dev{0};
-  if (int rc = lds_attr((const void *)k_stencilz_packed<double2, double, double2, NCK>, attr_dev, shmem))
+  if (int rc = lds_attr((const void *)k_stencilz_packed<double2, double, double2, NCK, NC>, attr_dev, shmem))
     return rc;
-  hipLaunchKernelGGL((k_stencilz_packed<double2, double, double2, NCK>), dim3(grid), dim3(kTile), shmem, st, sys,
-                     tiles, ntiles);
+  hipLaunchKernelGGL((k_stencilz_packed<double2, double, double2, NCK, NC>), dim3(ntiles), dim3(kTile), shmem, st, sys,
+                     tiles);
   LAUNCHCHK("k_stencilz_packed");
   return 0;
 }
 
-// the delayed-z y tiles for the terms without the Taylor sum, slots of nck 64-element chunks
-int launch_packed_z(hipStream_t st, int nck, const StencilArgs *sys, const int2 *tiles, int ntiles, int grid) {
+// the delayed-z y tiles, slots of nck 64-element chunks
+template <int NC>
+int launch_packed_z_n(hipStream_t st, int nck, const StencilArgs *sys, const int2 *tiles, int ntiles) {
   switch (nck) {
-    case 8: return launch_packed_z_t<8>(st, sys, tiles, ntiles, grid);
-    case 10: return launch_packed_z_t<10>(st, sys, tiles, ntiles, grid);
-    default: return launch_packed_z_t<12>(st, sys, tiles, ntiles, grid);
+    case 8: return launch_packed_z_t<8, NC>(st, sys, tiles, ntiles);
+    case 10: return launch_packed_z_t<10, NC>(st, sys, tiles, ntiles);
+    default: return launch_packed_z_t<12, NC>(st, sys, tiles, ntiles);
+  }
+}
+
+int launch_packed_z(hipStream_t st, int nck, int nc, const StencilArgs *sys, const int2 *tiles, int ntiles) {
+  switch (nc) {
+    case -1: return launch_packed_z_n<-1>(st, nck, sys, tiles, ntiles);
+    case 1: return launch_packed_z_n<1>(st, nck, sys, tiles, ntiles);
+    case 2: return launch_packed_z_n<2>(st, nck, sys, tiles, ntiles);
+    default: return launch_packed_z_n<3>(st, nck, sys, tiles, ntiles);
   }
 }
 
@@ -4339,7 +4433,7 @@ int batch_tables(salmon_hip_batch *b) {
     bool zok = g.hc <= 2;
     for (int i : g.mem) {
       const salmon_hip_t c = b->h[i];
-      zok = zok && c->tilez && c->nx <= 64 && c->nz % 4 == 0 && c->TY * c->nx <= kTile &&
+      zok = zok && c->nx <= 64 && c->TY * c->nx <= kTile &&
             (c->TY + 8) * c->nx <= 3 * kTile;
       zch = std::max(zch, tilez_chunks(c->TY, c->nx));
     }
@@ -4359,14 +4453,18 @@ int batch_tables(salmon_hip_batch *b) {
           c->mid_nzt = b->z_chunks;
           StencilArgs a = stencil_args(c, hh[n - 1], fin ? out : hh[n], fin, hh, n - 1, b->zc.data(), &bs, true);
           c->mid_nzt = save;
-          if (g.zch && !fin) {
+          if (g.zch) {  // whole groups of four planes (the kernel's loop) but in the last chunk
             a.TZ = (a.TZ + 3) / 4 * 4;
             a.nzt = (a.nz + a.TZ - 1) / a.TZ;
             a.nblk = c->norb * a.nyt * a.nzt;
           }
           args.push_back(a);
           if (p == 0 && (n == 1 || fin))
-            for (int t = 0; t < a.nblk; ++t) tiles[fin ? 1 : 0].push_back(make_int2((int)m, t));
+            for (int t = 0; t < a.nblk; ++t) {
+              // neighbouring tiles on one XCD, as in the per-system launches
+              const int n8 = a.nblk / 8, u = t < n8 * 8 ? (t % 8) * n8 + t / 8 : t;
+              tiles[fin ? 1 : 0].push_back(make_int2((int)m, u));
+            }
         }
     for (int k = 0; k < 2; ++k) {
       dfree(g.d_tiles[k]);
@@ -4387,8 +4485,8 @@ int batch_stencil(salmon_hip_batch *b, int p, int n) {
   for (auto &g : b->groups) {
     const StencilArgs *args = g.d_args + ((size_t)p * b->n_hamil + (n - 1)) * g.mem.size();
     const int k = nc >= 0 ? 1 : 0;
-    const int rc = (nc < 0 && g.zch) ? launch_packed_z(b->stream, g.zch, args, g.d_tiles[0], g.ntiles[0], g.grid[0])
-                                     : launch_packed(b->stream, g.hc, nc, args, g.d_tiles[k], g.ntiles[k], g.grid[k]);
+    const int rc = (nc <= kTilezComb && g.zch) ? launch_packed_z(b->stream, g.zch, nc, args, g.d_tiles[k], g.ntiles[k])
+                                               : launch_packed(b->stream, g.hc, nc, args, g.d_tiles[k], g.ntiles[k], g.grid[k]);
     if (rc) return rc;
   }
   return 0;
