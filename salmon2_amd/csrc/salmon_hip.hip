@@ -234,15 +234,101 @@ __device__ __forceinline__ int xcd_order(int b, int nblk) {
   return b < nfull ? (b % 8) * (nblk / 8) + b / 8 : b;
 }
 
-// LMX bounds the projectors of one atom (the tile and staging sizes)
+// Waves of a block on parts of the sphere (ProjStage's S): 4 where the operand staging is small, 1 where
+// four private stagings of it would cost more than they spread (d projectors under five weights,
+// 512 orbitals at 96 x 14 x 12: 79 us split, 57 us not; s+p projectors, 1024 orbitals at 32^3: 187 us split
+// and 202 us not for the fused pass, 128 orbitals there 14 us and 21 us for the projection).  It depends on
+// nothing else and the chunks of S = 4 are of one length: every form sums a projection in one order.
+constexpr int proj_split(int lm) { return lm <= 4 ? 4 : 1; }
+constexpr int proj_orb(int lm) { return proj_split(lm) == 4 ? 16 : kProjOrb; }
+
+// Staging of the contraction.  S = 1: a block takes 64 orbitals, 16 per wave, and the waves share the
+// projectors of a chunk of JC sphere points; S = 4: a block takes 16 orbitals and its waves every
+// fourth chunk each, with the partial sums added in wave order at the end (launches of few blocks).
+// The A operand lies in LDS as MT tiles of 8 weighted projectors (complex) per point, unused ones
+// zero, so that a lane's value for an MFMA is one 8-byte read and a sign; the orbitals as 16 per
+// wave and point.  Both are XOR-swizzled: writes (lanes on points) and reads (lanes on projectors or
+// orbitals) both spread over the banks.
+template <int NW, int LMX>
+struct ProjStage {
+  static constexpr int S = proj_split(LMX);
+  static constexpr int JC = NW == 1 && S == 1 ? kProjJC : kProjJC / 2;
+  static constexpr int MT = (NW * LMX + 7) / 8;
+  static constexpr int OB = proj_orb(LMX);       // orbitals per block
+  static constexpr int kPer = JC / 4;                 // orbital values per lane and chunk
+  static constexpr int kT = S == 4 ? 64 : kBlock;     // threads that stage one chunk's projectors
+  static constexpr int kZPer = (JC * LMX + kT - 1) / kT;
+  double2 sp[4][JC * 16];
+  double2 z[S][JC * 8 * MT];
+  static __device__ __forceinline__ int zs(int jj, int lw) {
+    return jj * 8 * MT + (lw ^ (((jj >> 1) & 7) | (MT % 2 == 0 ? (jj & 1) << 3 : 0)));
+  }
+  static __device__ __forceinline__ int so(int jj, int o) { return jj * 16 + (o ^ (jj & 15)); }
+};
+typedef double __attribute__((ext_vector_type(4))) d4;
+
+template <int S>
+__device__ __forceinline__ void stage_sync() {
+  if constexpr (S == 1) {
+    __syncthreads();
+  } else {  // wave-private staging: LDS accesses of one wave stay in order
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+}
+
+// acc += A B over one staged chunk
+template <int NW, int LMX>
+__device__ __forceinline__ void stage_mfma(const double2 *sp, const double2 *z, int lane, int ntile, d4 *acc) {
+  using P = ProjStage<NW, LMX>;
+  const int h = (lane >> 4) >> 1, comp = (lane >> 4) & 1;  // K row: point 2 ks + h, re/im of psi
+  const int oc = lane & 15;                                // orbital column (B) / output row (A)
+  const int part = (oc >> 2) & 1, lw0 = (oc >> 3) * 4 + (oc & 3);
+  const double *spd = (const double *)sp + comp, *zd = (const double *)z + (part ^ comp);
+  const unsigned neg = part && !comp ? 0x80000000u : 0u;
+#pragma unroll 4
+  for (int ks = 0; ks < P::JC / 2; ++ks) {
+    const int jp = 2 * ks + h;
+    const double bval = spd[2 * P::so(jp, oc)];
+#pragma unroll
+    for (int tt = 0; tt < P::MT; ++tt) {
+      if (tt < ntile) {
+        const double v = zd[2 * P::zs(jp, tt * 8 + lw0)];
+        const double aval = __hiloint2double(__double2hiint(v) ^ neg, __double2loint(v));
+        acc[tt] = __builtin_amdgcn_mfma_f64_16x16x4f64(aval, bval, acc[tt], 0, 0, 0);
+      }
+    }
+  }
+}
+
+// S = 4: the waves' sums into wave 0's, in wave order (red: 3 x MT x 64 d4, over the staging)
+template <int MT>
+__device__ __forceinline__ void stage_reduce(d4 *red, int wave, int lane, d4 *acc) {
+  __syncthreads();
+  if (wave > 0)
+#pragma unroll
+    for (int tt = 0; tt < MT; ++tt) red[((wave - 1) * MT + tt) * 64 + lane] = acc[tt];
+  __syncthreads();
+  if (wave == 0)
+#pragma unroll
+    for (int tt = 0; tt < MT; ++tt)
+      for (int w = 0; w < 3; ++w) acc[tt] += red[(w * MT + tt) * 64 + lane];
+}
+
+// LMX bounds the projectors of one atom (the tile and staging sizes).  Bound by the gathers: a sphere's
+// points of one orbital are runs of a few points, and nearly every 128-byte line of the orbitals is
+// read.  With the A values formed per wave from unswizzled tables (45 vector instructions an MFMA) NW = 5 took
+// 264 us for 64 atoms, 32^3 and 1024 orbitals, 131 us so (0.6 GB of lines, 4.6 TB/s), and 1183 and 692 us for
+// 216 atoms, 48^3 and 1728 orbitals (5.1 TB/s); NW = 1 for 64 atoms and 128 orbitals 37 and 14 us.
 template <int NW, typename TP, int LMX>
 __device__ __forceinline__ void proj_body(const ProjArgs &a, int bid) {
   static_assert(LMX <= kMaxLmaPerAtom, "LMX bounds the projectors of one atom");
-  constexpr int MAXT = (NW * LMX + 7) / 8;
-  __shared__ double2 sp[kProjJC][kProjOrb];
-  __shared__ double2 zsh[kProjJC][LMX];
-  __shared__ double2 zsh2[NW == 5 ? kProjJC : 1][LMX];
-  __shared__ double rsh[kProjJC][3];
+  using P = ProjStage<NW, LMX>;
+  constexpr int S = P::S, JC = P::JC, MT = P::MT;
+  constexpr size_t kRed = S == 4 ? sizeof(d4) * 3 * MT * 64 : 0;
+  __shared__ __attribute__((aligned(32))) char lds[sizeof(P) > kRed ? sizeof(P) : kRed];
+  P &st = *(P *)lds;
   const int grp = bid % a.ngrp;
   const int t = bid / a.ngrp;
   const int ia = t % a.natom;
@@ -254,55 +340,48 @@ __device__ __forceinline__ void proj_body(const ProjArgs &a, int bid) {
   const int nlw = NW * al.y;            // (lma, weight) pairs of this atom
   const int ntile = (nlw + 7) >> 3;     // 8 lw (16 rows) per MFMA tile
   const size_t kbase = (size_t)ik * a.nb;
+  const int ob0 = grp * P::OB + (S == 4 ? 0 : 16 * wave);  // first orbital of this wave
+  double2 *sp = st.sp[wave], *z = st.z[S == 4 ? wave : 0];
+  const int zt = S == 4 ? lane : (int)threadIdx.x;
 
-  typedef double __attribute__((ext_vector_type(4))) d4;
-  d4 acc[MAXT];
+  d4 acc[MT];
 #pragma unroll
-  for (int tt = 0; tt < MAXT; ++tt) acc[tt] = d4{0.0, 0.0, 0.0, 0.0};
+  for (int tt = 0; tt < MT; ++tt) acc[tt] = d4{0.0, 0.0, 0.0, 0.0};
+  for (int e = zt; e < JC * 8 * ntile; e += P::kT)
+    if (e / JC >= nlw) z[P::zs(e % JC, e / JC)] = make_double2(0.0, 0.0);
 
-  const int kq = lane >> 4;      // K row of this lane (0..3)
-  const int comp = kq & 1;       // 0: re, 1: im of psi
-  const int oc = lane & 15;      // orbital column (B) / output row (A)
-
-  // psi at kProjJC sphere points for the block's 64 orbitals: chunk j0 + kProjJC is loaded into
-  // registers while the MFMAs consume chunk j0 from LDS
-  constexpr int kPer = (kProjJC * kProjOrb) / kBlock;
-  constexpr int kZPer = (kProjJC * LMX + kBlock - 1) / kBlock;
-  TP pre[kPer];
-  double2 zpre[kZPer], zpre2[NW == 5 ? kZPer : 1];
-  double rpre = 0.0;
+  // the next chunk is loaded into registers while the MFMAs consume the staged one
+  TP pre[P::kPer];
+  double2 zpre[P::kZPer], zpre2[NW == 5 ? P::kZPer : 1];
+  double rpre[3] = {0.0, 0.0, 0.0};
   const TP *psi = (const TP *)a.psi;
   const int *jx = a.jidx + (size_t)a.nps * ia;
   const double2 *zk = a.zekr + (size_t)a.nps * ((size_t)al.x + (size_t)a.nlma * ik);
   const double2 *zk2 = NW == 5 ? a.zekr2 + (size_t)a.nps * ((size_t)al.x + (size_t)a.nlma * ik) : nullptr;
-  // every thread loads the same sphere point of each chunk (kBlock is a multiple of kProjJC);
-  // its grid index is fetched one chunk ahead, so the psi gathers wait on one load, not two
-  static_assert(kBlock % kProjJC == 0, "one sphere point per thread and chunk");
-  const int jt = threadIdx.x % kProjJC;
-  int jnext = jt < m ? jx[jt] : 0;
+  // every thread loads the same sphere point of each chunk; its grid index is fetched one chunk
+  // ahead, so the psi gathers wait on one load, not two
+  const int jt = lane % JC, o0 = lane / JC, l0 = zt / JC;
+  constexpr int kStep = S * JC;
+  const int jb = S == 4 ? wave * JC : 0;
+  int jnext = jb + jt < m ? jx[jb + jt] : 0;
   auto load_chunk = [&](int j0) {
     const int jv = jnext;
-    jnext = j0 + kProjJC + jt < m ? jx[j0 + kProjJC + jt] : 0;
+    const int j = j0 + jt;
+    jnext = j + kStep < m ? jx[j + kStep] : 0;
 #pragma unroll
-    for (int r = 0; r < kZPer; ++r) {
-      const int e = threadIdx.x + kBlock * r;  // (l, jj) = (e / kProjJC, e % kProjJC)
-      const int jj = e % kProjJC, l = e / kProjJC;
-      const int j = j0 + jj;
+    for (int r = 0; r < P::kZPer; ++r) {
+      const int l = l0 + (P::kT / JC) * r;
       zpre[r] = (j < m && l < al.y) ? zk[(size_t)j + (size_t)a.nps * l] : make_double2(0.0, 0.0);
       if constexpr (NW == 5)
         zpre2[r] = (j < m && l < al.y) ? zk2[(size_t)j + (size_t)a.nps * l] : make_double2(0.0, 0.0);
     }
-    if (NW > 1 && threadIdx.x < 3 * kProjJC) {
-      const int j = j0 + threadIdx.x / 3;
-      rpre = j < m ? a.rxyz[3 * ((size_t)j0 + (size_t)a.nps * ia) + threadIdx.x] : 0.0;
+    if constexpr (NW > 1) {
+#pragma unroll
+      for (int i = 0; i < 3; ++i) rpre[i] = j < m ? a.rxyz[3 * ((size_t)j + (size_t)a.nps * ia) + i] : 0.0;
     }
 #pragma unroll
-    for (int r = 0; r < kPer; ++r) {
-      const int e = threadIdx.x + kBlock * r;
-      const int jj = e % kProjJC;
-      const int o = e / kProjJC;
-      const int j = j0 + jj;
-      const int ob = grp * kProjOrb + o;
+    for (int r = 0; r < P::kPer; ++r) {
+      const int ob = ob0 + o0 + (64 / JC) * r;
       TP v;
       v.x = 0;
       v.y = 0;
@@ -310,62 +389,39 @@ __device__ __forceinline__ void proj_body(const ProjArgs &a, int bid) {
       pre[r] = v;
     }
   };
-  load_chunk(0);
-  for (int j0 = 0; j0 < m; j0 += kProjJC) {
+  load_chunk(jb);
+  for (int j0 = jb; j0 < m; j0 += kStep) {
 #pragma unroll
-    for (int r = 0; r < kPer; ++r) {
-      const int e = threadIdx.x + kBlock * r;
-      sp[e % kProjJC][e / kProjJC] = cvt2<double2>(pre[r]);
-    }
+    for (int r = 0; r < P::kPer; ++r) sp[P::so(jt, o0 + (64 / JC) * r)] = cvt2<double2>(pre[r]);
 #pragma unroll
-    for (int r = 0; r < kZPer; ++r) {
-      const int e = threadIdx.x + kBlock * r;
-      if (e < kProjJC * LMX) zsh[e % kProjJC][e / kProjJC] = zpre[r];
-      if constexpr (NW == 5)
-        if (e < kProjJC * LMX) zsh2[e % kProjJC][e / kProjJC] = zpre2[r];
-    }
-    if (NW > 1 && threadIdx.x < 3 * kProjJC) rsh[threadIdx.x / 3][threadIdx.x % 3] = rpre;
-    __syncthreads();
-    if (j0 + kProjJC < m) load_chunk(j0 + kProjJC);
-#pragma unroll 2
-    for (int ks = 0; ks < kProjJC / 2; ++ks) {
-      const int jp = 2 * ks + (kq >> 1);
-      const int j = j0 + jp;
-      const double2 pv = sp[jp][wave * 16 + oc];
-      const double bval = comp ? pv.y : pv.x;
-      double zr = 0.0, zi = 0.0, rw[3] = {0.0, 0.0, 0.0};
-      const bool jv = j < m;
-      if (jv && NW > 1) {
-        rw[0] = rsh[jp][0];
-        rw[1] = rsh[jp][1];
-        rw[2] = rsh[jp][2];
-      }
+    for (int r = 0; r < P::kZPer; ++r) {
+      const int l = l0 + (P::kT / JC) * r;
+      if (l < al.y) {
+        if constexpr (NW == 1) {
+          z[P::zs(jt, l)] = zpre[r];
+        } else {
+          z[P::zs(jt, l * NW)] = zpre[r];
 #pragma unroll
-      for (int tt = 0; tt < MAXT; ++tt) {
-        if (tt < ntile) {
-          const int part = (oc >> 2) & 1;
-          const int lw = tt * 8 + (oc >> 3) * 4 + (oc & 3);
-          double aval = 0.0;
-          if (jv && lw < nlw) {
-            const int w = lw % NW;
-            const int l = lw / NW;
-            const double2 z = (NW == 5 && w == 4) ? zsh2[jp][l] : zsh[jp][l];
-            const double r = (w == 0 || w == 4) ? 1.0 : rw[w - 1];
-            zr = z.x * r;
-            zi = z.y * r;
-            aval = part == 0 ? (comp ? zi : zr) : (comp ? zr : -zi);
-          }
-          acc[tt] = __builtin_amdgcn_mfma_f64_16x16x4f64(aval, bval, acc[tt], 0, 0, 0);
+          for (int i = 0; i < 3; ++i) z[P::zs(jt, l * NW + 1 + i)] = make_double2(zpre[r].x * rpre[i], zpre[r].y * rpre[i]);
+          if constexpr (NW == 5) z[P::zs(jt, l * NW + 4)] = zpre2[r];
         }
       }
     }
-    __syncthreads();
+    stage_sync<S>();
+    if (j0 + kStep < m) load_chunk(j0 + kStep);
+    stage_mfma<NW, LMX>(sp, z, lane, ntile, acc);
+    stage_sync<S>();
+  }
+  if constexpr (S == 4) {
+    stage_reduce<MT>((d4 *)lds, wave, lane, acc);
+    if (wave > 0) return;
   }
   // lane (kq, oc) holds rows kq + 4r: r = 2h -> re of lw = 8t + 4h + kq, r = 2h+1 -> its im
-  const int ob = grp * kProjOrb + wave * 16 + oc;
+  const int kq = lane >> 4;
+  const int ob = ob0 + (lane & 15);
   if (ob >= a.nb) return;
 #pragma unroll
-  for (int tt = 0; tt < MAXT; ++tt) {
+  for (int tt = 0; tt < MT; ++tt) {
     if (tt >= ntile) break;
 #pragma unroll
     for (int hh = 0; hh < 2; ++hh) {
@@ -388,8 +444,9 @@ __device__ __forceinline__ void proj_body(const ProjArgs &a, int bid) {
   }
 }
 
+// up to 4 projectors per atom the registers leave four waves per SIMD
 template <int NW, typename TP, int LMX>
-__global__ __launch_bounds__(kBlock) void k_proj(ProjArgs a) {
+__global__ __launch_bounds__(kBlock, LMX == 4 ? 4 : 2) void k_proj(ProjArgs a) {
   if (a.skip && *a.skip) return;  // a device-side gate switched this launch off
   proj_body<NW, TP, LMX>(a, xcd_order(blockIdx.x, gridDim.x));
 }
@@ -398,15 +455,17 @@ __global__ __launch_bounds__(kBlock) void k_proj(ProjArgs a) {
 // KB term of one H application fused with the projection of its result: for a Taylor term
 // h = H h_prev the pass adds s * sum_lma c_prev(lma) zekr(j, lma) at the sphere points that one
 // (atom, point) pair covers alone and projects the completed h onto the atom's projectors (the
-// c of the next term), reading h once.  Block = (k, atom, 64 orbitals) as in k_proj<1>: each
-// thread owns one sphere point of every 32-point chunk and 8 of the orbitals; after the chunk is
+// c of the next term), reading h once.  Block = (k, atom, orbitals) as in k_proj<1>: each
+// lane owns one sphere point of every chunk and part of the orbitals; after the chunk is
 // staged in LDS it completes its points (exclusive ones: KB sum in ascending ilma, in FP64, then
 // rounded to TP as k_nl_scatter stores it), writes them back and puts the rounded values into the
 // LDS tile the MFMAs read.  Points covered by several pairs are completed beforehand by
 // k_nl_scatter over their list, and no point is written by two blocks (an exclusive point
 // belongs to one atom, and the blocks of one atom split the orbitals), so the pass is
 // deterministic and race-free.  c_prev for the block's orbitals is staged in dynamic LDS
-// (cmax x 64 elements).
+// (cmax x orbitals of the block).  Bound by the lines read and written back: 64 atoms, 32^3, 1024
+// orbitals 213 us before the A values were staged and the points split over the waves, 187 us so
+// (0.9 GB, 4.8 TB/s); 216 atoms, 48^3, 1728 orbitals in complex FP32 990 and 953 us (4 GB).
 // ---------------------------------------------------------------------------
 struct ProjScatArgs {
   ProjArgs p;              // projection of h (p.psi = h, p.out = its c, scaled by rinv)
@@ -420,12 +479,12 @@ template <typename TP, int LM>
 __device__ __forceinline__ void proj_scatter_body(const ProjScatArgs &A, int bid) {
   static_assert(LM <= kMaxLmaPerAtom, "LM bounds the projectors of one atom");
   const ProjArgs &a = A.p;
-  constexpr int MAXT = (LM + 7) / 8;
-  // rows padded by one element: the per-point accesses of the completion step (lanes on points)
-  // then fall on different banks
-  __shared__ double2 sp[kProjJC][kProjOrb + 1];
-  __shared__ double2 zsh[kProjJC][LM + 1];
-  extern __shared__ double2 csh[];  // cmax x kProjOrb
+  using P = ProjStage<1, LM>;
+  constexpr int S = P::S, JC = P::JC, MT = P::MT;
+  constexpr size_t kRed = S == 4 ? sizeof(d4) * 3 * MT * 64 : 0;
+  __shared__ __attribute__((aligned(32))) char lds[sizeof(P) > kRed ? sizeof(P) : kRed];
+  P &st = *(P *)lds;
+  extern __shared__ double2 csh[];  // cmax x OB
   const int grp = bid % a.ngrp;
   const int t = bid / a.ngrp;
   const int ia = t % a.natom;
@@ -437,77 +496,74 @@ __device__ __forceinline__ void proj_scatter_body(const ProjScatArgs &A, int bid
   const int nlw = al.y;
   const int ntile = (nlw + 7) >> 3;
   const size_t kbase = (size_t)ik * a.nb;
+  const int ow = S == 4 ? 0 : 16 * wave;  // first orbital of this wave within the block
+  double2 *sp = st.sp[wave], *z = st.z[S == 4 ? wave : 0];
+  const int zt = S == 4 ? lane : (int)threadIdx.x;
 
-  for (int e = threadIdx.x; e < al.y * kProjOrb; e += kBlock) {
-    const int l = e / kProjOrb, o = e % kProjOrb, ob = grp * kProjOrb + o;
+  for (int e = threadIdx.x; e < al.y * P::OB; e += kBlock) {
+    const int l = e / P::OB, ob = grp * P::OB + e % P::OB;
     csh[e] = ob < a.nb ? A.cin[((size_t)ik * a.nlma + al.x + l) * a.nb + ob] : make_double2(0.0, 0.0);
   }
+  for (int e = zt; e < JC * 8 * ntile; e += P::kT)
+    if (e / JC >= nlw) z[P::zs(e % JC, e / JC)] = make_double2(0.0, 0.0);
   __syncthreads();
 
-  typedef double __attribute__((ext_vector_type(4))) d4;
-  d4 acc[MAXT];
+  d4 acc[MT];
 #pragma unroll
-  for (int tt = 0; tt < MAXT; ++tt) acc[tt] = d4{0.0, 0.0, 0.0, 0.0};
-  const int kq = lane >> 4;
-  const int comp = kq & 1;
-  const int oc = lane & 15;
-
-  constexpr int kPer = (kProjJC * kProjOrb) / kBlock;
-  constexpr int kZPer = (kProjJC * LM + kBlock - 1) / kBlock;
-  TP pre[kPer];
-  double2 zpre[kZPer];
-  TP *h = (TP *)a.psi;
+  for (int tt = 0; tt < MT; ++tt) acc[tt] = d4{0.0, 0.0, 0.0, 0.0};
+  TP pre[P::kPer];
+  double2 zpre[P::kZPer];
   const int *jx = a.jidx + (size_t)a.nps * ia;
   const int *jxe = A.jexcl + (size_t)a.nps * ia;
   const double2 *zk = a.zekr + (size_t)a.nps * ((size_t)al.x + (size_t)a.nlma * ik);
-  static_assert(kBlock % kProjJC == 0, "one sphere point per thread and chunk");
-  const int jt = threadIdx.x % kProjJC;
-  const int o0 = threadIdx.x / kProjJC;  // this thread's orbitals: o0 + (kBlock / kProjJC) r
-  int jnext = jt < m ? jx[jt] : 0;
-  int xnext = jt < m ? jxe[jt] : -1;
+  const int jt = lane % JC, o0 = ow + lane / JC, l0 = zt / JC;
+  TP *h = (TP *)a.psi + (kbase + grp * P::OB + o0) * a.osz;
+  const size_t hs = (64 / JC) * a.osz;
+  const int nor = a.nb - grp * P::OB - o0;  // orbitals of this lane: r with (64 / JC) r < nor
+  constexpr int kStep = S * JC;
+  const int jb = S == 4 ? wave * JC : 0;
+  int jnext = jb + jt < m ? jx[jb + jt] : 0;
+  int xnext = jb + jt < m ? jxe[jb + jt] : -1;
   int jload = 0, xload = -1;  // point offset and exclusive offset of the chunk last loaded
   double2 zown[LM];           // zekr of this thread's point of that chunk (exclusive points only)
   auto load_chunk = [&](int j0) {
     jload = jnext;
     xload = xnext;
+    const int j = j0 + jt;
 #pragma unroll
     for (int l = 0; l < LM; ++l)
-      zown[l] = (xload >= 0 && l < al.y) ? zk[(size_t)(j0 + jt) + (size_t)a.nps * l] : make_double2(0.0, 0.0);
-    const bool more = j0 + kProjJC + jt < m;
-    jnext = more ? jx[j0 + kProjJC + jt] : 0;
-    xnext = more ? jxe[j0 + kProjJC + jt] : -1;
+      zown[l] = (xload >= 0 && l < al.y) ? zk[(size_t)j + (size_t)a.nps * l] : make_double2(0.0, 0.0);
+    const bool more = j + kStep < m;
+    jnext = more ? jx[j + kStep] : 0;
+    xnext = more ? jxe[j + kStep] : -1;
 #pragma unroll
-    for (int r = 0; r < kZPer; ++r) {
-      const int e = threadIdx.x + kBlock * r;
-      const int jj = e % kProjJC, l = e / kProjJC;
-      const int j = j0 + jj;
+    for (int r = 0; r < P::kZPer; ++r) {
+      const int l = l0 + (P::kT / JC) * r;
       zpre[r] = (j < m && l < al.y) ? zk[(size_t)j + (size_t)a.nps * l] : make_double2(0.0, 0.0);
     }
 #pragma unroll
-    for (int r = 0; r < kPer; ++r) {
-      const int ob = grp * kProjOrb + o0 + (kBlock / kProjJC) * r;
+    for (int r = 0; r < P::kPer; ++r) {
       TP v;
       v.x = 0;
       v.y = 0;
-      if (j0 + jt < m && ob < a.nb) v = h[(kbase + ob) * a.osz + jload];
+      if (j < m && (64 / JC) * r < nor) v = h[r * hs + jload];
       pre[r] = v;
     }
   };
-  load_chunk(0);
-  for (int j0 = 0; j0 < m; j0 += kProjJC) {
+  load_chunk(jb);
+  for (int j0 = jb; j0 < m; j0 += kStep) {
     // complete this thread's point if one pair covers it (xload >= 0 implies j0 + jt < m) while
     // staging the chunk
 #pragma unroll
-    for (int r = 0; r < kPer; ++r) {
-      const int o = o0 + (kBlock / kProjJC) * r;
-      const int ob = grp * kProjOrb + o;
+    for (int r = 0; r < P::kPer; ++r) {
+      const int o = o0 + (64 / JC) * r;
       double2 v = cvt2<double2>(pre[r]);
-      if (xload >= 0 && ob < a.nb) {
+      if (xload >= 0 && (64 / JC) * r < nor) {
         double2 sum = make_double2(0.0, 0.0);
 #pragma unroll
         for (int l = 0; l < LM; ++l) {
           if (l < al.y) {
-            const double2 cv = csh[l * kProjOrb + o];
+            const double2 cv = csh[l * P::OB + o];
             sum.x += cv.x * zown[l].x - cv.y * zown[l].y;
             sum.y += cv.x * zown[l].y + cv.y * zown[l].x;
           }
@@ -515,45 +571,30 @@ __device__ __forceinline__ void proj_scatter_body(const ProjScatArgs &A, int bid
         v.x += A.s.x * sum.x - A.s.y * sum.y;
         v.y += A.s.x * sum.y + A.s.y * sum.x;
         const TP vt = cvt2<TP>(v);
-        h[(kbase + ob) * a.osz + jload] = vt;
+        h[r * hs + jload] = vt;
         v = cvt2<double2>(vt);
       }
-      sp[jt][o] = v;
+      sp[P::so(jt, o - ow)] = v;
     }
 #pragma unroll
-    for (int r = 0; r < kZPer; ++r) {
-      const int e = threadIdx.x + kBlock * r;
-      if (e < kProjJC * LM) zsh[e % kProjJC][e / kProjJC] = zpre[r];
+    for (int r = 0; r < P::kZPer; ++r) {
+      const int l = l0 + (P::kT / JC) * r;
+      if (l < al.y) z[P::zs(jt, l)] = zpre[r];
     }
-    __syncthreads();
-    if (j0 + kProjJC < m) load_chunk(j0 + kProjJC);
-#pragma unroll 2
-    for (int ks = 0; ks < kProjJC / 2; ++ks) {
-      const int jp = 2 * ks + (kq >> 1);
-      const int j = j0 + jp;
-      const double2 pv = sp[jp][wave * 16 + oc];
-      const double bval = comp ? pv.y : pv.x;
-      const bool jv = j < m;
-#pragma unroll
-      for (int tt = 0; tt < MAXT; ++tt) {
-        if (tt < ntile) {
-          const int part = (oc >> 2) & 1;
-          const int lw = tt * 8 + (oc >> 3) * 4 + (oc & 3);
-          double aval = 0.0;
-          if (jv && lw < nlw) {
-            const double2 z = zsh[jp][lw];
-            aval = part == 0 ? (comp ? z.y : z.x) : (comp ? z.x : -z.y);
-          }
-          acc[tt] = __builtin_amdgcn_mfma_f64_16x16x4f64(aval, bval, acc[tt], 0, 0, 0);
-        }
-      }
-    }
-    __syncthreads();
+    stage_sync<S>();
+    if (j0 + kStep < m) load_chunk(j0 + kStep);
+    stage_mfma<1, LM>(sp, z, lane, ntile, acc);
+    stage_sync<S>();
   }
-  const int ob = grp * kProjOrb + wave * 16 + oc;
+  if constexpr (S == 4) {
+    stage_reduce<MT>((d4 *)lds, wave, lane, acc);
+    if (wave > 0) return;
+  }
+  const int kq = lane >> 4;
+  const int ob = grp * P::OB + ow + (lane & 15);
   if (ob >= a.nb) return;
 #pragma unroll
-  for (int tt = 0; tt < MAXT; ++tt) {
+  for (int tt = 0; tt < MT; ++tt) {
     if (tt >= ntile) break;
 #pragma unroll
     for (int hh = 0; hh < 2; ++hh) {
@@ -568,7 +609,7 @@ __device__ __forceinline__ void proj_scatter_body(const ProjScatArgs &A, int bid
 }
 
 template <typename TP, int LM>
-__global__ __launch_bounds__(kBlock) void k_proj_scatter(ProjScatArgs A) {
+__global__ __launch_bounds__(kBlock, LM == 4 ? 4 : 2) void k_proj_scatter(ProjScatArgs A) {
   if (A.p.skip && *A.p.skip) return;  // a device-side gate switched this launch off
   proj_scatter_body<TP, LM>(A, xcd_order(blockIdx.x, gridDim.x));
 }
@@ -2978,7 +3019,10 @@ int salmon_hip_set_vec_ac(salmon_hip_t c, const double *vec_Ac) {
 }
 
 // projection of psi into out (c(nb, nlma, nk) scaled by rinv, or the current moments)
-static ProjArgs proj_args(salmon_hip_t c, const void *psi, double2 *out) {
+// The projector count that the projection kernels of atoms with up to cmax projectors are built for.
+static int proj_lm(int cmax) { return cmax <= 4 ? 4 : cmax <= 9 ? 9 : 16; }
+
+static ProjArgs proj_args(salmon_hip_t c, const void *psi, double2 *out, int lm) {
   ProjArgs a;
   a.psi = psi;
   a.zekr = c->d_zekr;
@@ -2994,7 +3038,7 @@ static ProjArgs proj_args(salmon_hip_t c, const void *psi, double2 *out) {
   a.natom = c->natom;
   a.nps = c->nps;
   a.nlma = c->nlma;
-  a.ngrp = (c->nb + kProjOrb - 1) / kProjOrb;
+  a.ngrp = (c->nb + proj_orb(lm) - 1) / proj_orb(lm);
   a.skip = c->d_skip;
   a.zekr2 = nullptr;
   a.out2 = nullptr;
@@ -3009,7 +3053,8 @@ static int launch_proj(salmon_hip_t c, const void *psi, int nw, bool f32 = false
     c->pre_state = 0;
     if (pre) return 0;
   }
-  ProjArgs a = proj_args(c, psi, nw == 1 ? c->d_c : c->d_curnl);
+  const int lmx = proj_lm(c->cmax);
+  ProjArgs a = proj_args(c, psi, nw == 1 ? c->d_c : c->d_curnl, lmx);
   if (nw == 5) {
     a.zekr2 = c->d_zekr_n;
     a.out2 = c->d_c;
@@ -3025,7 +3070,6 @@ static int launch_proj(salmon_hip_t c, const void *psi, int nw, bool f32 = false
     HIPCHK(hipStreamWaitEvent(c->side, c->ev_fork, 0));
     st = c->side;
   }
-  const int lmx = c->cmax <= 4 ? 4 : c->cmax <= 9 ? 9 : 16;
 #define PROJ_LAUNCH(NWv, TPv)                                                                             \
   do {                                                                                                   \
     if (lmx == 4) hipExtLaunchKernelGGL((k_proj<NWv, TPv, 4>), grid, dim3(kBlock), 0, st, e0, e1, 0, a);   \
@@ -3289,9 +3333,9 @@ static int launch_scatter(salmon_hip_t c, void *hout, double2 s, bool f32 = fals
 }
 
 // the fused KB pass of hout (cin = c of the previous term, cout = c of hout)
-static ProjScatArgs projscat_args(salmon_hip_t c, void *hout, const double2 *cin, double2 *cout) {
+static ProjScatArgs projscat_args(salmon_hip_t c, void *hout, const double2 *cin, double2 *cout, int lm) {
   ProjScatArgs A;
-  A.p = proj_args(c, hout, cout);
+  A.p = proj_args(c, hout, cout, lm);
   A.cin = cin;
   A.jexcl = c->d_jexcl;
   A.s = make_double2(1.0, 0.0);
@@ -3308,27 +3352,21 @@ static int launch_kb_fused(salmon_hip_t c, void *hout, bool f32) {
   const bool shared = c->ntp_shared > 0;
   if (shared)
     if (int rc = launch_scatter(c, hout, make_double2(1.0, 0.0), f32, true, e0, nullptr, false)) return rc;
-  const ProjScatArgs A = projscat_args(c, hout, c->d_c, c->d_c2);
-  const ProjArgs &a = A.p;
-  const size_t shmem = sizeof(double2) * (size_t)c->cmax * kProjOrb;
-  dim3 grid((unsigned)(a.ngrp * c->natom * c->nk));
+  const int lm = proj_lm(c->cmax);
+  const ProjScatArgs A = projscat_args(c, hout, c->d_c, c->d_c2, lm);
+  const size_t shmem = sizeof(double2) * (size_t)c->cmax * proj_orb(lm);
+  dim3 grid((unsigned)(A.p.ngrp * c->natom * c->nk));
   hipEvent_t s0 = shared ? nullptr : e0;
   // LM: registers for the projector values of one point (s+p: 4, up to d: 9, up to f: 16)
-  if (f32) {
-    if (c->cmax <= 4)
-      hipExtLaunchKernelGGL((k_proj_scatter<float2, 4>), grid, dim3(kBlock), shmem, c->stream, s0, e1, 0, A);
-    else if (c->cmax <= 9)
-      hipExtLaunchKernelGGL((k_proj_scatter<float2, 9>), grid, dim3(kBlock), shmem, c->stream, s0, e1, 0, A);
-    else
-      hipExtLaunchKernelGGL((k_proj_scatter<float2, 16>), grid, dim3(kBlock), shmem, c->stream, s0, e1, 0, A);
-  } else {
-    if (c->cmax <= 4)
-      hipExtLaunchKernelGGL((k_proj_scatter<double2, 4>), grid, dim3(kBlock), shmem, c->stream, s0, e1, 0, A);
-    else if (c->cmax <= 9)
-      hipExtLaunchKernelGGL((k_proj_scatter<double2, 9>), grid, dim3(kBlock), shmem, c->stream, s0, e1, 0, A);
-    else
-      hipExtLaunchKernelGGL((k_proj_scatter<double2, 16>), grid, dim3(kBlock), shmem, c->stream, s0, e1, 0, A);
-  }
+#define KB_LAUNCH(TPv)                                                                                                    \
+  do {                                                                                                                    \
+    if (lm == 4) hipExtLaunchKernelGGL((k_proj_scatter<TPv, 4>), grid, dim3(kBlock), shmem, c->stream, s0, e1, 0, A);      \
+    else if (lm == 9) hipExtLaunchKernelGGL((k_proj_scatter<TPv, 9>), grid, dim3(kBlock), shmem, c->stream, s0, e1, 0, A); \
+    else hipExtLaunchKernelGGL((k_proj_scatter<TPv, 16>), grid, dim3(kBlock), shmem, c->stream, s0, e1, 0, A);             \
+  } while (0)
+  if (f32) KB_LAUNCH(float2);
+  else KB_LAUNCH(double2);
+#undef KB_LAUNCH
   LAUNCHCHK("k_proj_scatter");
   std::swap(c->d_c, c->d_c2);
   c->pre_state = 0;
@@ -4256,7 +4294,8 @@ int launch_packed_z(hipStream_t st, int nck, int nc, const StencilArgs *sys, con
 // ranges of the bodies that order their blocks for the XCDs (projections, fused KB pass) are
 // padded to multiples of 8 blocks, so a local block index keeps its XCD (block b runs on XCD
 // b % 8); padding blocks return.  The per-system kernels and these run the same bodies on the
-// same records, so a packed step equals the per-system step bit for bit.
+// same records (a packed step differs from the per-system one only by the rounding of members that
+// take another form there).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ int pack_find(const int *off, int nsys, int b) {
   int lo = 0, hi = nsys;  // off[lo] <= b < off[hi]
@@ -4276,7 +4315,7 @@ __global__ __launch_bounds__(kBlock) void kp_update_kvector(const KvecArgs *args
 }
 
 template <int NW, int LMX>
-__global__ __launch_bounds__(kBlock) void kp_proj(const ProjArgs *args, const int *off, int nsys) {
+__global__ __launch_bounds__(kBlock, LMX == 4 ? 4 : 2) void kp_proj(const ProjArgs *args, const int *off, int nsys) {
   const int s = pack_find(off, nsys, blockIdx.x);
   const ProjArgs a = args[s];
   const int item = xcd_order((int)blockIdx.x - off[s], off[s + 1] - off[s]);
@@ -4285,7 +4324,7 @@ __global__ __launch_bounds__(kBlock) void kp_proj(const ProjArgs *args, const in
 }
 
 template <int LM>
-__global__ __launch_bounds__(kBlock) void kp_proj_scatter(const ProjScatArgs *args, const int *off, int nsys) {
+__global__ __launch_bounds__(kBlock, LM == 4 ? 3 : 2) void kp_proj_scatter(const ProjScatArgs *args, const int *off, int nsys) {
   const int s = pack_find(off, nsys, blockIdx.x);
   const ProjScatArgs A = args[s];
   const int item = xcd_order((int)blockIdx.x - off[s], off[s + 1] - off[s]);
@@ -4599,13 +4638,13 @@ int batch_packed_tables(salmon_hip_batch *b) {
     cmax = std::max(cmax, c->natom > 0 ? c->cmax : 0);
   }
   if (cmax > kMaxLmaPerAtom) return 0;
-  b->lm = cmax <= 4 ? 4 : cmax <= 9 ? 9 : 16;
+  b->lm = proj_lm(cmax);
   b->cm = cmax <= kScatCM ? kScatCM : 0;
   auto kb = [&](salmon_hip_t c) { return kb_fused_on(c); };
   auto scat_blocks = [&](salmon_hip_t c, int ntp) {
     return ntp > 0 ? ((ntp + kBlock - 1) / kBlock) * c->nk * ((c->nb + kScatG - 1) / kScatG) : 0;
   };
-  auto proj_blocks = [&](salmon_hip_t c) { return ((c->nb + kProjOrb - 1) / kProjOrb) * c->natom * c->nk; };
+  auto proj_blocks = [&](const ProjArgs &a) { return a.ngrp * a.natom * a.nk; };
   std::vector<int> cnt(ns);
   {
     std::vector<KvecArgs> r(ns);
@@ -4617,7 +4656,7 @@ int batch_packed_tables(salmon_hip_batch *b) {
   }
   size_t kb_shm = 0, cur_shm = 0;
   for (int i = 0; i < ns; ++i) {
-    kb_shm = std::max(kb_shm, sizeof(double2) * (size_t)b->h[i]->cmax * kProjOrb);
+    kb_shm = std::max(kb_shm, sizeof(double2) * (size_t)b->h[i]->cmax * proj_orb(b->lm));
     cur_shm = std::max(cur_shm, cur_shmem(b->h[i]));
   }
   for (int p = 0; p < 2; ++p) {
@@ -4630,8 +4669,8 @@ int batch_packed_tables(salmon_hip_batch *b) {
       salmon_hip_t c = b->h[i];
       void *hh[kMaxComb + 1], *out;
       batch_buffers(b, i, p, hh, &out);
-      pr[i] = proj_args(c, hh[0], c->d_c);
-      cnt[i] = kb(c) ? proj_blocks(c) : 0;
+      pr[i] = proj_args(c, hh[0], c->d_c, b->lm);
+      cnt[i] = kb(c) ? proj_blocks(pr[i]) : 0;
       const double2 *cl_buf = ((N - 1) % 2 == 1) ? c->d_c2 : c->d_c;
       last[i] = scatter_args(c, out, make_double2(b->zc[2 * (N - 1)], b->zc[2 * (N - 1) + 1]), cl_buf, false, false);
       cls[i] = kb(c) ? scat_blocks(c, c->ntp) : 0;
@@ -4639,8 +4678,8 @@ int batch_packed_tables(salmon_hip_batch *b) {
       const int gx = (int)((c->ngrid + kBlock - 1) / kBlock);
       cd[i] = gx * c->dens_ngrp * c->nspin;
       cs[i] = c->dens_ngrp > 1 ? (int)((c->ngrid * c->nspin + kBlock - 1) / kBlock) : 0;
-      p4[i] = proj_args(c, out, c->d_curnl);
-      c4[i] = c->natom > 0 ? proj_blocks(c) : 0;
+      p4[i] = proj_args(c, out, c->d_curnl, b->lm);
+      c4[i] = c->natom > 0 ? proj_blocks(p4[i]) : 0;
       cl[i] = cur_args(c, out);
       cl_n[i] = c->norb * c->nyt;
     }
@@ -4662,8 +4701,8 @@ int batch_packed_tables(salmon_hip_batch *b) {
         double2 *cout = (n % 2 == 1) ? c->d_c2 : c->d_c;
         sh[i] = scatter_args(c, hh[n], make_double2(1.0, 0.0), cin, true, false);
         shn[i] = kb(c) ? scat_blocks(c, c->ntp_shared) : 0;
-        fu[i] = projscat_args(c, hh[n], cin, cout);
-        fun[i] = kb(c) ? proj_blocks(c) : 0;
+        fu[i] = projscat_args(c, hh[n], cin, cout, b->lm);
+        fun[i] = kb(c) ? proj_blocks(fu[i].p) : 0;
       }
       if (int rc = pack_make(b, b->p_kbsh[p][n - 1], sh, shn, false)) return rc;
       if (int rc = pack_make(b, b->p_kbf[p][n - 1], fu, fun, true, kb_shm)) return rc;
