@@ -3216,6 +3216,35 @@ static int launch_tilez_t(salmon_hip_ctx *c, dim3 grid, hipEvent_t e0, hipEvent_
   }
 }
 
+// z chunks of the FP64 terms in stencil_tilez: a chunk moves 8 planes beside its own, so as few as keep
+// the chip busy.  With k blocks per CU a plane takes the larger of 0.65 us (one block's latency) and
+// 0.49 us k; that is within 15% of what 14 shapes measured (13 to 48 points an axis, 16 to 512 orbitals) and
+// picks the fastest of 1, 2, 3, 4 and 6 chunks for ten of them, the second for the rest.  Against 2048
+// blocks or chunks of 8 planes at least: 32^3, 128 orbitals 48 and 42 us, 13 x 28 x 57, 128 orbitals 49 and 41 us.
+static double tilez_planes(int nz, int nzt) {
+  const int TZ = (nz + nzt - 1) / nzt;
+  return (TZ + 7) / 4 * 4 + 4;
+}
+
+static void tilez_set_chunks(StencilArgs &a, int nzt) {
+  a.TZ = (a.nz + nzt - 1) / nzt;
+  a.nzt = (a.nz + a.TZ - 1) / a.TZ;
+  a.nblk = a.nk * a.nb * a.nxt * a.nyt * a.nzt;
+}
+
+static void tilez_zchunks(StencilArgs &a) {
+  const long tiles = (long)a.nk * a.nb * a.nxt * a.nyt;
+  int best = 1;
+  double tbest = 0.0;
+  for (int n = 1; n <= std::max(1, a.nz / 8); ++n) {
+    const double t = tilez_planes(a.nz, n) * std::max(0.65, 0.49 * ((tiles * n + 255) / 256));
+    if (n > 1 && t >= tbest) continue;
+    best = n;
+    tbest = t;
+  }
+  tilez_set_chunks(a, best);
+}
+
 template <bool XT>
 static int launch_tilez_fp64(salmon_hip_ctx *c, int nc, dim3 grid, hipEvent_t e0, hipEvent_t e1, const StencilArgs &a) {
   switch (nc) {
@@ -3437,15 +3466,16 @@ static int launch_hpsi(salmon_hip_t c, int kind, const void *in, void *hout, boo
   if (bs == 256) rc = launch_stencil_plane<256>(c, stage, grid, e0, e1, a);
   else if (bs == 512) rc = launch_stencil_wp<1>(c, stage, grid, e0, e1, a);
   else if (bs == 1024) rc = launch_stencil_wp<2>(c, stage, grid, e0, e1, a);
-  else if (tilez_fits(stage, nc, a))
-    rc = stage == kStagePlain ? launch_tilez_fp64<false>(c, nc, grid, e0, e1, a)
-                              : launch_tilez_t<double2, float, float2>(c, grid, e0, e1, a);
+  else if (tilez_fits(stage, nc, a) && stage == kStagePlain) {
+    if (c->mid_nzt == 0 || nc >= 0) tilez_zchunks(a);
+    rc = launch_tilez_fp64<false>(c, nc, dim3((unsigned)a.nblk), e0, e1, a);
+  } else if (tilez_fits(stage, nc, a)) rc = launch_tilez_t<double2, float, float2>(c, grid, e0, e1, a);
   else if (tile8_fits(c, stage, nc, a)) rc = launch_tile8_t<float2, float, float2>(c, grid, e0, e1, a);
   else if (stage == kStagePlain && nc <= kTilezComb && a.nx > 64) {
     tilez_xtiles(a);
+    if (c->mid_nzt == 0 || nc >= 0) tilez_zchunks(a);
     rc = launch_tilez_fp64<true>(c, nc, dim3((unsigned)a.nblk), e0, e1, a);
-  }
-  else if (hc <= 1) rc = launch_stencil_hc<1>(c, stage, nc, grid, e0, e1, a);
+  } else if (hc <= 1) rc = launch_stencil_hc<1>(c, stage, nc, grid, e0, e1, a);
   else if (hc <= 2) rc = launch_stencil_hc<2>(c, stage, nc, grid, e0, e1, a);
   else if (hc <= 4) rc = launch_stencil_hc<4>(c, stage, nc, grid, e0, e1, a);
   else rc = launch_stencil_hc<8>(c, stage, nc, grid, e0, e1, a);
@@ -4477,6 +4507,24 @@ int batch_tables(salmon_hip_batch *b) {
       zch = std::max(zch, tilez_chunks(c->TY, c->nx));
     }
     g.zch = zok ? zch : 0;
+    // the members' common number of z chunks by tilez_zchunks' measure of the whole group
+    int gz = 1;
+    double tbest = 0.0;
+    for (int n = 1; n <= 16; ++n) {
+      double sum = 0.0, lat = 0.0;
+      bool fits = n == 1;
+      for (int i : g.mem) {
+        const salmon_hip_t c = b->h[i];
+        const int ni = std::min(n, std::max(1, c->nz / 8));
+        fits = fits || ni == n;
+        sum += tilez_planes(c->nz, ni) * ((double)c->norb * c->nyt * ni);
+        lat = std::max(lat, tilez_planes(c->nz, ni));
+      }
+      const double t = std::max(0.65 * lat, 0.49 / 256 * sum);
+      if (!fits || (n > 1 && t >= tbest)) continue;
+      gz = n;
+      tbest = t;
+    }
     std::vector<int2> tiles[2];
     std::vector<StencilArgs> args;
     for (int p = 0; p < 2; ++p)
@@ -4492,8 +4540,9 @@ int batch_tables(salmon_hip_batch *b) {
           c->mid_nzt = b->z_chunks;
           StencilArgs a = stencil_args(c, hh[n - 1], fin ? out : hh[n], fin, hh, n - 1, b->zc.data(), &bs, true);
           c->mid_nzt = save;
-          if (g.zch) {  // whole groups of four planes (the kernel's loop) but in the last chunk
-            a.TZ = (a.TZ + 3) / 4 * 4;
+          if (g.zch) {
+            if (b->z_chunks == 0) tilez_set_chunks(a, std::min(gz, std::max(1, a.nz / 8)));
+            a.TZ = (a.TZ + 3) / 4 * 4;  // whole groups of four planes (the kernel's loop) but in the last chunk
             a.nzt = (a.nz + a.TZ - 1) / a.TZ;
             a.nblk = c->norb * a.nyt * a.nzt;
           }
