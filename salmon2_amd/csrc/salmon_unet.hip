@@ -207,8 +207,9 @@ __global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
 // shares in ascending order (k_wg_reduce).
 //
 // A wave per (tap, co tile, ci tile) gathering single 2-byte elements, three divisions each, took 91 us
-// per layer on average at 32^3 where the three kernels here take 20 (4 + 11 + 5); bound now by the
-// latency of the loads (288 waves at the finest level's 16 x 16 channels), not by the matrix cores.
+// per layer on average at 32^3 where the three kernels here take 20 (4 + 11 + 5) a layer at a time, bound
+// by the latency of the loads (288 waves at the finest level's 16 x 16 channels), not by the matrix
+// cores; all ten layers of a sample in one launch each take 74 us instead of 198 (11 + 54 + 10).
 // ---------------------------------------------------------------------------
 constexpr int kWgChunk = 1024;  // points per partial sum
 
@@ -224,11 +225,27 @@ struct WgArgs {
   int nx, ny, nz, npts, npad;  // npad: npts rounded up to whole 32-point steps (zeros past npts)
 };
 
+// Several layers in one launch: layer i owns the blocks [off[i], off[i + 1]).
+constexpr int kWgLayers = 10;
+struct WgAll {
+  WgArgs l[kWgLayers];
+  unsigned off[kWgLayers + 1];
+  int n;
+};
+
+__device__ __forceinline__ int wg_layer(const WgAll &A, unsigned b) {
+  int i = 0;
+  while (i + 1 < A.n && b >= A.off[i + 1]) ++i;
+  return i;
+}
+
 // one thread per (point, 8 channels): the input's threads, then dy's
-__global__ __launch_bounds__(256) void k_wg_pack(WgArgs a) {
+__global__ __launch_bounds__(256) void k_wg_pack(WgAll A) {
+  const int li = wg_layer(A, blockIdx.x);
+  const WgArgs &a = A.l[li];
   const int ci = a.c1 + a.c2;
   const size_t nxi = (size_t)a.npad * (ci / 8);
-  size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  size_t i = (size_t)(blockIdx.x - A.off[li]) * 256 + threadIdx.x;
   const s8v zero = {0, 0, 0, 0, 0, 0, 0, 0};
   if (i < nxi) {
     const int p = i % a.npad, c = 8 * (int)(i / a.npad);
@@ -271,17 +288,21 @@ template <> struct WgGroup<1> { typedef short T; };
 
 // NCO: output tiles per wave; G: points per load of the input (a divisor of nx)
 template <int NCO, int G>
-__global__ __launch_bounds__(64) void k_wgrad(WgArgs a) {
+__global__ __launch_bounds__(64) void k_wgrad(WgAll A) {
+  const int li = wg_layer(A, blockIdx.x);
+  const WgArgs &a = A.l[li];
   const int lane = threadIdx.x;
   const int row = lane & 15, kq = lane >> 4;
   const int ci = a.c1 + a.c2;
   const int nci = ci / 16, nct = a.co / 16 / NCO;
-  int t = blockIdx.x;
+  int t = blockIdx.x - A.off[li];
   const int cit = t % nci;
   t /= nci;
-  const int cot = NCO * (t % nct), g = t / nct;
+  const int cot = NCO * (t % nct);
+  t /= nct;
+  const int g = t % 9, chunk = t / 9;
   const int dz = g / 3 - 1, dyy = g % 3 - 1;
-  const int pbeg = blockIdx.y * kWgChunk, pend = min(pbeg + kWgChunk, a.npts);
+  const int pbeg = chunk * kWgChunk, pend = min(pbeg + kWgChunk, a.npts);
   f4v acc[3][NCO];
 #pragma unroll
   for (int d = 0; d < 3; ++d)
@@ -353,7 +374,7 @@ __global__ __launch_bounds__(64) void k_wgrad(WgArgs a) {
     if (pb + 64 * U < pend) load_group(pb + 64 * U, av[0], bv[0]);
     mfma_group(pb + 32 * U, av[1], bv[1]);
   }
-  float *part = a.part + (size_t)blockIdx.y * 27 * a.co * ci;
+  float *part = a.part + (size_t)chunk * 27 * a.co * ci;
 #pragma unroll
   for (int k = 0; k < NCO; ++k)
 #pragma unroll
@@ -363,12 +384,18 @@ __global__ __launch_bounds__(64) void k_wgrad(WgArgs a) {
         part[((size_t)(3 * g + d) * a.co + (cot + k) * 16 + 4 * kq + e) * ci + cit * 16 + row] = acc[d][k][e];
 }
 
-// grad[i] += sum_k part[k][i], k ascending, 8 loads in flight (the first nwb blocks), and the biases:
+// grad[i] += sum_k part[k][i], k ascending, 8 loads in flight (a layer's first nwb blocks), and the biases:
 // grad[nw + c] += sum_p dy[p][c], one block per channel, fixed-order tree
-__global__ __launch_bounds__(256) void k_wg_reduce(WgArgs a, int nk, size_t nw, unsigned nwb) {
+__global__ __launch_bounds__(256) void k_wg_reduce(WgAll A) {
   __shared__ float sh[256];
-  if (blockIdx.x < nwb) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  const int li = wg_layer(A, blockIdx.x);
+  const WgArgs &a = A.l[li];
+  const unsigned bx = blockIdx.x - A.off[li];
+  const int nk = (a.npts + kWgChunk - 1) / kWgChunk;
+  const size_t nw = (size_t)27 * a.co * (a.c1 + a.c2);
+  const unsigned nwb = (unsigned)((nw + 255) / 256);
+  if (bx < nwb) {
+    const size_t i = (size_t)bx * 256 + threadIdx.x;
     if (i >= nw) return;
     float s = 0.f;
     for (int k = 0; k < nk; k += 8) {
@@ -382,7 +409,7 @@ __global__ __launch_bounds__(256) void k_wg_reduce(WgArgs a, int nk, size_t nw, 
     a.grad[i] += s;
     return;
   }
-  const int c = blockIdx.x - nwb;
+  const int c = bx - nwb;
   const bf16_t *g = a.gt + (size_t)c * a.npad;
   float s = 0.f;
   for (int p0 = threadIdx.x; p0 < a.npts; p0 += 256 * 16) {
@@ -670,6 +697,7 @@ unsigned blocks(size_t n) { return (unsigned)((n + 255) / 256); }
 struct Layer {
   int co, c1, c2, up1, level;  // input [up(src1) (c1), src2 (c2)] at `level`
   size_t woff, boff;           // offsets in the flat parameter array
+  size_t xt_off, gt_off, part_off;  // its part of the weight gradients' work
   bf16_t *wt = nullptr, *wb = nullptr;
 };
 
@@ -689,7 +717,7 @@ struct salmon_unet {
   bf16_t *d_zero = nullptr;  // kConvZero zeros: the operands of k_conv outside the grid or past K
   // backward work
   float *d_out = nullptr, *d_dout = nullptr, *d_part = nullptr, *d_fx = nullptr, *d_fy = nullptr, *d_wpart = nullptr;
-  bf16_t *g_a = nullptr, *g_b = nullptr;
+  bf16_t *g[10] = {};        // pre-activation gradient of each layer
   bf16_t *d_xt = nullptr, *d_gt = nullptr;  // channel-major operands of the weight gradient
   size_t fx_n = 0;
   double *d_rpart = nullptr;  // residual partial maxima
@@ -794,46 +822,69 @@ int forward(salmon_unet *u, const float *in, float *out) {
   return 0;
 }
 
-template <int NCO>
-void launch_wgrad(hipStream_t st, const dim3 &grid, const WgArgs &a) {
-  if (a.nx % 8 == 0) hipLaunchKernelGGL((k_wgrad<NCO, 8>), grid, dim3(64), 0, st, a);
-  else if (a.nx % 4 == 0) hipLaunchKernelGGL((k_wgrad<NCO, 4>), grid, dim3(64), 0, st, a);
-  else if (a.nx % 2 == 0) hipLaunchKernelGGL((k_wgrad<NCO, 2>), grid, dim3(64), 0, st, a);
-  else hipLaunchKernelGGL((k_wgrad<NCO, 1>), grid, dim3(64), 0, st, a);
-}
-
 size_t wg_pad(size_t npts) { return (npts + 31) / 32 * 32; }
 
-// weight and bias gradient of conv layer l (act index i) from its pre-activation gradient g
-int layer_wgrad(salmon_unet *u, int i, const Layer &l, const bf16_t *g) {
-  const int ci = l.c1 + l.c2;
+// weight and bias gradient of conv layer li (act index i) from its pre-activation gradient
+WgArgs wg_args(salmon_unet *u, int li, int i) {
+  const Layer &l = u->L[li];
   WgArgs a;
-  a.dy = g; a.co = l.co;
+  a.dy = u->g[li]; a.co = l.co;
   a.src1 = layer_src1(u, i); a.src2 = layer_src2(u, i); a.c1 = l.c1; a.c2 = l.c2; a.up1 = l.up1;
-  a.xt = u->d_xt; a.gt = u->d_gt;
-  a.part = u->d_wpart;
+  a.xt = u->d_xt + l.xt_off; a.gt = u->d_gt + l.gt_off;
+  a.part = u->d_wpart + l.part_off;
   a.grad = u->d_g + l.woff;  // the layer's weights and biases lie side by side
   a.nx = u->n[l.level][0]; a.ny = u->n[l.level][1]; a.nz = u->n[l.level][2];
   a.npts = (int)u->np[l.level];
   a.npad = (int)wg_pad(a.npts);
-  hipLaunchKernelGGL(k_wg_pack, dim3(blocks((size_t)a.npad * (ci + l.co) / 8)), dim3(256), 0, u->stream, a);
+  return a;
+}
+
+void wg_add(WgAll &A, const WgArgs &a, size_t nblk) {
+  if (A.n == 0) A.off[0] = 0;
+  A.l[A.n] = a;
+  A.off[A.n + 1] = A.off[A.n] + (unsigned)nblk;
+  ++A.n;
+}
+
+// Weight and bias gradients of all layers once their pre-activation gradients stand: three launches (the
+// main one split by the two forms below), where one layer alone leaves most of the chip idle.
+int weight_grads(salmon_unet *u, const int *conv_act) {
+  WgAll P, R, W[2][4];
+  P.n = R.n = 0;
+  for (auto &w : W)
+    for (WgAll &x : w) x.n = 0;
+  for (int li = 9; li >= 0; --li) {
+    const WgArgs a = wg_args(u, li, conv_act[li]);
+    const int ci = a.c1 + a.c2;
+    const size_t nw = (size_t)27 * a.co * ci;
+    const int nchunk = (a.npts + kWgChunk - 1) / kWgChunk;
+    wg_add(P, a, blocks((size_t)a.npad * (ci + a.co) / 8));
+    wg_add(R, a, blocks(nw) + a.co);
+    // two output tiles per wave share the input's loads where that leaves a wave for every CU
+    const size_t tasks = (size_t)9 * (ci / 16) * (a.co / 16) * nchunk;
+    const int two = a.co % 32 == 0 && tasks / 2 >= 256;
+    const int g = a.nx % 8 == 0 ? 3 : a.nx % 4 == 0 ? 2 : a.nx % 2 == 0 ? 1 : 0;
+    wg_add(W[two][g], a, two ? tasks / 2 : tasks);
+  }
+  hipLaunchKernelGGL(k_wg_pack, dim3(P.off[P.n]), dim3(256), 0, u->stream, P);
   ULAUNCH("k_wg_pack");
-  const int nchunk = (a.npts + kWgChunk - 1) / kWgChunk;
-  // two output tiles per wave share the input's loads where that leaves a wave for every CU
-  const int tasks = 9 * (ci / 16) * (l.co / 16);
-  if (l.co % 32 == 0 && tasks * nchunk / 2 >= 256) launch_wgrad<2>(u->stream, dim3(tasks / 2, nchunk), a);
-  else launch_wgrad<1>(u->stream, dim3(tasks, nchunk), a);
-  ULAUNCH("k_wgrad");
-  const size_t nw = (size_t)27 * l.co * ci;
-  hipLaunchKernelGGL(k_wg_reduce, dim3(blocks(nw) + l.co), dim3(256), 0, u->stream, a, nchunk, nw, blocks(nw));
+#define WG_LAUNCH(two, g, G)                                                                                           \
+  if (W[two][g].n) {                                                                                                   \
+    hipLaunchKernelGGL((k_wgrad<two + 1, G>), dim3(W[two][g].off[W[two][g].n]), dim3(64), 0, u->stream, W[two][g]);     \
+    ULAUNCH("k_wgrad");                                                                                                \
+  }
+  WG_LAUNCH(0, 3, 8) WG_LAUNCH(0, 2, 4) WG_LAUNCH(0, 1, 2) WG_LAUNCH(0, 0, 1)
+  WG_LAUNCH(1, 3, 8) WG_LAUNCH(1, 2, 4) WG_LAUNCH(1, 1, 2) WG_LAUNCH(1, 0, 1)
+#undef WG_LAUNCH
+  hipLaunchKernelGGL(k_wg_reduce, dim3(R.off[R.n]), dim3(256), 0, u->stream, R);
   ULAUNCH("k_wg_reduce");
   return 0;
 }
 
-// FP32 data gradient of conv layer l's input into u->d_fx ([np][c1 + c2])
-int layer_dgrad(salmon_unet *u, const Layer &l, const bf16_t *g) {
+// FP32 data gradient of conv layer l's input into fx ([np][c1 + c2])
+int layer_dgrad(salmon_unet *u, const Layer &l, const bf16_t *g, float *fx) {
   const int ci = l.c1 + l.c2;
-  return launch_conv(u, g, l.co, 0, nullptr, 0, l.wb, nullptr, ci, 0, l.level, nullptr, u->d_fx);
+  return launch_conv(u, g, l.co, 0, nullptr, 0, l.wb, nullptr, ci, 0, l.level, nullptr, fx);
 }
 
 int backward(salmon_unet *u, const float *target, float *loss) {
@@ -847,18 +898,20 @@ int backward(salmon_unet *u, const float *target, float *loss) {
   }
   hipLaunchKernelGGL(k_head_grad, dim3(5), dim3(256), 0, u->stream, u->d_dout, u->act[D1B], n0, u->d_g + u->head_off);
   ULAUNCH("k_head_grad");
-  bf16_t *g = u->g_a, *gn = u->g_b;
   hipLaunchKernelGGL(k_head_back, dim3(blocks(n0 * 16)), dim3(256), 0, u->stream, u->d_dout, u->d_w + u->head_off,
-                     u->act[D1B], n0, g);
+                     u->act[D1B], n0, u->g[9]);
   ULAUNCH("k_head_back");
   // conv layers in reverse; layer index li <-> act index
   static const int conv_act[10] = {E1A, E1B, E2A, E2B, E3A, E3B, D2A, D2B, D1A, D1B};
   for (int li = 9; li >= 0; --li) {
     const Layer &l = u->L[li];
     const int i = conv_act[li];
-    if (int rc = layer_wgrad(u, i, l, g)) return rc;
     if (li == 0) break;
-    if (int rc = layer_dgrad(u, l, g)) return rc;
+    const bf16_t *g = u->g[li];
+    bf16_t *gn = u->g[li - 1];
+    // the gradients of D1A's and D2A's inputs are kept for their skip parts (fx is reused by the next layers)
+    float *fx = i == D1A ? u->d_fx + u->fx_n : i == D2A ? u->d_fx + u->fx_n + n0 * 48 : u->d_fx;
+    if (int rc = layer_dgrad(u, l, g, fx)) return rc;
     const int lv = l.level;
     const int ci = l.c1 + l.c2;
     switch (i) {
@@ -874,15 +927,12 @@ int backward(salmon_unet *u, const float *target, float *loss) {
         const int up = i == D1A ? D2B : E3B;
         const int C1 = l.c1;
         float *fy = u->d_fy;
-        hipLaunchKernelGGL(k_downsum, dim3(blocks(u->np[lv + 1] * C1)), dim3(256), 0, u->stream, u->d_fx, ci, 0, C1,
+        hipLaunchKernelGGL(k_downsum, dim3(blocks(u->np[lv + 1] * C1)), dim3(256), 0, u->stream, fx, ci, 0, C1,
                            fy, u->n[lv + 1][0], u->n[lv + 1][1], u->n[lv + 1][2]);
         ULAUNCH("k_downsum");
         hipLaunchKernelGGL(k_mask, dim3(blocks(u->np[lv + 1] * C1)), dim3(256), 0, u->stream, fy, C1, 0, C1,
                            u->act[up], u->np[lv + 1], gn);
         ULAUNCH("k_mask");
-        // keep the skip gradient: copy the FP32 tensor aside (fx is reused by the next layers)
-        float *keep = i == D1A ? u->d_fx + u->fx_n : u->d_fx + u->fx_n + n0 * 48;
-        UHIP(hipMemcpyAsync(keep, u->d_fx, sizeof(float) * u->np[lv] * ci, hipMemcpyDeviceToDevice, u->stream));
         break;
       }
       case E3A: case E2A: {
@@ -900,9 +950,8 @@ int backward(salmon_unet *u, const float *target, float *loss) {
       default:
         return ufail(SALMON_HIP_EINVAL, "internal: layer %d", i);
     }
-    std::swap(g, gn);
   }
-  return 0;
+  return weight_grads(u, conv_act);
 }
 
 int ucheck(salmon_unet_t u) { return u ? 0 : ufail(SALMON_HIP_EINVAL, "null predictor handle"); }
@@ -958,16 +1007,20 @@ int salmon_unet_create(int nx, int ny, int nz, unsigned long long seed, salmon_u
   size_t wp = 0, xt = 0, gt = 0;
   for (Layer &l : u->L) {
     const size_t ci = l.c1 + l.c2, np = u->np[l.level];
-    wp = std::max(wp, (np + kWgChunk - 1) / kWgChunk * 27 * l.co * ci);
-    xt = std::max(xt, 3 * ci * wg_pad(np));
-    gt = std::max(gt, l.co * wg_pad(np));
+    l.part_off = wp;
+    l.xt_off = xt;
+    l.gt_off = gt;
+    wp += (np + kWgChunk - 1) / kWgChunk * 27 * l.co * ci;
+    xt += 3 * ci * wg_pad(np);
+    gt += l.co * wg_pad(np);
   }
   if ((rc = ualloc(u, &u->d_out, n0)) || (rc = ualloc(u, &u->d_dout, n0)) || (rc = ualloc(u, &u->d_part, blocks(n0))) ||
       (rc = ualloc(u, &u->d_fx, u->fx_n + n0 * 48 + n1 * 96)) || (rc = ualloc(u, &u->d_fy, n1 * 64)) ||
       (rc = ualloc(u, &u->d_wpart, wp)) || (rc = ualloc(u, &u->d_xt, xt)) || (rc = ualloc(u, &u->d_gt, gt)) ||
-      (rc = ualloc(u, &u->g_a, n0 * 64)) || (rc = ualloc(u, &u->g_b, n0 * 64)) ||
       (rc = ualloc(u, &u->d_rpart, 1024)))
     return bail(rc);
+  for (int li = 0; li < 10; ++li)
+    if ((rc = ualloc(u, &u->g[li], u->np[u->L[li].level] * u->L[li].co))) return bail(rc);
   // He-normal weights, zero biases; head: small normal weights, zero bias
   std::vector<float> w(off, 0.f);
   std::mt19937_64 gen(seed);
