@@ -88,7 +88,8 @@ struct ConvArgs {
   int c1, c2, up1;
   const bf16_t *w;      // [27][co][c1 + c2]
   const float *bias;    // [co] or null
-  bf16_t *out_bf;       // [npts][co] (bias, optional relu), or
+  const bf16_t *mask;   // [npts][co]: results where it is not above 0 are 0 (the gradient of relu), or null
+  bf16_t *out_bf;       // [npts][co] (bias, optional relu, mask), or
   float *out_f;         // [npts][co] raw
   int co, relu;
   int nx, ny, nz, npts;
@@ -103,12 +104,15 @@ struct ConvArgs {
 // operands per K step and 14 to 81 steps): U steps' loads are issued together, the next group's while the
 // MFMAs of a group run, and the channel count is a constant so that a step's addresses cost no division.
 // With one step ahead and runtime divisions a 16 -> 16 layer took 12.7 us at 32^3, now 6.2.
+// blockIdx.y takes NT output tiles each: with SK one per block, as a coarse level's points alone leave most
+// CUs idle (64 -> 64 channels at 8^3 13.8 us with four tiles per wave, 6.5 us so).
 template <int NT, bool SK, int CI>
 __global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int p0 = (SK ? blockIdx.x : blockIdx.x * 4 + wave) * 16;
   if (p0 >= a.npts) return;
   const int row = lane & 15, kq = lane >> 4;
+  const int ct = blockIdx.y * NT * 16;  // first output channel of this block
   const int p = p0 + row;
   const bool pv = p < a.npts;
   const int pp = pv ? p : 0;
@@ -140,7 +144,7 @@ __global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
     av = *(const s8v *)((fv && pv) ? src : a.zero);
     const bf16_t *wt = fv ? a.w + (size_t)(tap * a.co) * ci + c : a.zero;
 #pragma unroll
-    for (int t = 0; t < NT; ++t) bv[t] = *(const s8v *)(wt + (t * 16 + row) * ci);
+    for (int t = 0; t < NT; ++t) bv[t] = *(const s8v *)(wt + (ct + t * 16 + row) * ci);
   };
   // this wave's K steps fs, fs + kst, ... in two sets of U operands (steps past the end multiply zeros
   // and are left out); the accumulation order is that of the steps
@@ -182,12 +186,13 @@ __global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int pr = p0 + 4 * kq + r;
-      const int ch = t * 16 + row;
+      const int ch = ct + t * 16 + row;
       if (pr >= a.npts) continue;
       float v = acc[t][r];
       if (a.out_bf) {
         if (a.bias) v += a.bias[ch];
         if (a.relu) v = fmaxf(v, 0.f);
+        if (a.mask && !(bf2f(a.mask[(size_t)pr * a.co + ch]) > 0.f)) v = 0.f;
         a.out_bf[(size_t)pr * a.co + ch] = f2bf(v);
       } else {
         a.out_f[(size_t)pr * a.co + ch] = v;
@@ -446,9 +451,9 @@ __global__ __launch_bounds__(256) void k_pool(const bf16_t *in, bf16_t *out, int
   out[i] = f2bf(s * 0.125f);
 }
 
-// out[q][c] = sum of the 8 children of q of gin[.][off + c] (gradient of nearest upsampling)
-__global__ __launch_bounds__(256) void k_downsum(const float *gin, int Cs, int off, int C, float *out, int hx, int hy,
-                                                 int hz) {
+// out[q][c] = bf16((sum of the 8 children of q of gin[.][c]) * (act[q][c] > 0)) (gradient of nearest upsampling)
+__global__ __launch_bounds__(256) void k_downsum(const float *gin, int Cs, int C, const bf16_t *act, bf16_t *out, int hx,
+                                                 int hy, int hz) {
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
   const size_t n = (size_t)hx * hy * hz * C;
   if (i >= n) return;
@@ -459,21 +464,9 @@ __global__ __launch_bounds__(256) void k_downsum(const float *gin, int Cs, int o
   float s = 0.f;
   for (int k = 0; k < 8; ++k) {
     const int xx = 2 * x + (k & 1), yy = 2 * y + ((k >> 1) & 1), zz = 2 * z + (k >> 2);
-    s += gin[((size_t)xx + (size_t)nx * ((size_t)yy + (size_t)ny * zz)) * Cs + off + c];
+    s += gin[((size_t)xx + (size_t)nx * ((size_t)yy + (size_t)ny * zz)) * Cs + c];
   }
-  out[i] = s;
-}
-
-// out[p][c] = bf16(gin[p][off + c] * (act[p][c] > 0)), act null = no mask
-__global__ __launch_bounds__(256) void k_mask(const float *gin, int Cs, int off, int C, const bf16_t *act, size_t npts,
-                                              bf16_t *out) {
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= npts * C) return;
-  const size_t p = i / C;
-  const int c = i % C;
-  float v = gin[p * Cs + off + c];
-  if (act && !(bf2f(act[i]) > 0.f)) v = 0.f;
-  out[i] = f2bf(v);
+  out[i] = f2bf(bf2f(act[i]) > 0.f ? s : 0.f);
 }
 
 // out[p][c] = bf16((gp[parent(p)][c] / 8 + gskip[p][off + c]) * (act[p][c] > 0))
@@ -593,16 +586,27 @@ __global__ __launch_bounds__(256) void k_adam(size_t n, float *w, float *g, floa
   g[i] = 0.f;
 }
 
-// wt[tap][co][ci] = bf16(w), wb[26 - tap][ci][co] = bf16(w) (data-gradient weights)
-__global__ __launch_bounds__(256) void k_pack_w(const float *w, int co, int ci, bf16_t *wt, bf16_t *wb) {
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+// wt[tap][co][ci] = bf16(w), wb[26 - tap][ci][co] = bf16(w) (data-gradient weights), all layers: layer i owns
+// the blocks [off[i], off[i + 1])
+struct PackArgs {
+  const float *w[kWgLayers];
+  bf16_t *wt[kWgLayers], *wb[kWgLayers];
+  int co[kWgLayers], ci[kWgLayers];
+  unsigned off[kWgLayers + 1];
+};
+
+__global__ __launch_bounds__(256) void k_pack_w(PackArgs A) {
+  int li = 0;
+  while (li + 1 < kWgLayers && blockIdx.x >= A.off[li + 1]) ++li;
+  const int co = A.co[li], ci = A.ci[li];
+  const size_t i = (size_t)(blockIdx.x - A.off[li]) * 256 + threadIdx.x;
   if (i >= (size_t)27 * co * ci) return;
   const int c = i % ci;
   const int o = (i / ci) % co;
   const int tap = i / ((size_t)co * ci);
-  const bf16_t h = f2bf(w[i]);
-  wt[i] = h;
-  wb[((size_t)(26 - tap) * ci + c) * co + o] = h;
+  const bf16_t h = f2bf(A.w[li][i]);
+  A.wt[li][i] = h;
+  A.wb[li][((size_t)(26 - tap) * ci + c) * co + o] = h;
 }
 
 // ---------------------------------------------------------------------------
@@ -716,7 +720,7 @@ struct salmon_unet {
   bf16_t *x0 = nullptr, *act[12] = {};
   bf16_t *d_zero = nullptr;  // kConvZero zeros: the operands of k_conv outside the grid or past K
   // backward work
-  float *d_out = nullptr, *d_dout = nullptr, *d_part = nullptr, *d_fx = nullptr, *d_fy = nullptr, *d_wpart = nullptr;
+  float *d_out = nullptr, *d_dout = nullptr, *d_part = nullptr, *d_fx = nullptr, *d_wpart = nullptr;
   bf16_t *g[10] = {};        // pre-activation gradient of each layer
   bf16_t *d_xt = nullptr, *d_gt = nullptr;  // channel-major operands of the weight gradient
   size_t fx_n = 0;
@@ -738,22 +742,24 @@ int ualloc(salmon_unet *u, T **p, size_t n) {
 }
 
 int launch_conv(salmon_unet *u, const bf16_t *s1, int c1, int up1, const bf16_t *s2, int c2, const bf16_t *w,
-                const float *bias, int co, int relu, int level, bf16_t *out_bf, float *out_f) {
+                const float *bias, int co, int relu, int level, bf16_t *out_bf, float *out_f,
+                const bf16_t *mask = nullptr) {
   ConvArgs a;
   a.src1 = s1; a.src2 = s2; a.c1 = c1; a.c2 = c2; a.up1 = up1;
-  a.w = w; a.bias = bias; a.out_bf = out_bf; a.out_f = out_f; a.co = co; a.relu = relu;
+  a.w = w; a.bias = bias; a.mask = mask; a.out_bf = out_bf; a.out_f = out_f; a.co = co; a.relu = relu;
   a.nx = u->n[level][0]; a.ny = u->n[level][1]; a.nz = u->n[level][2];
   a.npts = (int)u->np[level];
   a.zero = u->d_zero;
   if ((size_t)co * (c1 + c2) + 8 > kConvZero)
     return ufail(SALMON_HIP_EUNSUPPORTED, "conv %d -> %d channels above the zero operand", c1 + c2, co);
-  // fewer 64-point blocks than CUs: split K over the four waves of 16-point blocks
+  // fewer 64-point blocks than CUs: split K over the four waves of 16-point blocks, one tile of output
+  // channels each
   const bool sk = (a.npts + 63) / 64 < 256;
   const unsigned nb = (unsigned)(sk ? (a.npts + 15) / 16 : (a.npts + 63) / 64);
-#define CONV_LAUNCH(NTv, CIv)                                                                   \
-  case 16 * NTv + CIv:                                                                          \
-    if (sk) hipLaunchKernelGGL((k_conv<NTv, true, CIv>), dim3(nb), dim3(256), 0, u->stream, a); \
-    else hipLaunchKernelGGL((k_conv<NTv, false, CIv>), dim3(nb), dim3(256), 0, u->stream, a);   \
+#define CONV_LAUNCH(NTv, CIv)                                                                      \
+  case 16 * NTv + CIv:                                                                             \
+    if (sk) hipLaunchKernelGGL((k_conv<1, true, CIv>), dim3(nb, NTv), dim3(256), 0, u->stream, a); \
+    else hipLaunchKernelGGL((k_conv<NTv, false, CIv>), dim3(nb), dim3(256), 0, u->stream, a);      \
     break
   // output and input tiles of the layers, forward and (transposed) backward
   switch (c1 % 16 == 0 && c2 % 16 == 0 && co % 16 == 0 ? co + (c1 + c2) / 16 : 0) {
@@ -786,12 +792,19 @@ const bf16_t *layer_src2(salmon_unet *u, int i) {
 }
 
 int pack_weights(salmon_unet *u) {
-  for (Layer &l : u->L) {
-    const int ci = l.c1 + l.c2;
-    hipLaunchKernelGGL(k_pack_w, dim3(blocks((size_t)27 * l.co * ci)), dim3(256), 0, u->stream, u->d_w + l.woff, l.co,
-                       ci, l.wt, l.wb);
-    ULAUNCH("k_pack_w");
+  PackArgs A;
+  A.off[0] = 0;
+  for (int li = 0; li < kWgLayers; ++li) {
+    const Layer &l = u->L[li];
+    A.w[li] = u->d_w + l.woff;
+    A.wt[li] = l.wt;
+    A.wb[li] = l.wb;
+    A.co[li] = l.co;
+    A.ci[li] = l.c1 + l.c2;
+    A.off[li + 1] = A.off[li] + blocks((size_t)27 * l.co * (l.c1 + l.c2));
   }
+  hipLaunchKernelGGL(k_pack_w, dim3(A.off[kWgLayers]), dim3(256), 0, u->stream, A);
+  ULAUNCH("k_pack_w");
   u->packed = true;
   return 0;
 }
@@ -881,10 +894,11 @@ int weight_grads(salmon_unet *u, const int *conv_act) {
   return 0;
 }
 
-// FP32 data gradient of conv layer l's input into fx ([np][c1 + c2])
-int layer_dgrad(salmon_unet *u, const Layer &l, const bf16_t *g, float *fx) {
+// data gradient of conv layer l's input ([np][c1 + c2]): FP32 into fx, or masked by the activation into gn
+int layer_dgrad(salmon_unet *u, const Layer &l, const bf16_t *g, float *fx, bf16_t *gn = nullptr,
+                const bf16_t *mask = nullptr) {
   const int ci = l.c1 + l.c2;
-  return launch_conv(u, g, l.co, 0, nullptr, 0, l.wb, nullptr, ci, 0, l.level, nullptr, fx);
+  return launch_conv(u, g, l.co, 0, nullptr, 0, l.wb, nullptr, ci, 0, l.level, gn, fx, mask);
 }
 
 int backward(salmon_unet *u, const float *target, float *loss) {
@@ -911,28 +925,20 @@ int backward(salmon_unet *u, const float *target, float *loss) {
     bf16_t *gn = u->g[li - 1];
     // the gradients of D1A's and D2A's inputs are kept for their skip parts (fx is reused by the next layers)
     float *fx = i == D1A ? u->d_fx + u->fx_n : i == D2A ? u->d_fx + u->fx_n + n0 * 48 : u->d_fx;
-    if (int rc = layer_dgrad(u, l, g, fx)) return rc;
+    const bool chain = i == D1B || i == D2B || i == E3B || i == E2B || i == E1B;  // input is the previous activation
+    if (int rc = chain ? layer_dgrad(u, l, g, nullptr, gn, u->act[i - 1]) : layer_dgrad(u, l, g, fx)) return rc;
     const int lv = l.level;
     const int ci = l.c1 + l.c2;
     switch (i) {
-      case D1B: case D2B: case E3B: case E2B: case E1B: {
-        // input is the previous activation: mask by it
-        hipLaunchKernelGGL(k_mask, dim3(blocks(u->np[lv] * ci)), dim3(256), 0, u->stream, u->d_fx, ci, 0, ci,
-                           u->act[i - 1], u->np[lv], gn);
-        ULAUNCH("k_mask");
+      case D1B: case D2B: case E3B: case E2B: case E1B:
         break;
-      }
       case D1A: case D2A: {
         // input [up(d2b | e3b), e1b | e2b]: the up part goes to the coarse activation, the skip part is kept
         const int up = i == D1A ? D2B : E3B;
         const int C1 = l.c1;
-        float *fy = u->d_fy;
-        hipLaunchKernelGGL(k_downsum, dim3(blocks(u->np[lv + 1] * C1)), dim3(256), 0, u->stream, fx, ci, 0, C1,
-                           fy, u->n[lv + 1][0], u->n[lv + 1][1], u->n[lv + 1][2]);
+        hipLaunchKernelGGL(k_downsum, dim3(blocks(u->np[lv + 1] * C1)), dim3(256), 0, u->stream, fx, ci, C1,
+                           u->act[up], gn, u->n[lv + 1][0], u->n[lv + 1][1], u->n[lv + 1][2]);
         ULAUNCH("k_downsum");
-        hipLaunchKernelGGL(k_mask, dim3(blocks(u->np[lv + 1] * C1)), dim3(256), 0, u->stream, fy, C1, 0, C1,
-                           u->act[up], u->np[lv + 1], gn);
-        ULAUNCH("k_mask");
         break;
       }
       case E3A: case E2A: {
@@ -1015,7 +1021,7 @@ int salmon_unet_create(int nx, int ny, int nz, unsigned long long seed, salmon_u
     gt += l.co * wg_pad(np);
   }
   if ((rc = ualloc(u, &u->d_out, n0)) || (rc = ualloc(u, &u->d_dout, n0)) || (rc = ualloc(u, &u->d_part, blocks(n0))) ||
-      (rc = ualloc(u, &u->d_fx, u->fx_n + n0 * 48 + n1 * 96)) || (rc = ualloc(u, &u->d_fy, n1 * 64)) ||
+      (rc = ualloc(u, &u->d_fx, u->fx_n + n0 * 48 + n1 * 96)) ||
       (rc = ualloc(u, &u->d_wpart, wp)) || (rc = ualloc(u, &u->d_xt, xt)) || (rc = ualloc(u, &u->d_gt, gt)) ||
       (rc = ualloc(u, &u->d_rpart, 1024)))
     return bail(rc);
