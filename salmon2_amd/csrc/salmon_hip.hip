@@ -102,7 +102,6 @@ struct KvecArgs {
   const double *rxyz;    // (3, nps, natom)
   const double *uv;      // (nps, nlma)
   const int *mps;        // (natom)
-  const int *lma_atom;   // (nlma) 0-based atom of each projector
   const int2 *atom_lma;  // (natom): first ilma, count
   const int *entof;      // (nps, natom): CSR entry of each sphere point
   double2 *zekr;         // (nps, nlma, nk)
@@ -115,7 +114,7 @@ struct KvecArgs {
   const double *actab;
   const int *itt;
   int tmax;              // last row of actab (nt + 1); the step counter is clamped to 1..tmax
-  int nlma, nps, nk, nent, cmax;
+  int natom, nlma, nps, nk, nent, cmax;
 };
 
 // the midpoint field of the current step from the device table, else the by-value field
@@ -132,13 +131,14 @@ __device__ __forceinline__ void kvec_field(const KvecArgs &a, double &ax, double
   }
 }
 
-__device__ __forceinline__ void update_kvector_body(const KvecArgs &a, int ilma, int ik) {
+// One block per atom and k: a point's phase serves all projectors of its atom.
+__device__ __forceinline__ void update_kvector_body(const KvecArgs &a, int ia, int ik) {
   double ax, ay, az;
   kvec_field(a, ax, ay, az);
   const double kx = a.veck[3 * ik + 0] + ax;
   const double ky = a.veck[3 * ik + 1] + ay;
   const double kz = a.veck[3 * ik + 2] + az;
-  if (ilma == 0 && threadIdx.x == 0) {
+  if (ia == 0 && threadIdx.x == 0) {
     double *kp = a.kpar + 16 * ik;
     double ss = kx * kx;
     ss = ss + ky * ky;
@@ -153,19 +153,28 @@ __device__ __forceinline__ void update_kvector_body(const KvecArgs &a, int ilma,
     kp[14] = ky;
     kp[15] = kz;
   }
-  if (ilma >= a.nlma) return;
-  const int ia = a.lma_atom[ilma];
+  if (ia >= a.natom) return;
+  const int2 al = a.atom_lma[ia];
   const int m = a.mps[ia];
   for (int j = threadIdx.x; j < m; j += blockDim.x) {
+    const double *uv = a.uv + (size_t)j + (size_t)a.nps * al.x;
+    double u[4];  // the first projectors' values beside the phase's latency
+#pragma unroll
+    for (int l = 0; l < 4; ++l) u[l] = l < al.y ? uv[(size_t)a.nps * l] : 0.0;
+    const int e = a.entof[(size_t)j + (size_t)a.nps * ia];
     const double *r = a.rxyz + 3 * ((size_t)j + (size_t)a.nps * ia);
     const double th = kx * r[0] + ky * r[1] + kz * r[2];
     double s, c;
     sincos(th, &s, &c);
-    const double u = a.uv[(size_t)j + (size_t)a.nps * ilma];
-    const double2 z = make_double2(c * u, -s * u);
-    a.zekr[(size_t)j + (size_t)a.nps * ((size_t)ilma + (size_t)a.nlma * ik)] = z;
-    const int e = a.entof[(size_t)j + (size_t)a.nps * ia];
-    a.zent[(size_t)(ilma - a.atom_lma[ia].x) + (size_t)a.cmax * ((size_t)e + (size_t)a.nent * ik)] = z;
+    double2 *ze = a.zent + (size_t)a.cmax * ((size_t)e + (size_t)a.nent * ik);
+    double2 *zk = a.zekr + (size_t)j + (size_t)a.nps * ((size_t)al.x + (size_t)a.nlma * ik);
+#pragma unroll
+    for (int l = 0; l < 4; ++l)
+      if (l < al.y) zk[(size_t)a.nps * l] = ze[l] = make_double2(c * u[l], -s * u[l]);
+    for (int l = 4; l < al.y; ++l) {
+      const double ul = uv[(size_t)a.nps * l];
+      zk[(size_t)a.nps * l] = ze[l] = make_double2(c * ul, -s * ul);
+    }
   }
 }
 
@@ -2549,7 +2558,7 @@ struct salmon_hip_ctx {
   // nonlocal
   int natom = 0, nps = 0, nlma = 0, nent = 0;
   int cmax = 0;
-  int *d_mps = nullptr, *d_jidx = nullptr, *d_lma_atom = nullptr, *d_pt_off = nullptr;
+  int *d_mps = nullptr, *d_jidx = nullptr, *d_pt_off = nullptr;
   int *d_pt_lma = nullptr, *d_entof = nullptr;
   int4 *d_tp_info = nullptr;  // per touched point: orbital-block offset, first entry, entry count, its pt_lma
   int ntp = 0;
@@ -2718,7 +2727,7 @@ int salmon_hip_destroy(salmon_hip_t c) {
   if (c->own) (void)hipStreamSynchronize(c->own);
   if (c->stream && c->stream != c->own) (void)hipStreamSynchronize(c->stream);
   dfree(c->d_veck); dfree(c->d_rocc); dfree(c->d_wtk); dfree(c->d_V); dfree(c->d_kpar); dfree(c->d_kpar_n);
-  dfree(c->d_mps); dfree(c->d_jidx); dfree(c->d_lma_atom); dfree(c->d_pt_off);
+  dfree(c->d_mps); dfree(c->d_jidx); dfree(c->d_pt_off);
   dfree(c->d_atom_lma); dfree(c->d_pt_lma); dfree(c->d_entof); dfree(c->d_rxyz); dfree(c->d_uv);
   dfree(c->d_rinv); dfree(c->d_zekr); dfree(c->d_zent); dfree(c->d_c); dfree(c->d_curnl);
   dfree(c->d_zekr_n); dfree(c->d_zent_n);
@@ -2754,7 +2763,7 @@ int salmon_hip_set_nonlocal(salmon_hip_t c, int natom, int nps, const int *mps, 
                             const double *uv) {
   if (int rc = check(c)) return rc;
   HIPCHK(hipStreamSynchronize(c->stream));
-  dfree(c->d_mps); dfree(c->d_jidx); dfree(c->d_lma_atom); dfree(c->d_pt_off);
+  dfree(c->d_mps); dfree(c->d_jidx); dfree(c->d_pt_off);
   dfree(c->d_atom_lma); dfree(c->d_pt_lma); dfree(c->d_entof); dfree(c->d_rxyz); dfree(c->d_uv);
   dfree(c->d_rinv); dfree(c->d_zekr); dfree(c->d_zent); dfree(c->d_c); dfree(c->d_curnl);
   dfree(c->d_zekr_n); dfree(c->d_zent_n);
@@ -2769,7 +2778,6 @@ int salmon_hip_set_nonlocal(salmon_hip_t c, int natom, int nps, const int *mps, 
     return fail(SALMON_HIP_EINVAL, "invalid projector tables");
   // validate: sphere sizes and grid indices, projectors contiguous per atom
   std::vector<int2> atom_lma(natom, make_int2(0, 0));
-  std::vector<int> lma_atom(nlma);
   for (int l = 0; l < nlma; ++l) {
     const int ia = ia_tbl[l] - 1;
     if (ia < 0 || ia >= natom) return fail(SALMON_HIP_EINVAL, "ia_tbl(%d)=%d out of range", l + 1, ia + 1);
@@ -2778,7 +2786,6 @@ int salmon_hip_set_nonlocal(salmon_hip_t c, int natom, int nps, const int *mps, 
     else if (atom_lma[ia].x + atom_lma[ia].y != l)
       return fail(SALMON_HIP_EUNSUPPORTED, "projectors of atom %d not contiguous", ia + 1);
     atom_lma[ia].y += 1;
-    lma_atom[l] = ia;
   }
   for (int ia = 0; ia < natom; ++ia)
     if (atom_lma[ia].y > kMaxLmaPerAtom)
@@ -2852,7 +2859,7 @@ int salmon_hip_set_nonlocal(salmon_hip_t c, int natom, int nps, const int *mps, 
   if ((rc = dalloc(&c->d_jexcl, jexcl.size())) || (rc = dalloc(&c->d_c2, (size_t)nlma * c->norb))) return rc;
   HIPCHK(hipMemcpy(c->d_jexcl, jexcl.data(), sizeof(int) * jexcl.size(), hipMemcpyHostToDevice));
   if ((rc = dalloc(&c->d_mps, natom)) || (rc = dalloc(&c->d_jidx, (size_t)natom * nps)) ||
-      (rc = dalloc(&c->d_lma_atom, nlma)) || (rc = dalloc(&c->d_pt_off, c->ngrid + 1)) ||
+      (rc = dalloc(&c->d_pt_off, c->ngrid + 1)) ||
       (rc = dalloc(&c->d_atom_lma, natom)) || (rc = dalloc(&c->d_pt_lma, pt_lma.size())) ||
       (rc = dalloc(&c->d_entof, entof.size())) ||
       (rc = dalloc(&c->d_rxyz, 3 * (size_t)nps * natom)) || (rc = dalloc(&c->d_uv, (size_t)nps * nlma)) ||
@@ -2862,7 +2869,6 @@ int salmon_hip_set_nonlocal(salmon_hip_t c, int natom, int nps, const int *mps, 
     return rc;
   HIPCHK(hipMemcpy(c->d_mps, mps, sizeof(int) * natom, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c->d_jidx, jidx.data(), sizeof(int) * jidx.size(), hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(c->d_lma_atom, lma_atom.data(), sizeof(int) * nlma, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c->d_pt_off, cnt.data(), sizeof(int) * cnt.size(), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c->d_atom_lma, atom_lma.data(), sizeof(int2) * natom, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c->d_pt_lma, pt_lma.data(), sizeof(int) * pt_lma.size(), hipMemcpyHostToDevice));
@@ -2947,7 +2953,7 @@ static KvecArgs kvec_args(salmon_hip_t c, const double *vec_Ac, const double *ac
   a.rxyz = c->d_rxyz;
   a.uv = c->d_uv;
   a.mps = c->d_mps;
-  a.lma_atom = c->d_lma_atom;
+  a.natom = c->nlma > 0 ? c->natom : 0;
   a.atom_lma = c->d_atom_lma;
   a.entof = c->d_entof;
   a.zekr = c->d_zekr;
@@ -2984,7 +2990,7 @@ static int update_kvector_impl(salmon_hip_t c, const double *vec_Ac, const doubl
   c->staged = false;
   c->pre_state = 0;
   const KvecArgs a = kvec_args(c, vec_Ac, actab, itt, tmax);
-  dim3 grid(std::max(1, c->nlma), c->nk);
+  dim3 grid(std::max(1, a.natom), c->nk);
   hipLaunchKernelGGL(k_update_kvector, grid, dim3(kBlock), 0, c->stream, a);
   LAUNCHCHK("k_update_kvector");
   c->have_k = true;
@@ -4040,7 +4046,7 @@ int salmon_hip_current_next(salmon_hip_t c, const double *vec_Ac, const void *ps
   ka.zekr = c->d_zekr_n;
   ka.zent = c->d_zent_n;
   ka.kpar = c->d_kpar_n;
-  hipLaunchKernelGGL(k_update_kvector, dim3(std::max(1, c->nlma), c->nk), dim3(kBlock), 0, c->stream, ka);
+  hipLaunchKernelGGL(k_update_kvector, dim3(std::max(1, ka.natom), c->nk), dim3(kBlock), 0, c->stream, ka);
   LAUNCHCHK("k_update_kvector");
   c->staged = true;
   memcpy(c->staged_A, vec_Ac_next, sizeof(c->staged_A));
@@ -4340,7 +4346,7 @@ __device__ __forceinline__ int pack_find(const int *off, int nsys, int b) {
 __global__ __launch_bounds__(kBlock) void kp_update_kvector(const KvecArgs *args, const int *off, int nsys) {
   const int s = pack_find(off, nsys, blockIdx.x);
   const KvecArgs a = args[s];
-  const int lb = (int)blockIdx.x - off[s], gx = max(1, a.nlma);
+  const int lb = (int)blockIdx.x - off[s], gx = max(1, a.natom);
   update_kvector_body(a, lb % gx, lb / gx);
 }
 
@@ -4699,7 +4705,7 @@ int batch_packed_tables(salmon_hip_batch *b) {
     std::vector<KvecArgs> r(ns);
     for (int i = 0; i < ns; ++i) {
       r[i] = kvec_args(b->h[i], nullptr, b->sys[i].actab, b->d_itt, b->sys[i].nt + 1);
-      cnt[i] = std::max(1, b->h[i]->nlma) * b->h[i]->nk;
+      cnt[i] = std::max(1, r[i].natom) * b->h[i]->nk;
     }
     if (int rc = pack_make(b, b->p_kvec, r, cnt, false)) return rc;
   }
