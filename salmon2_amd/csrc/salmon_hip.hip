@@ -246,10 +246,12 @@ __device__ __forceinline__ int xcd_order(int b, int nblk) {
 // Waves of a block on parts of the sphere (ProjStage's S): 4 where the operand staging is small, 1 where
 // four private stagings of it would cost more than they spread (d projectors under five weights,
 // 512 orbitals at 96 x 14 x 12: 79 us split, 57 us not; s+p projectors, 1024 orbitals at 32^3: 187 us split
-// and 202 us not for the fused pass, 128 orbitals there 14 us and 21 us for the projection).  It depends on
-// nothing else and the chunks of S = 4 are of one length: every form sums a projection in one order.
-constexpr int proj_split(int lm) { return lm <= 4 ? 4 : 1; }
-constexpr int proj_orb(int lm) { return proj_split(lm) == 4 ? 16 : kProjOrb; }
+// and 202 us not for the fused pass, 128 orbitals there 14 us and 21 us for the projection).  Handles of
+// the mixed precision keep the points in one sequence (fused pass of 216 atoms, 1728 orbitals 985 us, 953 us
+// split): what is rounded to FP32 after it must not depend on how the sum is grouped.  One handle's
+// forms all sum a projection in one order (the chunks of S = 4 are of one length).
+constexpr int proj_split(int lm, bool mixed) { return lm <= 4 && !mixed ? 4 : 1; }
+constexpr int proj_orb(int split) { return split == 4 ? 16 : kProjOrb; }
 
 // Staging of the contraction.  S = 1: a block takes 64 orbitals, 16 per wave, and the waves share the
 // projectors of a chunk of JC sphere points; S = 4: a block takes 16 orbitals and its waves every
@@ -258,12 +260,11 @@ constexpr int proj_orb(int lm) { return proj_split(lm) == 4 ? 16 : kProjOrb; }
 // zero, so that a lane's value for an MFMA is one 8-byte read and a sign; the orbitals as 16 per
 // wave and point.  Both are XOR-swizzled: writes (lanes on points) and reads (lanes on projectors or
 // orbitals) both spread over the banks.
-template <int NW, int LMX>
+template <int NW, int LMX, int S>
 struct ProjStage {
-  static constexpr int S = proj_split(LMX);
   static constexpr int JC = NW == 1 && S == 1 ? kProjJC : kProjJC / 2;
   static constexpr int MT = (NW * LMX + 7) / 8;
-  static constexpr int OB = proj_orb(LMX);       // orbitals per block
+  static constexpr int OB = proj_orb(S);           // orbitals per block
   static constexpr int kPer = JC / 4;                 // orbital values per lane and chunk
   static constexpr int kT = S == 4 ? 64 : kBlock;     // threads that stage one chunk's projectors
   static constexpr int kZPer = (JC * LMX + kT - 1) / kT;
@@ -288,9 +289,9 @@ __device__ __forceinline__ void stage_sync() {
 }
 
 // acc += A B over one staged chunk
-template <int NW, int LMX>
+template <int NW, int LMX, int S>
 __device__ __forceinline__ void stage_mfma(const double2 *sp, const double2 *z, int lane, int ntile, d4 *acc) {
-  using P = ProjStage<NW, LMX>;
+  using P = ProjStage<NW, LMX, S>;
   const int h = (lane >> 4) >> 1, comp = (lane >> 4) & 1;  // K row: point 2 ks + h, re/im of psi
   const int oc = lane & 15;                                // orbital column (B) / output row (A)
   const int part = (oc >> 2) & 1, lw0 = (oc >> 3) * 4 + (oc & 3);
@@ -330,11 +331,11 @@ __device__ __forceinline__ void stage_reduce(d4 *red, int wave, int lane, d4 *ac
 // read.  With the A values formed per wave from unswizzled tables (45 vector instructions an MFMA) NW = 5 took
 // 264 us for 64 atoms, 32^3 and 1024 orbitals, 131 us so (0.6 GB of lines, 4.6 TB/s), and 1183 and 692 us for
 // 216 atoms, 48^3 and 1728 orbitals (5.1 TB/s); NW = 1 for 64 atoms and 128 orbitals 37 and 14 us.
-template <int NW, typename TP, int LMX>
+template <int NW, typename TP, int LMX, int S>
 __device__ __forceinline__ void proj_body(const ProjArgs &a, int bid) {
   static_assert(LMX <= kMaxLmaPerAtom, "LMX bounds the projectors of one atom");
-  using P = ProjStage<NW, LMX>;
-  constexpr int S = P::S, JC = P::JC, MT = P::MT;
+  using P = ProjStage<NW, LMX, S>;
+  constexpr int JC = P::JC, MT = P::MT;
   constexpr size_t kRed = S == 4 ? sizeof(d4) * 3 * MT * 64 : 0;
   __shared__ __attribute__((aligned(32))) char lds[sizeof(P) > kRed ? sizeof(P) : kRed];
   P &st = *(P *)lds;
@@ -418,7 +419,7 @@ __device__ __forceinline__ void proj_body(const ProjArgs &a, int bid) {
     }
     stage_sync<S>();
     if (j0 + kStep < m) load_chunk(j0 + kStep);
-    stage_mfma<NW, LMX>(sp, z, lane, ntile, acc);
+    stage_mfma<NW, LMX, S>(sp, z, lane, ntile, acc);
     stage_sync<S>();
   }
   if constexpr (S == 4) {
@@ -454,10 +455,10 @@ __device__ __forceinline__ void proj_body(const ProjArgs &a, int bid) {
 }
 
 // up to 4 projectors per atom the registers leave four waves per SIMD
-template <int NW, typename TP, int LMX>
+template <int NW, typename TP, int LMX, int S>
 __global__ __launch_bounds__(kBlock, LMX == 4 ? 4 : 2) void k_proj(ProjArgs a) {
   if (a.skip && *a.skip) return;  // a device-side gate switched this launch off
-  proj_body<NW, TP, LMX>(a, xcd_order(blockIdx.x, gridDim.x));
+  proj_body<NW, TP, LMX, S>(a, xcd_order(blockIdx.x, gridDim.x));
 }
 
 // ---------------------------------------------------------------------------
@@ -484,12 +485,12 @@ struct ProjScatArgs {
   int cmax;                // projectors per atom, at most (the row count of the staged c)
 };
 
-template <typename TP, int LM>
+template <typename TP, int LM, int S>
 __device__ __forceinline__ void proj_scatter_body(const ProjScatArgs &A, int bid) {
   static_assert(LM <= kMaxLmaPerAtom, "LM bounds the projectors of one atom");
   const ProjArgs &a = A.p;
-  using P = ProjStage<1, LM>;
-  constexpr int S = P::S, JC = P::JC, MT = P::MT;
+  using P = ProjStage<1, LM, S>;
+  constexpr int JC = P::JC, MT = P::MT;
   constexpr size_t kRed = S == 4 ? sizeof(d4) * 3 * MT * 64 : 0;
   __shared__ __attribute__((aligned(32))) char lds[sizeof(P) > kRed ? sizeof(P) : kRed];
   P &st = *(P *)lds;
@@ -592,7 +593,7 @@ __device__ __forceinline__ void proj_scatter_body(const ProjScatArgs &A, int bid
     }
     stage_sync<S>();
     if (j0 + kStep < m) load_chunk(j0 + kStep);
-    stage_mfma<1, LM>(sp, z, lane, ntile, acc);
+    stage_mfma<1, LM, S>(sp, z, lane, ntile, acc);
     stage_sync<S>();
   }
   if constexpr (S == 4) {
@@ -617,10 +618,10 @@ __device__ __forceinline__ void proj_scatter_body(const ProjScatArgs &A, int bid
   }
 }
 
-template <typename TP, int LM>
+template <typename TP, int LM, int S>
 __global__ __launch_bounds__(kBlock, LM == 4 ? 4 : 2) void k_proj_scatter(ProjScatArgs A) {
   if (A.p.skip && *A.p.skip) return;  // a device-side gate switched this launch off
-  proj_scatter_body<TP, LM>(A, xcd_order(blockIdx.x, gridDim.x));
+  proj_scatter_body<TP, LM, S>(A, xcd_order(blockIdx.x, gridDim.x));
 }
 
 constexpr int kMaxComb = 5;   // Taylor order up to 6
@@ -3028,7 +3029,7 @@ int salmon_hip_set_vec_ac(salmon_hip_t c, const double *vec_Ac) {
 // The projector count that the projection kernels of atoms with up to cmax projectors are built for.
 static int proj_lm(int cmax) { return cmax <= 4 ? 4 : cmax <= 9 ? 9 : 16; }
 
-static ProjArgs proj_args(salmon_hip_t c, const void *psi, double2 *out, int lm) {
+static ProjArgs proj_args(salmon_hip_t c, const void *psi, double2 *out, int split) {
   ProjArgs a;
   a.psi = psi;
   a.zekr = c->d_zekr;
@@ -3044,7 +3045,7 @@ static ProjArgs proj_args(salmon_hip_t c, const void *psi, double2 *out, int lm)
   a.natom = c->natom;
   a.nps = c->nps;
   a.nlma = c->nlma;
-  a.ngrp = (c->nb + proj_orb(lm) - 1) / proj_orb(lm);
+  a.ngrp = (c->nb + proj_orb(split) - 1) / proj_orb(split);
   a.skip = c->d_skip;
   a.zekr2 = nullptr;
   a.out2 = nullptr;
@@ -3060,7 +3061,8 @@ static int launch_proj(salmon_hip_t c, const void *psi, int nw, bool f32 = false
     if (pre) return 0;
   }
   const int lmx = proj_lm(c->cmax);
-  ProjArgs a = proj_args(c, psi, nw == 1 ? c->d_c : c->d_curnl, lmx);
+  const int split = proj_split(lmx, c->prec != SALMON_HIP_PREC_FP64);
+  ProjArgs a = proj_args(c, psi, nw == 1 ? c->d_c : c->d_curnl, split);
   if (nw == 5) {
     a.zekr2 = c->d_zekr_n;
     a.out2 = c->d_c;
@@ -3076,17 +3078,25 @@ static int launch_proj(salmon_hip_t c, const void *psi, int nw, bool f32 = false
     HIPCHK(hipStreamWaitEvent(c->side, c->ev_fork, 0));
     st = c->side;
   }
-#define PROJ_LAUNCH(NWv, TPv)                                                                             \
-  do {                                                                                                   \
-    if (lmx == 4) hipExtLaunchKernelGGL((k_proj<NWv, TPv, 4>), grid, dim3(kBlock), 0, st, e0, e1, 0, a);   \
-    else if (lmx == 9) hipExtLaunchKernelGGL((k_proj<NWv, TPv, 9>), grid, dim3(kBlock), 0, st, e0, e1, 0, a); \
-    else hipExtLaunchKernelGGL((k_proj<NWv, TPv, 16>), grid, dim3(kBlock), 0, st, e0, e1, 0, a);           \
+#define PROJ_LAUNCH_S(NWv, TPv, LMv, Sv) \
+  hipExtLaunchKernelGGL((k_proj<NWv, TPv, LMv, Sv>), grid, dim3(kBlock), 0, st, e0, e1, 0, a)
+#define PROJ_LAUNCH(NWv, TPv)                         \
+  do {                                                \
+    if (lmx == 4) PROJ_LAUNCH_S(NWv, TPv, 4, 1);      \
+    else if (lmx == 9) PROJ_LAUNCH_S(NWv, TPv, 9, 1); \
+    else PROJ_LAUNCH_S(NWv, TPv, 16, 1);              \
   } while (0)
+  if (split == 4) {
+    if (nw == 1) PROJ_LAUNCH_S(1, double2, 4, 4);
+    else if (nw == 5) PROJ_LAUNCH_S(5, double2, 4, 4);
+    else PROJ_LAUNCH_S(4, double2, 4, 4);
+  } else
   if (nw == 1 && f32) PROJ_LAUNCH(1, float2);
   else if (nw == 1) PROJ_LAUNCH(1, double2);
   else if (nw == 5) PROJ_LAUNCH(5, double2);
   else PROJ_LAUNCH(4, double2);
 #undef PROJ_LAUNCH
+#undef PROJ_LAUNCH_S
   LAUNCHCHK("k_proj");
   if (c->overlap) {
     HIPCHK(hipEventRecord(c->ev_join, c->side));
@@ -3368,9 +3378,9 @@ static int launch_scatter(salmon_hip_t c, void *hout, double2 s, bool f32 = fals
 }
 
 // the fused KB pass of hout (cin = c of the previous term, cout = c of hout)
-static ProjScatArgs projscat_args(salmon_hip_t c, void *hout, const double2 *cin, double2 *cout, int lm) {
+static ProjScatArgs projscat_args(salmon_hip_t c, void *hout, const double2 *cin, double2 *cout, int split) {
   ProjScatArgs A;
-  A.p = proj_args(c, hout, cout, lm);
+  A.p = proj_args(c, hout, cout, split);
   A.cin = cin;
   A.jexcl = c->d_jexcl;
   A.s = make_double2(1.0, 0.0);
@@ -3388,20 +3398,25 @@ static int launch_kb_fused(salmon_hip_t c, void *hout, bool f32) {
   if (shared)
     if (int rc = launch_scatter(c, hout, make_double2(1.0, 0.0), f32, true, e0, nullptr, false)) return rc;
   const int lm = proj_lm(c->cmax);
-  const ProjScatArgs A = projscat_args(c, hout, c->d_c, c->d_c2, lm);
-  const size_t shmem = sizeof(double2) * (size_t)c->cmax * proj_orb(lm);
+  const int split = proj_split(lm, c->prec != SALMON_HIP_PREC_FP64);
+  const ProjScatArgs A = projscat_args(c, hout, c->d_c, c->d_c2, split);
+  const size_t shmem = sizeof(double2) * (size_t)c->cmax * proj_orb(split);
   dim3 grid((unsigned)(A.p.ngrp * c->natom * c->nk));
   hipEvent_t s0 = shared ? nullptr : e0;
   // LM: registers for the projector values of one point (s+p: 4, up to d: 9, up to f: 16)
-#define KB_LAUNCH(TPv)                                                                                                    \
-  do {                                                                                                                    \
-    if (lm == 4) hipExtLaunchKernelGGL((k_proj_scatter<TPv, 4>), grid, dim3(kBlock), shmem, c->stream, s0, e1, 0, A);      \
-    else if (lm == 9) hipExtLaunchKernelGGL((k_proj_scatter<TPv, 9>), grid, dim3(kBlock), shmem, c->stream, s0, e1, 0, A); \
-    else hipExtLaunchKernelGGL((k_proj_scatter<TPv, 16>), grid, dim3(kBlock), shmem, c->stream, s0, e1, 0, A);             \
+#define KB_LAUNCH_S(TPv, LMv, Sv) \
+  hipExtLaunchKernelGGL((k_proj_scatter<TPv, LMv, Sv>), grid, dim3(kBlock), shmem, c->stream, s0, e1, 0, A)
+#define KB_LAUNCH(TPv)                        \
+  do {                                        \
+    if (lm == 4) KB_LAUNCH_S(TPv, 4, 1);      \
+    else if (lm == 9) KB_LAUNCH_S(TPv, 9, 1); \
+    else KB_LAUNCH_S(TPv, 16, 1);             \
   } while (0)
-  if (f32) KB_LAUNCH(float2);
+  if (split == 4) KB_LAUNCH_S(double2, 4, 4);
+  else if (f32) KB_LAUNCH(float2);
   else KB_LAUNCH(double2);
 #undef KB_LAUNCH
+#undef KB_LAUNCH_S
   LAUNCHCHK("k_proj_scatter");
   std::swap(c->d_c, c->d_c2);
   c->pre_state = 0;
@@ -4356,7 +4371,7 @@ __global__ __launch_bounds__(kBlock, LMX == 4 ? 4 : 2) void kp_proj(const ProjAr
   const ProjArgs a = args[s];
   const int item = xcd_order((int)blockIdx.x - off[s], off[s + 1] - off[s]);
   if (item >= a.ngrp * a.natom * a.nk) return;
-  proj_body<NW, double2, LMX>(a, item);
+  proj_body<NW, double2, LMX, proj_split(LMX, false)>(a, item);
 }
 
 template <int LM>
@@ -4365,7 +4380,7 @@ __global__ __launch_bounds__(kBlock, LM == 4 ? 3 : 2) void kp_proj_scatter(const
   const ProjScatArgs A = args[s];
   const int item = xcd_order((int)blockIdx.x - off[s], off[s + 1] - off[s]);
   if (item >= A.p.ngrp * A.p.natom * A.p.nk) return;
-  proj_scatter_body<double2, LM>(A, item);
+  proj_scatter_body<double2, LM, proj_split(LM, false)>(A, item);
 }
 
 template <int CM>
@@ -4711,7 +4726,7 @@ int batch_packed_tables(salmon_hip_batch *b) {
   }
   size_t kb_shm = 0, cur_shm = 0;
   for (int i = 0; i < ns; ++i) {
-    kb_shm = std::max(kb_shm, sizeof(double2) * (size_t)b->h[i]->cmax * proj_orb(b->lm));
+    kb_shm = std::max(kb_shm, sizeof(double2) * (size_t)b->h[i]->cmax * proj_orb(proj_split(b->lm, false)));
     cur_shm = std::max(cur_shm, cur_shmem(b->h[i]));
   }
   for (int p = 0; p < 2; ++p) {
@@ -4724,7 +4739,7 @@ int batch_packed_tables(salmon_hip_batch *b) {
       salmon_hip_t c = b->h[i];
       void *hh[kMaxComb + 1], *out;
       batch_buffers(b, i, p, hh, &out);
-      pr[i] = proj_args(c, hh[0], c->d_c, b->lm);
+      pr[i] = proj_args(c, hh[0], c->d_c, proj_split(b->lm, false));
       cnt[i] = kb(c) ? proj_blocks(pr[i]) : 0;
       const double2 *cl_buf = ((N - 1) % 2 == 1) ? c->d_c2 : c->d_c;
       last[i] = scatter_args(c, out, make_double2(b->zc[2 * (N - 1)], b->zc[2 * (N - 1) + 1]), cl_buf, false, false);
@@ -4733,7 +4748,7 @@ int batch_packed_tables(salmon_hip_batch *b) {
       const int gx = (int)((c->ngrid + kBlock - 1) / kBlock);
       cd[i] = gx * c->dens_ngrp * c->nspin;
       cs[i] = c->dens_ngrp > 1 ? (int)((c->ngrid * c->nspin + kBlock - 1) / kBlock) : 0;
-      p4[i] = proj_args(c, out, c->d_curnl, b->lm);
+      p4[i] = proj_args(c, out, c->d_curnl, proj_split(b->lm, false));
       c4[i] = c->natom > 0 ? proj_blocks(p4[i]) : 0;
       cl[i] = cur_args(c, out);
       cl_n[i] = c->norb * c->nyt;
@@ -4756,7 +4771,7 @@ int batch_packed_tables(salmon_hip_batch *b) {
         double2 *cout = (n % 2 == 1) ? c->d_c2 : c->d_c;
         sh[i] = scatter_args(c, hh[n], make_double2(1.0, 0.0), cin, true, false);
         shn[i] = kb(c) ? scat_blocks(c, c->ntp_shared) : 0;
-        fu[i] = projscat_args(c, hh[n], cin, cout, b->lm);
+        fu[i] = projscat_args(c, hh[n], cin, cout, proj_split(b->lm, false));
         fun[i] = kb(c) ? proj_blocks(fu[i].p) : 0;
       }
       if (int rc = pack_make(b, b->p_kbsh[p][n - 1], sh, shn, false)) return rc;
