@@ -1855,6 +1855,9 @@ __global__ __launch_bounds__(kBlock) void k_density_sum(DensArgs a) {
 // whole column: z-forward neighbours from a 5-deep register queue, x and
 // y-forward neighbours from an LDS plane carrying 4 extra rows below the tile.
 // Each block writes its 4 partial sums (fixed-order tree) to part(4, tile, orbital).
+// Bound by the rows read; in XCD order the tiles of one orbital share their halo rows' lines in one L2 (96 x 14
+// x 12, 512 orbitals 76 us in launch order, 61 us so; 48^3, 1728 orbitals 868 and 831 us; full rows of 30 and 32
+// points within 1 us, and no gain in the packed launch over many systems).
 // ---------------------------------------------------------------------------
 struct CurArgs {
   const double2 *psi;
@@ -1990,7 +1993,9 @@ __device__ __forceinline__ void current_local_body(const CurArgs &a, int bid) {
   }
 }
 
-__global__ __launch_bounds__(kBlock) void k_current_local(CurArgs a) { current_local_body(a, blockIdx.x); }
+__global__ __launch_bounds__(kBlock) void k_current_local(CurArgs a) {
+  current_local_body(a, xcd_order(blockIdx.x, gridDim.x));
+}
 
 struct CurFinArgs {
   const double *part;      // (4, nslab, norb)
