@@ -417,7 +417,7 @@ def run_batch(steps, warmup):
         "one_by_one_steps_per_s": seq_steps / tseq,
         "speedup_vs_one_by_one": (steps / (t1 - t0)) / (seq_steps / tseq),
         "autotune_choice": choice,
-        "form": "fixed-potential FP64 step; one persistent stencil kernel per halo class and Taylor term, one "
+        "form": "fixed-potential FP64 step; one stencil launch per halo class and Taylor term, one "
                 "packed launch per phase for all systems (phase table, projections, fused KB passes, scatter, "
                 "density, current, dipole); eager launches (graph capture switched off)",
     }

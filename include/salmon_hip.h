@@ -302,9 +302,10 @@ int salmon_hip_update_potential(salmon_hip_t h, const double *rho_dev, const dou
  * orbitals, projectors, V_local); the batch runs the plain fixed-potential step
  * (update_kvector, taylor, calc_density, calc_current, calc_dip of
  * src/rt/time_evolution_step.f90) for all of them together: the stencil passes of
- * all systems of one halo class run as ONE persistent kernel over a combined tile
- * list (the terms without the Taylor sum on the single-system path's delayed-z tiles
- * when every member's rows fit them, z chunks rounded up to multiples of 4 planes),
+ * all systems of one halo class run as ONE launch over a combined tile list (on the
+ * single-system path's delayed-z tiles for rows of up to 64 points and orders up to 4,
+ * one block per tile, z chunks rounded up to multiples of 4 planes; else a persistent
+ * kernel),
  * every other phase (phase table, projections, fused KB passes, scatter,
  * density, current, dipole) runs as ONE launch for all systems (per-system argument
  * records and block offsets on the device; when a system with projectors cannot run
@@ -320,8 +321,8 @@ int salmon_hip_update_potential(salmon_hip_t h, const double *rho_dev, const dou
  *   batch_prepare: Taylor coefficients; builds the tile lists, descriptor tables and
  *     the packed launches' records, sets the step counter to 1.
  *   batch_autotune: times the packed stencil for each candidate (z-chunks per orbital:
- *     the systems' rule, 1 or 2; persistent blocks: 256, 512, 1024, 2048 or one per
- *     tile) and keeps the fastest; *choice = 100*z + blocks/256 (99 = one per tile).
+ *     the rule, 1 or 2; persistent blocks, where the stencil's form is a persistent
+ *     kernel: 256, 512, 1024, 2048 or one per tile) and keeps the fastest; *choice = 100*z + blocks/256 (99 = one per tile).
  *   batch_step: enqueue one step; SALMON_HIP_EINVAL once the step counter has passed the
  *     shortest system's nt (the field tables end there).
  *   batch_set_time: set the step counter (1 .. nt_min + 1).

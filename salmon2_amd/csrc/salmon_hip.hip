@@ -8,8 +8,9 @@
 //                     (v_mfma_f64_16x16x4f64): uVpsi of zpseudo
 //                     (src/common/nonlocal_potential.f90:360-369) for NW = 1 and the
 //                     four moments of calc_current_nonlocal (density_matrix.f90:532-591)
-//                     for NW = 4
-//   k_stencil<HC,NC>  25-point stencil + V_local + k+A gradient
+//                     for NW = 4 (NW = 5: with the next step's projection)
+//   k_proj_scatter    the KB term of a Taylor term with the projection of its result
+//   k_stencilz, k_stencil8, k_stencil<HC,NC>  25-point stencil + V_local + k+A gradient
 //                     (zstencil_typical_seq, zstencil_core/typical/seq.f90:17-127) fed by
 //                     direct global->LDS DMA rings; in the last Taylor term it also forms
 //                     the sum of taylor.f90:53-114

@@ -16,13 +16,14 @@
 // conv = 3x3x3 periodic, weights [27][co][ci]; `up` = nearest upsampling, read on the fly.
 //
 // Kernels:
-//   k_conv<NT>     implicit GEMM on gfx950's double-K v_mfma_f32_16x16x32_bf16: M = 16
+//   k_conv<NT,SK,CI>  implicit GEMM on gfx950's double-K v_mfma_f32_16x16x32_bf16: M = 16
 //                  points per wave, N = NT x 16 output channels, K = 32 of the flattened
 //                  (tap, input channel) index (two taps per instruction at 16 channels);
-//                  also the data gradient (flipped, transposed weights, FP32 output)
+//                  also the data gradient (flipped, transposed weights; FP32 output, or masked by
+//                  the activation)
 //   k_wg_pack, k_wgrad, k_wg_reduce  weight and bias gradient as MFMA over points (M = co, N = ci, K = 32
 //                  points of channel-major copies), FP32 partials reduced in fixed order
-//   small kernels  pooling, gradient routing (mask, down-sum, pool-back), head, MSE, Adam
+//   small kernels  pooling, gradient routing (down-sum, pool-back), head, MSE, Adam
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
