@@ -1632,13 +1632,13 @@ __global__ __launch_bounds__(BS) void k_stencil_packed(const StencilArgs *__rest
 // One thread per touched point and G orbitals of one k-point.  The kernel is
 // bound by the latency of its dependent loads, so the per-point record
 // (orbital-block offset, first entry, entry count, first entry's ilma0 | cnt)
-// comes in one 16-byte load, and with CM > 0 the CM projectors of an entry are
-// loaded together (clamped to the entry's own, unused ones weighted by zero are
-// skipped in the sum, so the order of the additions is the sequential one).
+// comes in one 16-byte load, and with CM > 0 an entry's projectors are loaded CM at a
+// time (clamped to the entry's own, which are skipped in the sum, so the order of the
+// additions is the sequential one).
 // ---------------------------------------------------------------------------
-// Orbitals per thread and projectors per entry loaded together (entries with cmax <= CM), per
-// element type of the chain: FP64 <8, 4>, FP32 <4, 0> (the fastest of G in {4, 8}, CM in {0, 4}
-// measured at 32^3 with 64 s+p atoms).
+// Orbitals per thread and projectors of an entry loaded together, per element type of the chain:
+// FP64 <8, 4>, FP32 <4, 0> (the fastest of G in {4, 8}, CM in {0, 4} measured at 32^3 with 64 s+p
+// atoms; with 9 projectors each, 96 x 14 x 12 and 512 orbitals, CM = 4 takes 51 us and CM = 0 56 us).
 constexpr int kScatG = 8, kScatCM = 4;
 constexpr int kScatG32 = 4, kScatCM32 = 0;
 
@@ -1681,21 +1681,23 @@ __device__ __forceinline__ void nl_scatter_body(const ScatterArgs &a, int bx, in
     const int cnt = lc >> 24;
     const double2 *ze = zb + (size_t)e * a.cmax;
     if (CM > 0) {
-      double2 zv[CM > 0 ? CM : 1], cv[CM > 0 ? CM : 1][G];
+      for (int l0 = 0; l0 < cnt; l0 += CM) {
+        double2 zv[CM > 0 ? CM : 1], cv[CM > 0 ? CM : 1][G];
 #pragma unroll
-      for (int l = 0; l < CM; ++l) {
-        const int lx = min(l, cnt - 1);
-        zv[l] = ze[lx];
+        for (int l = 0; l < CM; ++l) {
+          const int lx = min(l0 + l, cnt - 1);
+          zv[l] = ze[lx];
 #pragma unroll
-        for (int o = 0; o < G; ++o) cv[l][o] = cb[(size_t)(ilma0 + lx) * a.nb + min(o, nob - 1)];
-      }
+          for (int o = 0; o < G; ++o) cv[l][o] = cb[(size_t)(ilma0 + lx) * a.nb + min(o, nob - 1)];
+        }
 #pragma unroll
-      for (int l = 0; l < CM; ++l) {
-        if (l < cnt) {
+        for (int l = 0; l < CM; ++l) {
+          if (l0 + l < cnt) {
 #pragma unroll
-          for (int o = 0; o < G; ++o) {
-            acc[o].x += cv[l][o].x * zv[l].x - cv[l][o].y * zv[l].y;
-            acc[o].y += cv[l][o].x * zv[l].y + cv[l][o].y * zv[l].x;
+            for (int o = 0; o < G; ++o) {
+              acc[o].x += cv[l][o].x * zv[l].x - cv[l][o].y * zv[l].y;
+              acc[o].y += cv[l][o].x * zv[l].y + cv[l][o].y * zv[l].x;
+            }
           }
         }
       }
@@ -3369,15 +3371,9 @@ static int launch_scatter(salmon_hip_t c, void *hout, double2 s, bool f32 = fals
   if (own_events) prof_events(c, SALMON_HIP_KERNEL_NL_SCATTER, &e0, &e1);
   dim3 grid((unsigned)((a.ntp + kBlock - 1) / kBlock), (unsigned)(c->nk * a.ngrp));
   if (f32) {
-    if (c->cmax <= kScatCM32)
-      hipExtLaunchKernelGGL((k_nl_scatter<float2, kScatG32, kScatCM32>), grid, dim3(kBlock), 0, c->stream, e0, e1, 0, a);
-    else
-      hipExtLaunchKernelGGL((k_nl_scatter<float2, kScatG32, 0>), grid, dim3(kBlock), 0, c->stream, e0, e1, 0, a);
+    hipExtLaunchKernelGGL((k_nl_scatter<float2, kScatG32, kScatCM32>), grid, dim3(kBlock), 0, c->stream, e0, e1, 0, a);
   } else {
-    if (c->cmax <= kScatCM)
-      hipExtLaunchKernelGGL((k_nl_scatter<double2, kScatG, kScatCM>), grid, dim3(kBlock), 0, c->stream, e0, e1, 0, a);
-    else
-      hipExtLaunchKernelGGL((k_nl_scatter<double2, kScatG, 0>), grid, dim3(kBlock), 0, c->stream, e0, e1, 0, a);
+    hipExtLaunchKernelGGL((k_nl_scatter<double2, kScatG, kScatCM>), grid, dim3(kBlock), 0, c->stream, e0, e1, 0, a);
   }
   LAUNCHCHK("k_nl_scatter");
   return 0;
@@ -4389,12 +4385,11 @@ __global__ __launch_bounds__(kBlock, LM == 4 ? 3 : 2) void kp_proj_scatter(const
   proj_scatter_body<double2, LM, proj_split(LM, false)>(A, item);
 }
 
-template <int CM>
 __global__ __launch_bounds__(kBlock) void kp_nl_scatter(const ScatterArgs *args, const int *off, int nsys) {
   const int s = pack_find(off, nsys, blockIdx.x);
   const ScatterArgs a = args[s];
   const int lb = (int)blockIdx.x - off[s], gx = (a.ntp + kBlock - 1) / kBlock;
-  nl_scatter_body<double2, kScatG, CM>(a, lb % gx, lb / gx);
+  nl_scatter_body<double2, kScatG, kScatCM>(a, lb % gx, lb / gx);
 }
 
 __global__ __launch_bounds__(kBlock) void kp_density_part(const DensArgs *args, const int *off, int nsys) {
@@ -4494,7 +4489,7 @@ struct salmon_hip_batch {
   // [term] for the fused KB passes); used when every system with projectors runs the fused
   // KB pass, else the step forks per-system launches onto the lanes
   bool packed = false;
-  int lm = 4, cm = 0;                     // template choices common to the systems
+  int lm = 4;                             // template choice common to the systems
   Packed p_kvec, p_proj[2], p_kbsh[2][kMaxComb], p_kbf[2][kMaxComb], p_last[2];
   Packed p_dpart[2], p_dsum[2], p_proj4[2], p_curl[2], p_curo, p_curs, p_dipp, p_dips;
 };
@@ -4715,7 +4710,6 @@ int batch_packed_tables(salmon_hip_batch *b) {
   }
   if (cmax > kMaxLmaPerAtom) return 0;
   b->lm = proj_lm(cmax);
-  b->cm = cmax <= kScatCM ? kScatCM : 0;
   auto kb = [&](salmon_hip_t c) { return kb_fused_on(c); };
   auto scat_blocks = [&](salmon_hip_t c, int ntp) {
     return ntp > 0 ? ((ntp + kBlock - 1) / kBlock) * c->nk * ((c->nb + kScatG - 1) / kScatG) : 0;
@@ -4822,8 +4816,7 @@ int batch_step_packed(salmon_hip_batch *b, int p) {
   for (int n = 1; n <= N; ++n) {
     if (int rc = batch_stencil(b, p, n)) return rc;
     const Packed &S = n < N ? b->p_kbsh[p][n - 1] : b->p_last[p];
-    if (b->cm == kScatCM) PACKED_LAUNCH(kp_nl_scatter<kScatCM>, S, ScatterArgs);
-    else PACKED_LAUNCH(kp_nl_scatter<0>, S, ScatterArgs);
+    PACKED_LAUNCH(kp_nl_scatter, S, ScatterArgs);
     if (n < N) {
       const Packed &F = b->p_kbf[p][n - 1];
       if (b->lm == 4) PACKED_LAUNCH(kp_proj_scatter<4>, F, ProjScatArgs);
