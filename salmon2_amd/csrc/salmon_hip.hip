@@ -1639,7 +1639,11 @@ __global__ __launch_bounds__(BS) void k_stencil_packed(const StencilArgs *__rest
 // Orbitals per thread and projectors of an entry loaded together, per element type of the chain:
 // FP64 <8, 4>, FP32 <4, 0> (the fastest of G in {4, 8}, CM in {0, 4} measured at 32^3 with 64 s+p
 // atoms; with 9 projectors each, 96 x 14 x 12 and 512 orbitals, CM = 4 takes 51 us and CM = 0 56 us).
+// Up to four orbitals with more than four projectors per atom take CM = 0: the clamped loads of CM = 4
+// are G per projector whatever the orbital count (256 x 8 x 8, 128 atoms of 16 projectors, one orbital:
+// 32 us, 11 us with CM = 0; 24 x 22 x 16, 8 atoms, 16 orbitals: 18 us, 31 us with CM = 0).
 constexpr int kScatG = 8, kScatCM = 4;
+constexpr bool scat_plain(int cmax, int nb) { return cmax > kScatCM && 2 * nb <= kScatG; }
 constexpr int kScatG32 = 4, kScatCM32 = 0;
 
 struct ScatterArgs {
@@ -3372,6 +3376,8 @@ static int launch_scatter(salmon_hip_t c, void *hout, double2 s, bool f32 = fals
   dim3 grid((unsigned)((a.ntp + kBlock - 1) / kBlock), (unsigned)(c->nk * a.ngrp));
   if (f32) {
     hipExtLaunchKernelGGL((k_nl_scatter<float2, kScatG32, kScatCM32>), grid, dim3(kBlock), 0, c->stream, e0, e1, 0, a);
+  } else if (scat_plain(c->cmax, c->nb)) {
+    hipExtLaunchKernelGGL((k_nl_scatter<double2, kScatG, 0>), grid, dim3(kBlock), 0, c->stream, e0, e1, 0, a);
   } else {
     hipExtLaunchKernelGGL((k_nl_scatter<double2, kScatG, kScatCM>), grid, dim3(kBlock), 0, c->stream, e0, e1, 0, a);
   }
@@ -4385,11 +4391,12 @@ __global__ __launch_bounds__(kBlock, LM == 4 ? 3 : 2) void kp_proj_scatter(const
   proj_scatter_body<double2, LM, proj_split(LM, false)>(A, item);
 }
 
+template <int CM>
 __global__ __launch_bounds__(kBlock) void kp_nl_scatter(const ScatterArgs *args, const int *off, int nsys) {
   const int s = pack_find(off, nsys, blockIdx.x);
   const ScatterArgs a = args[s];
   const int lb = (int)blockIdx.x - off[s], gx = (a.ntp + kBlock - 1) / kBlock;
-  nl_scatter_body<double2, kScatG, kScatCM>(a, lb % gx, lb / gx);
+  nl_scatter_body<double2, kScatG, CM>(a, lb % gx, lb / gx);
 }
 
 __global__ __launch_bounds__(kBlock) void kp_density_part(const DensArgs *args, const int *off, int nsys) {
@@ -4489,7 +4496,7 @@ struct salmon_hip_batch {
   // [term] for the fused KB passes); used when every system with projectors runs the fused
   // KB pass, else the step forks per-system launches onto the lanes
   bool packed = false;
-  int lm = 4;                             // template choice common to the systems
+  int lm = 4, cm = kScatCM;               // template choices common to the systems
   Packed p_kvec, p_proj[2], p_kbsh[2][kMaxComb], p_kbf[2][kMaxComb], p_last[2];
   Packed p_dpart[2], p_dsum[2], p_proj4[2], p_curl[2], p_curo, p_curs, p_dipp, p_dips;
 };
@@ -4710,6 +4717,9 @@ int batch_packed_tables(salmon_hip_batch *b) {
   }
   if (cmax > kMaxLmaPerAtom) return 0;
   b->lm = proj_lm(cmax);
+  b->cm = cmax > kScatCM ? 0 : kScatCM;  // 0 where it is every larger system's form
+  for (salmon_hip_t c : b->h)
+    if (c->natom > 0 && c->cmax > kScatCM && !scat_plain(c->cmax, c->nb)) b->cm = kScatCM;
   auto kb = [&](salmon_hip_t c) { return kb_fused_on(c); };
   auto scat_blocks = [&](salmon_hip_t c, int ntp) {
     return ntp > 0 ? ((ntp + kBlock - 1) / kBlock) * c->nk * ((c->nb + kScatG - 1) / kScatG) : 0;
@@ -4816,7 +4826,8 @@ int batch_step_packed(salmon_hip_batch *b, int p) {
   for (int n = 1; n <= N; ++n) {
     if (int rc = batch_stencil(b, p, n)) return rc;
     const Packed &S = n < N ? b->p_kbsh[p][n - 1] : b->p_last[p];
-    PACKED_LAUNCH(kp_nl_scatter, S, ScatterArgs);
+    if (b->cm == kScatCM) PACKED_LAUNCH(kp_nl_scatter<kScatCM>, S, ScatterArgs);
+    else PACKED_LAUNCH(kp_nl_scatter<0>, S, ScatterArgs);
     if (n < N) {
       const Packed &F = b->p_kbf[p][n - 1];
       if (b->lm == 4) PACKED_LAUNCH(kp_proj_scatter<4>, F, ProjScatArgs);
