@@ -527,10 +527,14 @@ __device__ __forceinline__ void proj_scatter_body(const ProjScatArgs &A, int bid
   const int *jx = a.jidx + (size_t)a.nps * ia;
   const int *jxe = A.jexcl + (size_t)a.nps * ia;
   const double2 *zk = a.zekr + (size_t)a.nps * ((size_t)al.x + (size_t)a.nlma * ik);
-  const int jt = lane % JC, o0 = ow + lane / JC, l0 = zt / JC;
+  // This thread's point of a chunk and its orbitals o0 + kOs r.  S = 1: over the whole block, so that all waves
+  // complete points where the orbitals fill one wave's MFMA columns only (16 orbitals of 20 x 26 x 28, 8 atoms of 9
+  // projectors, mixed: Taylor step 619 us, 813 us with each wave on its own 16; 64 orbitals the same).
+  constexpr int kOs = P::kT / JC;
+  const int jt = zt % JC, o0 = zt / JC, l0 = o0;
   TP *h = (TP *)a.psi + (kbase + grp * P::OB + o0) * a.osz;
-  const size_t hs = (64 / JC) * a.osz;
-  const int nor = a.nb - grp * P::OB - o0;  // orbitals of this lane: r with (64 / JC) r < nor
+  const size_t hs = kOs * a.osz;
+  const int nor = a.nb - grp * P::OB - o0;  // orbitals of this thread: r with kOs r < nor
   constexpr int kStep = S * JC;
   const int jb = S == 4 ? wave * JC : 0;
   int jnext = jb + jt < m ? jx[jb + jt] : 0;
@@ -557,7 +561,7 @@ __device__ __forceinline__ void proj_scatter_body(const ProjScatArgs &A, int bid
       TP v;
       v.x = 0;
       v.y = 0;
-      if (j < m && (64 / JC) * r < nor) v = h[r * hs + jload];
+      if (j < m && kOs * r < nor) v = h[r * hs + jload];
       pre[r] = v;
     }
   };
@@ -567,9 +571,9 @@ __device__ __forceinline__ void proj_scatter_body(const ProjScatArgs &A, int bid
     // staging the chunk
 #pragma unroll
     for (int r = 0; r < P::kPer; ++r) {
-      const int o = o0 + (64 / JC) * r;
+      const int o = o0 + kOs * r;
       double2 v = cvt2<double2>(pre[r]);
-      if (xload >= 0 && (64 / JC) * r < nor) {
+      if (xload >= 0 && kOs * r < nor) {
         double2 sum = make_double2(0.0, 0.0);
 #pragma unroll
         for (int l = 0; l < LM; ++l) {
@@ -585,7 +589,7 @@ __device__ __forceinline__ void proj_scatter_body(const ProjScatArgs &A, int bid
         h[r * hs + jload] = vt;
         v = cvt2<double2>(vt);
       }
-      sp[P::so(jt, o - ow)] = v;
+      (S == 4 ? sp : st.sp[o >> 4])[P::so(jt, o & 15)] = v;
     }
 #pragma unroll
     for (int r = 0; r < P::kZPer; ++r) {
