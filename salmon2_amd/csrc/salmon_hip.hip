@@ -116,6 +116,7 @@ struct KvecArgs {
   const int *itt;
   int tmax;              // last row of actab (nt + 1); the step counter is clamped to 1..tmax
   int natom, nlma, nps, nk, nent, cmax;
+  int split;             // blocks per atom and k: 1, or cmax of one projector each
 };
 
 // the midpoint field of the current step from the device table, else the by-value field
@@ -132,14 +133,15 @@ __device__ __forceinline__ void kvec_field(const KvecArgs &a, double &ax, double
   }
 }
 
-// One block per atom and k: a point's phase serves all projectors of its atom.
-__device__ __forceinline__ void update_kvector_body(const KvecArgs &a, int ia, int ik) {
+// A block takes all projectors of an atom at one k (a point's phase serves them all) or, in launches of
+// few atoms and k-points, one of them (kvec_split).
+__device__ __forceinline__ void update_kvector_body(const KvecArgs &a, int ib, int ik) {
   double ax, ay, az;
   kvec_field(a, ax, ay, az);
   const double kx = a.veck[3 * ik + 0] + ax;
   const double ky = a.veck[3 * ik + 1] + ay;
   const double kz = a.veck[3 * ik + 2] + az;
-  if (ia == 0 && threadIdx.x == 0) {
+  if (ib == 0 && threadIdx.x == 0) {
     double *kp = a.kpar + 16 * ik;
     double ss = kx * kx;
     ss = ss + ky * ky;
@@ -154,25 +156,29 @@ __device__ __forceinline__ void update_kvector_body(const KvecArgs &a, int ia, i
     kp[14] = ky;
     kp[15] = kz;
   }
+  const int ia = ib / a.split;
   if (ia >= a.natom) return;
   const int2 al = a.atom_lma[ia];
+  const int l0 = ib - ia * a.split;
+  const int nl = a.split > 1 ? min(1, al.y - l0) : al.y;  // the block's projectors: l0 .. l0 + nl - 1
+  if (nl < 1) return;
   const int m = a.mps[ia];
   for (int j = threadIdx.x; j < m; j += blockDim.x) {
-    const double *uv = a.uv + (size_t)j + (size_t)a.nps * al.x;
+    const double *uv = a.uv + (size_t)j + (size_t)a.nps * (al.x + l0);
     double u[4];  // the first projectors' values beside the phase's latency
 #pragma unroll
-    for (int l = 0; l < 4; ++l) u[l] = l < al.y ? uv[(size_t)a.nps * l] : 0.0;
+    for (int l = 0; l < 4; ++l) u[l] = l < nl ? uv[(size_t)a.nps * l] : 0.0;
     const int e = a.entof[(size_t)j + (size_t)a.nps * ia];
     const double *r = a.rxyz + 3 * ((size_t)j + (size_t)a.nps * ia);
     const double th = kx * r[0] + ky * r[1] + kz * r[2];
     double s, c;
     sincos(th, &s, &c);
-    double2 *ze = a.zent + (size_t)a.cmax * ((size_t)e + (size_t)a.nent * ik);
-    double2 *zk = a.zekr + (size_t)j + (size_t)a.nps * ((size_t)al.x + (size_t)a.nlma * ik);
+    double2 *ze = a.zent + (size_t)a.cmax * ((size_t)e + (size_t)a.nent * ik) + l0;
+    double2 *zk = a.zekr + (size_t)j + (size_t)a.nps * ((size_t)(al.x + l0) + (size_t)a.nlma * ik);
 #pragma unroll
     for (int l = 0; l < 4; ++l)
-      if (l < al.y) zk[(size_t)a.nps * l] = ze[l] = make_double2(c * u[l], -s * u[l]);
-    for (int l = 4; l < al.y; ++l) {
+      if (l < nl) zk[(size_t)a.nps * l] = ze[l] = make_double2(c * u[l], -s * u[l]);
+    for (int l = 4; l < nl; ++l) {
       const double ul = uv[(size_t)a.nps * l];
       zk[(size_t)a.nps * l] = ze[l] = make_double2(c * ul, -s * ul);
     }
@@ -2964,6 +2970,14 @@ int salmon_hip_copy_if(salmon_hip_t c, const int *flag_dev, double *dst_dev, con
   return 0;
 }
 
+// Blocks per atom and k of the phase table for a launch over `atoms` (atom, k) pairs: one (one phase a point) from
+// half a block per CU on; fewer leave the chip idle and take one per projector (32^3, one atom of 16 projectors, 4
+// bohr: 21 us against 161; 64 atoms, radius 5: 16 projectors each 35 and 49 us, four 12.4 and 13.3; 128 pairs
+// of them 68 and 49 us, 18.7 and 15.3; 512 pairs of 16 at radius 2.5 33 and 26 us).
+static int kvec_split(long atoms, int cmax) { return atoms >= 128 ? 1 : std::max(1, cmax); }
+
+static int kvec_blocks(const KvecArgs &a) { return std::max(1, a.natom * a.split); }
+
 static KvecArgs kvec_args(salmon_hip_t c, const double *vec_Ac, const double *actab, const int *itt, int tmax) {
   KvecArgs a;
   a.veck = c->d_veck;
@@ -2971,6 +2985,7 @@ static KvecArgs kvec_args(salmon_hip_t c, const double *vec_Ac, const double *ac
   a.uv = c->d_uv;
   a.mps = c->d_mps;
   a.natom = c->nlma > 0 ? c->natom : 0;
+  a.split = kvec_split((long)a.natom * c->nk, c->cmax);
   a.atom_lma = c->d_atom_lma;
   a.entof = c->d_entof;
   a.zekr = c->d_zekr;
@@ -3007,7 +3022,7 @@ static int update_kvector_impl(salmon_hip_t c, const double *vec_Ac, const doubl
   c->staged = false;
   c->pre_state = 0;
   const KvecArgs a = kvec_args(c, vec_Ac, actab, itt, tmax);
-  dim3 grid(std::max(1, a.natom), c->nk);
+  dim3 grid(kvec_blocks(a), c->nk);
   hipLaunchKernelGGL(k_update_kvector, grid, dim3(kBlock), 0, c->stream, a);
   LAUNCHCHK("k_update_kvector");
   c->have_k = true;
@@ -4073,7 +4088,7 @@ int salmon_hip_current_next(salmon_hip_t c, const double *vec_Ac, const void *ps
   ka.zekr = c->d_zekr_n;
   ka.zent = c->d_zent_n;
   ka.kpar = c->d_kpar_n;
-  hipLaunchKernelGGL(k_update_kvector, dim3(std::max(1, ka.natom), c->nk), dim3(kBlock), 0, c->stream, ka);
+  hipLaunchKernelGGL(k_update_kvector, dim3(kvec_blocks(ka), c->nk), dim3(kBlock), 0, c->stream, ka);
   LAUNCHCHK("k_update_kvector");
   c->staged = true;
   memcpy(c->staged_A, vec_Ac_next, sizeof(c->staged_A));
@@ -4373,7 +4388,7 @@ __device__ __forceinline__ int pack_find(const int *off, int nsys, int b) {
 __global__ __launch_bounds__(kBlock) void kp_update_kvector(const KvecArgs *args, const int *off, int nsys) {
   const int s = pack_find(off, nsys, blockIdx.x);
   const KvecArgs a = args[s];
-  const int lb = (int)blockIdx.x - off[s], gx = max(1, a.natom);
+  const int lb = (int)blockIdx.x - off[s], gx = max(1, a.natom * a.split);
   update_kvector_body(a, lb % gx, lb / gx);
 }
 
@@ -4732,9 +4747,14 @@ int batch_packed_tables(salmon_hip_batch *b) {
   std::vector<int> cnt(ns);
   {
     std::vector<KvecArgs> r(ns);
+    long atoms = 0;
     for (int i = 0; i < ns; ++i) {
       r[i] = kvec_args(b->h[i], nullptr, b->sys[i].actab, b->d_itt, b->sys[i].nt + 1);
-      cnt[i] = std::max(1, r[i].natom) * b->h[i]->nk;
+      atoms += (long)r[i].natom * r[i].nk;
+    }
+    for (int i = 0; i < ns; ++i) {
+      r[i].split = kvec_split(atoms, r[i].cmax);
+      cnt[i] = kvec_blocks(r[i]) * r[i].nk;
     }
     if (int rc = pack_make(b, b->p_kvec, r, cnt, false)) return rc;
   }

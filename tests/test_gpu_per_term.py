@@ -81,3 +81,35 @@ def test_batch_few_orbitals(oracle_lib, nos):
         _, cur, dip, rne = oracle_lib.Oracle(s).rt_run(nt=nt, psi=s.psi)
         for k, ref in (("curr", cur), ("dip", dip), ("rne", rne)):
             assert rel(g[k], ref) <= 1e-9, k
+
+
+@pytest.mark.parametrize("whole", [True, False])
+@pytest.mark.parametrize("nk,lmax", [((1, 1, 1), 0), ((1, 3, 5), 3), ((1, 2, 8), 2), ((1, 2, 8), 3), ((1, 1, 17), 1)])
+def test_phase_table_blocks(oracle_lib, nk, lmax, whole):
+    """The phase table by projector (below 128 atoms x k: 8 x 15) and by atom (from 8 x 16 on), as H psi reads it:
+    its per-point form in the projections and its per-entry form in the scatter and the shared points."""
+    import torch
+
+    from salmon2_amd.hip import Handle
+
+    print(f"[gpu] phase table k={nk} lmax={lmax} whole={whole}", flush=True)
+    s = system.make_si_system(n=(12, 11, 13), no=1, lmax=lmax, rcut=3.6, nkgrid=nk, seed=347)
+    h = Handle(s, stream=torch.cuda.current_stream())
+    if not whole:
+        h._set_shape(0, 0)
+    O = oracle_lib.Oracle(s)
+    psi = torch.from_numpy(s.psi).cuda()
+    out = torch.zeros_like(psi)
+    cur = torch.zeros(3, dtype=torch.float64, device="cuda")
+    for a in (A, -2.0 * A):
+        h.update_kvector(a)
+        O.update_kvector(a)
+        h.hpsi(psi, out)
+        ref = O.hpsi(a, s.psi)[..., : s.ny, :]
+        assert rel(out.cpu().numpy()[..., : s.ny, :], ref) <= 1e-12
+    h.current_next(a, psi, cur, A)  # the table of A built ahead
+    h.update_kvector(A)
+    O.update_kvector(A)
+    h.hpsi(psi, out)
+    assert rel(out.cpu().numpy()[..., : s.ny, :], O.hpsi(A, s.psi)[..., : s.ny, :]) <= 1e-12
+    h.close()
