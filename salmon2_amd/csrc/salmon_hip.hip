@@ -2372,8 +2372,9 @@ __device__ __forceinline__ void dft_pair(const T *x, const double2 *tw, int n, i
 __device__ __forceinline__ double2 times_i(double s, const double2 &b) { return make_double2(-s * b.y, s * b.x); }
 
 // forward z of the real density: out[kz][column], kz = 0 .. n/2
+template <int COLS>
 __global__ __launch_bounds__(256) void k_dft_zr(DftArgs a) {
-  constexpr int COLS = 16, BS = 256;
+  constexpr int BS = 256;
   extern __shared__ double2 lds[];
   if (a.skip && *a.skip) return;  // a device-side gate switched this launch off
   double2 *tw = lds;
@@ -4159,9 +4160,14 @@ int salmon_hip_set_poisson(salmon_hip_t c, const double *al) {
 // Columns per block of the complex passes: 8 (whole 128-byte lines) while their tile fits, else 4.
 static int dft_cols(int n) { return n <= 128 ? 8 : 4; }
 
+// Few columns of many planes: 4 of them per block in the z passes too (16 in the first and 8 in the last leave
+// most CUs idle and a thread several rounds of outputs).  Potential update, one and two spins: 12 x 12 x 96 34 and 39
+// us with 16 and 8, 23 and 26 us with 4; 16 x 16 x 256 87 and 94 us, 54 and 61 us; 64^3 44 us both, 128^3 200 us
+// with 16 and 8, 214 us with 4; 31 x 37 x 41, two spins, 28 and 30 us.
+static bool dft_few(int n, int plane) { return n >= 64 && plane <= 4096; }
+
 template <typename F8, typename F4>
-static void launch_dft(hipStream_t st, const DftArgs &a, int tiles, F8 f8, F4 f4) {
-  const int cols = dft_cols(a.n);
+static void launch_dft(hipStream_t st, const DftArgs &a, int tiles, int cols, F8 f8, F4 f4) {
   const size_t shm = sizeof(double2) * (size_t)a.n * (1 + tiles * cols);
   const dim3 grid((unsigned)((a.ncols + cols - 1) / cols));
   if (cols == 8) hipLaunchKernelGGL(f8, grid, dim3(256), shm, st, a);
@@ -4196,30 +4202,34 @@ static int hartree_impl(salmon_hip_t c, const double *rho_dev, const double *rho
   a.out = c->d_fft[0];
   a.tw = c->d_tw[2];
   a.n = c->nz; a.inner = plane; a.ncols = plane;
-  hipLaunchKernelGGL(k_dft_zr, dim3((unsigned)((plane + 15) / 16)), dim3(256), sizeof(double2) * c->nz * 9, c->stream, a);
+  const bool few = dft_few(c->nz, plane);
+  if (few)
+    hipLaunchKernelGGL(k_dft_zr<4>, dim3((unsigned)((plane + 3) / 4)), dim3(256), sizeof(double2) * c->nz * 3, c->stream, a);
+  else
+    hipLaunchKernelGGL(k_dft_zr<16>, dim3((unsigned)((plane + 15) / 16)), dim3(256), sizeof(double2) * c->nz * 9, c->stream, a);
   LAUNCHCHK("k_dft_zr");
   a.in = c->d_fft[0]; a.out = c->d_fft[1];
   a.tw = c->d_tw[1];
   a.n = c->ny; a.inner = c->nx; a.ncols = nkz * c->nx;
-  launch_dft(c->stream, a, 1, k_dft_y<8>, k_dft_y<4>);
+  launch_dft(c->stream, a, 1, dft_cols(a.n), k_dft_y<8>, k_dft_y<4>);
   LAUNCHCHK("k_dft_y");
   a.in = a.out = c->d_fft[1];
   a.tw = c->d_tw[0];
   a.n = c->nx; a.inner = 1; a.ncols = nkz * c->ny;
-  launch_dft(c->stream, a, 2, k_dft_x<8>, k_dft_x<4>);
+  launch_dft(c->stream, a, 2, dft_cols(a.n), k_dft_x<8>, k_dft_x<4>);
   LAUNCHCHK("k_dft_x");
   a.sg = 1.0;
   a.in = c->d_fft[1]; a.out = c->d_fft[0];
   a.tw = c->d_tw[1];
   a.n = c->ny; a.inner = c->nx; a.ncols = nkz * c->nx;
-  launch_dft(c->stream, a, 1, k_dft_y<8>, k_dft_y<4>);
+  launch_dft(c->stream, a, 1, dft_cols(a.n), k_dft_y<8>, k_dft_y<4>);
   LAUNCHCHK("k_dft_y");
   a.in = c->d_fft[0]; a.out = nullptr;
   a.tw = c->d_tw[2];
   a.n = c->nz; a.inner = plane; a.ncols = plane;
   a.vh = vh_dev;
   if (!vh_dev) a.v = *v;
-  launch_dft(c->stream, a, 1, k_dft_zi<8>, k_dft_zi<4>);
+  launch_dft(c->stream, a, 1, few ? 4 : dft_cols(a.n), k_dft_zi<8>, k_dft_zi<4>);
   LAUNCHCHK("k_dft_zi");
   return 0;
 }
