@@ -3306,7 +3306,7 @@ static int launch_tilez_fp64(salmon_hip_ctx *c, int nc, dim3 grid, hipEvent_t e0
 
 // Tiles of at most 256 points with a halo on x and y for rows above 64 points: the split of the plane
 // that moves the fewest slot chunks.
-static void tilez_xtiles(StencilArgs &a) {
+static int tilez_xtiles(StencilArgs &a) {
   int best = INT_MAX;
   for (int nxt = 2; nxt <= 16; ++nxt) {
     const int TX = (a.nx + nxt - 1) / nxt;
@@ -3322,9 +3322,11 @@ static void tilez_xtiles(StencilArgs &a) {
       break;
     }
   }
+  if (best == INT_MAX) return fail(SALMON_HIP_EINVAL, "no x/y tiles for a plane of %d x %d points", a.nx, a.ny);
   a.nxt = (a.nx + a.TX - 1) / a.TX;
   a.nyt = (a.ny + a.TY - 1) / a.TY;
   a.nblk = a.nk * a.nb * a.nxt * a.nyt * a.nzt;
+  return 0;
 }
 
 template <typename TI, typename R, typename TO, int NCH, bool PR>
@@ -3359,7 +3361,9 @@ static int launch_stencil_hc(salmon_hip_ctx *c, int stage, int nc, dim3 grid, hi
     }
   }
   if (nc == 4) return launch_stencil_t<double2, double, double2, HC, 4>(c, grid, e0, e1, a);
-  return launch_stencil_t<double2, double, double2, HC, 5>(c, grid, e0, e1, a);
+  if (nc == 5) return launch_stencil_t<double2, double, double2, HC, 5>(c, grid, e0, e1, a);
+  // the other FP64 terms are stencil_tilez's on every grid (tilez_fits, tilez_xtiles)
+  return fail(SALMON_HIP_EINVAL, "no stencil form for %d earlier terms on rows of %d points", nc, a.nx);
 }
 
 extern "C" {
@@ -3521,7 +3525,7 @@ static int launch_hpsi(salmon_hip_t c, int kind, const void *in, void *hout, boo
   } else if (tilez_fits(stage, nc, a)) rc = launch_tilez_t<double2, float, float2>(c, grid, e0, e1, a);
   else if (tile8_fits(c, stage, nc, a)) rc = launch_tile8_t<float2, float, float2>(c, grid, e0, e1, a);
   else if (stage == kStagePlain && nc <= kTilezComb && a.nx > 64) {
-    tilez_xtiles(a);
+    if (int rx = tilez_xtiles(a)) return rx;
     if (c->mid_nzt == 0 || nc >= 0) tilez_zchunks(a);
     rc = launch_tilez_fp64<true>(c, nc, dim3((unsigned)a.nblk), e0, e1, a);
   } else if (hc <= 1) rc = launch_stencil_hc<1>(c, stage, nc, grid, e0, e1, a);
