@@ -2582,6 +2582,7 @@ struct salmon_hip_ctx {
   // nonlocal
   int natom = 0, nps = 0, nlma = 0, nent = 0;
   int cmax = 0;
+  double kbval = 0.0;  // projector values of an orbital: sum over atoms of sphere points x projectors
   int *d_mps = nullptr, *d_jidx = nullptr, *d_pt_off = nullptr;
   int *d_pt_lma = nullptr, *d_entof = nullptr;
   int4 *d_tp_info = nullptr;  // per touched point: orbital-block offset, first entry, entry count, its pt_lma
@@ -2795,6 +2796,7 @@ int salmon_hip_set_nonlocal(salmon_hip_t c, int natom, int nps, const int *mps, 
   c->pre_state = 0;
   dfree(c->d_c2); dfree(c->d_jexcl); dfree(c->d_tp_shared);
   dfree(c->d_tp_info);
+  c->kbval = 0.0;
   c->natom = c->nps = c->nlma = c->nent = c->cmax = c->ntp = c->ntp_shared = 0;
   c->have_k = false;
   if (natom == 0 || nlma == 0) return 0;
@@ -2833,7 +2835,11 @@ int salmon_hip_set_nonlocal(salmon_hip_t c, int natom, int nps, const int *mps, 
   for (size_t g = 0; g < c->ngrid; ++g) cnt[g + 1] += cnt[g];
   const int nent = cnt[c->ngrid];
   int cmax = 1;
-  for (int ia = 0; ia < natom; ++ia) cmax = std::max(cmax, atom_lma[ia].y);
+  double kbval = 0.0;
+  for (int ia = 0; ia < natom; ++ia) {
+    cmax = std::max(cmax, atom_lma[ia].y);
+    kbval += (double)mps[ia] * atom_lma[ia].y;
+  }
   // CSR point -> (atom, j) entries; atom-major fill keeps each point's entries
   // in ascending ilma, the order zpseudo adds them in
   std::vector<int> pt_lma(std::max(nent, 1), 0);
@@ -2905,6 +2911,7 @@ int salmon_hip_set_nonlocal(salmon_hip_t c, int natom, int nps, const int *mps, 
   c->nlma = nlma;
   c->nent = nent;
   c->cmax = cmax;
+  c->kbval = kbval;
   c->ntp = (int)tp_info.size();
   c->ntp_shared = (int)tp_shared.size();
   return 0;
@@ -3613,6 +3620,36 @@ static bool small_fits(const salmon_hip_ctx *c) {
   return small_shape(c).cls >= 0;
 }
 
+// Where the per-term kernels are the faster ones on such a grid: a block reads all projector values of its
+// orbital (kbval) in every term, k_proj and k_proj_scatter once for 16 or 64 orbitals, and spread over more
+// blocks with more atoms.  Up to one orbital per CU the whole-orbital step always won or tied; with few values it
+// keeps that for any number of orbitals.  Measured, one Taylor step of order 4, whole orbital against per term:
+// 16^3, 8 atoms of 9 projectors (18 000 values), 4096 orbitals 1369 and 1385 us; 18^3, 9 projectors (26 000), 1024
+// orbitals 757 and 807 us, 2048 1573 and 1239 us; 12^3, 16 projectors (56 000), 512 orbitals 620 and 794 us, 2048
+// 2336 and 1320 us; 12 x 12 x 24, 16 atoms of 16 (24 000), 768 orbitals 324 and 342 us, 2048 885 and 759 us.  Half of
+// that with more than eight atoms where one block fills a CU's LDS: 10 x 20 x 30, 16 atoms of 9 (26 000), 512
+// orbitals 423 and 428 us, 768 635 and 522 us.
+static bool small_one_per_cu(const salmon_hip_ctx *c) { return c->natom > 8 && small_shape(c).lds > 80 * 1024; }
+
+static bool small_step(const salmon_hip_ctx *c, int n_hamil) {
+  if (!small_fits(c)) return false;
+  return c->norb <= 256 || c->kbval <= 21e3 ||
+         (double)c->norb * c->kbval * c->natom <= (small_one_per_cu(c) ? 47e6 : 94e6) * n_hamil;
+}
+
+// One application alone: the per-term kernels' three launches are worth their cost above about a thousand
+// orbitals (16^3, 1024 orbitals: 93 us in one launch, 112 per term; 15x17x14, 1600 orbitals: 150 and 126;
+// 12x12x24, 2048 orbitals: 171 and 158), with many projector values or atoms earlier (18^3, 26 000 values, 512
+// orbitals 120 and 147 us, 1024 235 and 200 us; 14 x 13 x 15, 86 000, 256 orbitals 148 and 172 us, 320 261 and
+// 182 us), and beyond one orbital per CU where no second block fits its LDS and 16 atoms fill the projections
+// (10 x 20 x 30, 320 orbitals 106 and 64 us).
+static bool small_hpsi(const salmon_hip_ctx *c) {
+  if (c->norb > 1024 || !small_fits(c)) return false;
+  if (c->norb <= 256) return true;
+  if (small_one_per_cu(c)) return false;
+  return (double)c->norb * c->kbval * c->natom <= 196e6;
+}
+
 static SmallArgs small_args(salmon_hip_t c, const void *psi, void *out, void *h1) {
   SmallArgs a;
   memset(&a, 0, sizeof(a));
@@ -3694,10 +3731,7 @@ int salmon_hip_hpsi(salmon_hip_t c, const void *tpsi, void *htpsi) {
   if (int rc = check(c)) return rc;
   if (!tpsi || !htpsi || tpsi == htpsi) return fail(SALMON_HIP_EINVAL, "tpsi/htpsi invalid or aliased");
   if (int rc = ready(c)) return rc;
-  // one application alone: the per-term kernels' three launches are worth their cost above about a
-  // thousand orbitals (16^3, 1024 orbitals: 93 us in one launch, 112 per term; 15x17x14, 1600
-  // orbitals: 150 and 126; 12x12x24, 2048 orbitals: 171 and 158)
-  if (c->norb <= 1024 && small_fits(c)) {
+  if (small_hpsi(c)) {
     SmallArgs a = small_args(c, tpsi, nullptr, htpsi);
     return launch_taylor_small(c, SALMON_HIP_KERNEL_HPSI0, a);
   }
@@ -3761,7 +3795,7 @@ extern "C" {
 // first = 1: the whole chain; first = 2: h_1 = sshtpsi is H psi of a previous call, to be shifted by dv
 static int taylor_fp64(salmon_hip_t c, const double *zc, int n_hamil, void *tspsi_in, void *tspsi_out, void *sshtpsi,
                        int first, const double *dv = nullptr) {
-  if (small_fits(c)) {
+  if (small_step(c, n_hamil)) {
     SmallArgs a = small_args(c, tspsi_in, tspsi_out, n_hamil >= 2 ? sshtpsi : nullptr);
     for (int n = 0; n < n_hamil; ++n) a.zc[n] = make_double2(zc[2 * n], zc[2 * n + 1]);
     a.nterm = n_hamil;
@@ -4016,6 +4050,16 @@ static bool small_current_args(salmon_hip_t c, const void *psi, const CurFinArgs
   return small_current_lds(c, a.nsub) <= kSmallLds;
 }
 
+// The whole-orbital current: alone on a CU it is bound by the local part's LDS reads and by an orbital's moments,
+// which the per-term kernels spread over the chip once the orbitals are many.  Measured, whole orbital
+// against per term: 16^3, 2048 orbitals of 4, 9 and 16 projectors per atom 81 and 83, 113 and 126, 146 and 159 us,
+// 4096 orbitals 166 and 146, 241 and 172, 319 and 208 us; 18^3, 1024 orbitals of 9 103 and 133 us, 2048 225 and
+// 194 us; up to 3456 points with up to 4 projectors it stays ahead (12^3, 4096 orbitals 77 and 101 us).
+static bool small_current(const salmon_hip_ctx *c) {
+  if (!small_fits(c)) return false;
+  return (double)c->norb * c->ngrid <= 8.5e6 || (c->cmax <= 4 && c->ngrid <= 3500);
+}
+
 static int launch_current_small(salmon_hip_t c, const SmallCurArgs &a) {
   static std::atomic<unsigned long long> attr_dev{0};
   if (int rc = lds_attr((const void *)k_current_small, attr_dev, kSmallLds)) return rc;
@@ -4029,7 +4073,7 @@ static int launch_current_small(salmon_hip_t c, const SmallCurArgs &a) {
 
 static int current_impl(salmon_hip_t c, const double *vec_Ac, const double *actab, const int *itt, const void *psi,
                         double *curr_dev, int tmax = 0, bool next = false) {
-  if (!actab && small_fits(c)) {
+  if (!actab && !next && small_current(c)) {
     SmallCurArgs a;
     if (small_current_args(c, psi, curfin_args(c, vec_Ac, actab, itt, curr_dev, tmax), a)) {
       if (int rc = launch_current_small(c, a)) return rc;
@@ -4097,8 +4141,8 @@ int salmon_hip_current_next(salmon_hip_t c, const double *vec_Ac, const void *ps
   LAUNCHCHK("k_update_kvector");
   c->staged = true;
   memcpy(c->staged_A, vec_Ac_next, sizeof(c->staged_A));
-  // (the whole-orbital current of a small grid leaves the projection to the whole-orbital Taylor step)
-  const void *pre = small_fits(c) ? nullptr : psi;
+  // (the whole-orbital kernels of a small grid form no projection ahead and use none)
+  const void *pre = small_step(c, 4) || small_current(c) ? nullptr : psi;
   if (int rc = current_impl(c, vec_Ac, nullptr, nullptr, psi, curr_dev, 0, pre != nullptr)) return rc;
   c->pre_state = pre ? 1 : 0;
   c->pre_psi = pre;
