@@ -174,15 +174,20 @@ int salmon_hip_set_precision(salmon_hip_t h, int mode);
 
 /*
  * Project autotuner (no counterpart in the reference): times the stencil pass of the
- * terms without the Taylor sum under each candidate launch shape — whole xy-plane
- * tiles (when nx*ny <= 1024) with 1 or 2 z-chunks per orbital, 256-point y-tiles with
- * 1, 2 or 4 z-chunks — `reps` launches each on handle-allocated scratch, and keeps the
- * fastest for later hpsi/taylor calls.  *choice = 10*plane + z_chunks, *best_ms its
- * time per launch (either may be null).  Needs V_local and vec_Ac set; synchronises.
+ * terms without the Taylor sum under each candidate launch shape — the rule by sizes that
+ * a new handle has, whole xy-plane tiles (when nx*ny <= 1024) with 1 or 2 z-chunks per
+ * orbital, 256-point y-tiles with 1, 2 or 4 z-chunks — `reps` launches each on
+ * handle-allocated scratch, and keeps the fastest for later hpsi/taylor calls (the rule
+ * unless another is more than 2% faster).  Where the rule runs each orbital of a small grid
+ * in one block (FP64), the rule is kept and that kernel's time for one H psi returned.
+ * *choice = 10*plane + z_chunks (-10: the rule), *best_ms its time per launch (either may
+ * be null).  Needs V_local and vec_Ac set; synchronises.
  */
 int salmon_hip_autotune(salmon_hip_t h, int reps, int *choice, double *best_ms);
 
-/* Set the launch shape directly: whole_plane -1 (rule) / 0 / 1, z_chunks 0 (rule) or a count. */
+/* Set the launch shape directly: whole_plane -1 (rule) / 0 / 1, z_chunks 0 (rule) or a count.
+   (-1, 0) is the rule and the state of a new handle; any other shape also selects the per-term
+   kernels on the small grids where the rule runs each orbital in one block. */
 int salmon_hip_set_launch_shape(salmon_hip_t h, int whole_plane, int z_chunks);
 
 /* Run the KB projections on a second stream of the handle, concurrently with the stencil
