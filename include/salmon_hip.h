@@ -326,8 +326,10 @@ int salmon_hip_update_potential(salmon_hip_t h, const double *rho_dev, const dou
  *   batch_prepare: Taylor coefficients; builds the tile lists, descriptor tables and
  *     the packed launches' records, sets the step counter to 1.
  *   batch_autotune: times the packed stencil for each candidate (z-chunks per orbital:
- *     the rule, 1 or 2; persistent blocks, where the stencil's form is a persistent
- *     kernel: 256, 512, 1024, 2048 or one per tile) and keeps the fastest; *choice = 100*z + blocks/256 (99 = one per tile).
+ *     the rule, 1 or 2; persistent blocks, where a middle term's form is a persistent
+ *     kernel (rows above 64 points): 256, 512, 1024, 2048 or one per tile, else the 1024 that
+ *     a new batch has) and keeps the fastest; *choice = 100*z + blocks/256 of the persistent
+ *     launches (99 = one per tile, also where no launch of the step is persistent).
  *   batch_step: enqueue one step; SALMON_HIP_EINVAL once the step counter has passed the
  *     shortest system's nt (the field tables end there).
  *   batch_set_time: set the step counter (1 .. nt_min + 1).

@@ -5142,8 +5142,13 @@ int salmon_hip_batch_autotune(salmon_hip_batch_t b, int reps, int *choice, doubl
   double best = 1e30;
   int bz = 0, bg = 4;
   int rc = 0;
+  // the persistent grid matters only to groups outside the delayed-z form (one block per tile there); without
+  // such a group the timed terms are the same launch for every grid, and the default stays
+  bool mid = false, last = b->n_hamil - 1 > kTilezComb;  // persistent middle terms; last terms
+  for (const auto &g : b->groups) mid = mid || g.zch == 0;
+  const std::vector<int> grids = mid ? std::vector<int>{1, 2, 4, 8, 1 << 20} : std::vector<int>{bg};
   for (int z : {0, 1, 2}) {
-    for (int gm : {1, 2, 4, 8, 1 << 20}) {
+    for (int gm : grids) {
       b->z_chunks = z;
       b->grid_mult = gm;
       if ((rc = batch_tables(b))) break;
@@ -5167,7 +5172,7 @@ int salmon_hip_batch_autotune(salmon_hip_batch_t b, int reps, int *choice, doubl
   b->z_chunks = bz;
   b->grid_mult = bg;
   if (int rc2 = batch_tables(b)) return rc2;
-  if (choice) *choice = 100 * bz + (bg > 64 ? 99 : bg);
+  if (choice) *choice = 100 * bz + (bg > 64 || !(mid || last) ? 99 : bg);
   if (best_ms) *best_ms = best;
   return 0;
 }

@@ -54,3 +54,39 @@ def test_autotune_then_step(oracle_lib, kw, whole):
     e = np.abs(first[0].cpu().numpy()[..., : s.ny, :] - ref).max() / np.abs(ref).max()
     assert e <= 1e-12
     h.close()
+
+
+# (extents, order, whether some launch of the step is a persistent one): rows of up to 64 points take one block per
+# tile in every term up to order 4; above that the last term is persistent, and rows above 64 points always are
+@pytest.mark.parametrize("ns,order,persistent", [
+    (((12, 11, 13), (20, 16, 24)), 4, False),
+    (((12, 11, 13), (20, 16, 24)), 5, True),
+    (((12, 11, 13), (66, 8, 9)), 4, True),
+    (((66, 8, 9), (130, 6, 10), (13, 8, 9)), 2, True),
+    (((66, 8, 9), (128, 6, 10), (13, 8, 9)), 5, True),
+])
+def test_batch_autotune(oracle_lib, ns, order, persistent):
+    """The batched step on either side of its persistent form, before and after tuning: the tuner's grid choice
+    where there is one to make, and every member's series against the oracle (1e-9, the series bar)."""
+    from salmon2_amd.batch import BatchRunner
+
+    print(f"[gpu] batch autotune {ns} order {order}", flush=True)
+    nt = 3
+    systems = [system.make_si_system(ncell=(6, 1, 1) if n[0] > 64 else (1, 1, 1), n=n, no=3, rcut=1.8, n_hamil=order,
+                                     seed=510 + i, nt=nt) for i, n in enumerate(ns)]
+    br = BatchRunner(systems, nt)
+    refs = []
+    for s in systems:
+        _, cur, dip, rne = oracle_lib.Oracle(s).rt_run(nt=nt, psi=s.psi)
+        refs.append(dict(curr=cur, dip=dip, rne=rne))
+    for tuned in (False, True):
+        if tuned:
+            choice, ms = br.batch.autotune(reps=2)
+            assert ms > 0.0 and (choice % 100 != 99 or any(n[0] > 64 for n in ns)) == persistent
+            br.reset()
+        br.run(nt)
+        for g, ref in zip(br.results(nt), refs):
+            for k in ref:
+                e = np.abs(np.asarray(g[k]) - ref[k]).max() / np.abs(ref[k]).max()
+                assert e <= 1e-9, (tuned, k, e)
+    br.close()
