@@ -721,7 +721,10 @@ struct salmon_unet {
   bf16_t *x0 = nullptr, *act[12] = {};
   bf16_t *d_zero = nullptr;  // kConvZero zeros: the operands of k_conv outside the grid or past K
   // backward work
-  float *d_out = nullptr, *d_dout = nullptr, *d_part = nullptr, *d_fx = nullptr, *d_wpart = nullptr;
+  float *d_out = nullptr, *d_dout = nullptr, *d_part = nullptr;
+  // the weight gradients run last: their operands and partial sums lie where the data gradients (d_fx with
+  // d_xt) and, once packed, the layers' gradients (g with d_wpart) lay
+  float *d_fx = nullptr, *d_wpart = nullptr;
   bf16_t *g[10] = {};        // pre-activation gradient of each layer
   bf16_t *d_xt = nullptr, *d_gt = nullptr;  // channel-major operands of the weight gradient
   size_t fx_n = 0;
@@ -1011,7 +1014,7 @@ int salmon_unet_create(int nx, int ny, int nz, unsigned long long seed, salmon_u
     if ((rc = ualloc(u, &u->act[i], act_n[i]))) return bail(rc);
   // d_fx: data gradient (max np * ci) followed by the two kept skip gradients (n0 x 48, n1 x 96)
   u->fx_n = std::max({n0 * 48, n1 * 96, n2 * 64, n1 * 32, n0 * 16});
-  size_t wp = 0, xt = 0, gt = 0;
+  size_t wp = 0, xt = 0, gt = 0, gl = 0;
   for (Layer &l : u->L) {
     const size_t ci = l.c1 + l.c2, np = u->np[l.level];
     l.part_off = wp;
@@ -1020,14 +1023,22 @@ int salmon_unet_create(int nx, int ny, int nz, unsigned long long seed, salmon_u
     wp += (np + kWgChunk - 1) / kWgChunk * 27 * l.co * ci;
     xt += 3 * ci * wg_pad(np);
     gt += l.co * wg_pad(np);
+    gl += l.co * np;
   }
+  const size_t fx_all = u->fx_n + n0 * 48 + n1 * 96;
+  float *data, *grad;
   if ((rc = ualloc(u, &u->d_out, n0)) || (rc = ualloc(u, &u->d_dout, n0)) || (rc = ualloc(u, &u->d_part, blocks(n0))) ||
-      (rc = ualloc(u, &u->d_fx, u->fx_n + n0 * 48 + n1 * 96)) ||
-      (rc = ualloc(u, &u->d_wpart, wp)) || (rc = ualloc(u, &u->d_xt, xt)) || (rc = ualloc(u, &u->d_gt, gt)) ||
-      (rc = ualloc(u, &u->d_rpart, 1024)))
+      (rc = ualloc(u, &data, std::max(fx_all, (xt + 1) / 2))) || (rc = ualloc(u, &grad, std::max(wp, (gl + 1) / 2))) ||
+      (rc = ualloc(u, &u->d_gt, gt)) || (rc = ualloc(u, &u->d_rpart, 1024)))
     return bail(rc);
-  for (int li = 0; li < 10; ++li)
-    if ((rc = ualloc(u, &u->g[li], u->np[u->L[li].level] * u->L[li].co))) return bail(rc);
+  u->d_fx = data;
+  u->d_xt = (bf16_t *)data;
+  u->d_wpart = grad;
+  gl = 0;
+  for (int li = 0; li < 10; ++li) {  // (each a whole number of 32 bytes: co is a multiple of 16)
+    u->g[li] = (bf16_t *)grad + gl;
+    gl += u->np[u->L[li].level] * u->L[li].co;
+  }
   // He-normal weights, zero biases; head: small normal weights, zero bias
   std::vector<float> w(off, 0.f);
   std::mt19937_64 gen(seed);
