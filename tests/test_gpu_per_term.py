@@ -113,3 +113,92 @@ def test_phase_table_blocks(oracle_lib, nk, lmax, whole):
     h.hpsi(psi, out)
     assert rel(out.cpu().numpy()[..., : s.ny, :], O.hpsi(A, s.psi)[..., : s.ny, :]) <= 1e-12
     h.close()
+
+
+# points covered by up to two and up to ten (atom, point) pairs, and up to 16 projectors per atom
+@pytest.mark.parametrize("kw", [
+    dict(n=12, no=4, nkgrid=(1, 1, 2), rcut=3.6, seed=23),
+    dict(n=12, no=4, nkgrid=(1, 1, 2), rcut=5.3, seed=23),
+    dict(n=12, no=9, rcut=5.3, lmax=2, seed=23),
+    dict(n=14, no=5, nkgrid=(1, 1, 2), seed=59, lmax=3),
+    dict(n=12, no=17, rcut=5.3, lmax=3, seed=61),
+])
+def test_covered_points(oracle_lib, kw):
+    import torch
+
+    print(f"[gpu] per-term covered points {kw}", flush=True)
+    s = system.make_si_system(**kw)
+    check_step(oracle_lib, s, str(kw))
+    h = per_term(s)
+    psi = torch.from_numpy(s.psi).cuda()
+    cur = torch.zeros((s.nspin, 3), dtype=torch.float64, device="cuda")
+    h.current(A, psi, cur)
+    O = oracle_lib.Oracle(s)
+    O.update_kvector(A)
+    assert rel(cur.cpu().numpy(), O.current(A, s.psi)) <= 1e-9
+    h.close()
+
+
+@pytest.mark.parametrize("n_hamil", [1, 2, 3, 5, 6])
+def test_orders(oracle_lib, n_hamil):
+    """Chains of 0 .. 5 fused KB passes."""
+    print(f"[gpu] per-term order {n_hamil}", flush=True)
+    check_step(oracle_lib, system.make_si_system(n=12, no=4, nkgrid=(1, 1, 2), rcut=3.6, seed=29, n_hamil=n_hamil),
+               f"order {n_hamil}")
+
+
+@pytest.mark.parametrize("lmax", [1, 3])
+def test_prepared_projection(lmax):
+    """current_next's projection of psi is the one that the next step uses, bit for bit, and is discarded under
+    any other field than the one it was formed for."""
+    import torch
+
+    from salmon2_amd.hip import Handle
+
+    print(f"[gpu] per-term prepared projection lmax={lmax}", flush=True)
+    s = system.make_si_system(n=12, no=4, nkgrid=(1, 1, 2), lmax=lmax, seed=7)
+    h = Handle(s, stream=torch.cuda.current_stream())
+    h._set_shape(0, 0)
+    psi = torch.from_numpy(s.psi).cuda()
+    cur = torch.zeros(3 * s.nspin, dtype=torch.float64, device="cuda")
+    B = np.array([0.02, -0.01, 0.0])
+
+    def step():
+        out, work = torch.zeros_like(psi), torch.zeros_like(psi)
+        h.prof_start(64)
+        h.taylor(s.zc(), psi, out, work)
+        n = h.prof_read("proj")[1]
+        h.prof_end()
+        return n, out
+
+    h.update_kvector(A)
+    n, plain = step()
+    assert n == 1  # the first term's projection; the others are fused with the KB pass before
+    h.update_kvector(B)
+    h.current_next(B, psi, cur, A)
+    h.update_kvector(A)
+    n, out = step()
+    assert n == 0 and torch.equal(out, plain)
+    h.current_next(A, psi, cur, B)
+    h.update_kvector(A)
+    n, out = step()
+    assert n == 1 and torch.equal(out, plain)
+    h.close()
+
+
+@pytest.mark.parametrize("name,kw", [("tiny", dict()), ("c1", dict()), ("c1", dict(scf=True, pc=True))])
+def test_fused_current_equals_unfused(name, kw):
+    """The RT step with current_next's gather and without it, bit for bit."""
+    from salmon2_amd.rt import RTPropagator
+
+    print(f"[gpu] per-term current_next {name} {kw}", flush=True)
+    s = system.config(name)
+    r = []
+    for fuse in (False, True):
+        p = RTPropagator(s, fuse_current=fuse, **kw)
+        p.h._set_shape(0, 0)
+        r.append((p.run(8), p.psi_a.cpu().numpy()))
+        p.close()
+    for k in ("curr", "dip", "rne"):
+        assert np.array_equal(r[0][0][k], r[1][0][k]), k
+    assert np.array_equal(r[0][1], r[1][1])
