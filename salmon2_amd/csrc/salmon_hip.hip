@@ -3620,34 +3620,60 @@ static bool small_fits(const salmon_hip_ctx *c) {
   return small_shape(c).cls >= 0;
 }
 
-// Where the per-term kernels are the faster ones on such a grid: a block reads all projector values of its
-// orbital (kbval) in every term, k_proj and k_proj_scatter once for 16 or 64 orbitals, and spread over more
-// blocks with more atoms.  Up to one orbital per CU the whole-orbital step always won or tied; with few values it
-// keeps that for any number of orbitals.  Measured, one Taylor step of order 4, whole orbital against per term:
-// 16^3, 8 atoms of 9 projectors (18 000 values), 4096 orbitals 1369 and 1385 us; 18^3, 9 projectors (26 000), 1024
-// orbitals 757 and 807 us, 2048 1573 and 1239 us; 12^3, 16 projectors (56 000), 512 orbitals 620 and 794 us, 2048
-// 2336 and 1320 us; 12 x 12 x 24, 16 atoms of 16 (24 000), 768 orbitals 324 and 342 us, 2048 885 and 759 us.  Half of
-// that with more than eight atoms where one block fills a CU's LDS: 10 x 20 x 30, 16 atoms of 9 (26 000), 512
-// orbitals 423 and 428 us, 768 635 and 522 us.
-static bool small_one_per_cu(const salmon_hip_ctx *c) { return c->natom > 8 && small_shape(c).lds > 80 * 1024; }
-
-static bool small_step(const salmon_hip_ctx *c, int n_hamil) {
-  if (!small_fits(c)) return false;
-  return c->norb <= 256 || c->kbval <= 21e3 ||
-         (double)c->norb * c->kbval * c->natom <= (small_one_per_cu(c) ? 47e6 : 94e6) * n_hamil;
+// What a block of the whole-orbital kernels walks one after another in a KB pass: for the busiest wave, 64-point
+// pieces of its atoms' spheres times groups of four projectors (with more than four, the points are completed in a
+// pass of their own).
+static double small_chain(const salmon_hip_ctx *c, const SmallShape &s) {
+  if (c->natom == 0) return 0.0;
+  const int ngroup = s.bs / 64 / s.nsub, pts = (int)std::ceil(c->kbval / c->nlma);
+  const double pieces = (double)((c->natom + ngroup - 1) / ngroup) * ((pts + 64 * s.nsub - 1) / (64 * s.nsub));
+  return pieces * ((c->cmax + 3) / 4 + (c->cmax > 4 ? 0.25 * c->cmax : 0.0));
 }
 
-// One application alone: the per-term kernels' three launches are worth their cost above about a thousand
-// orbitals (16^3, 1024 orbitals: 93 us in one launch, 112 per term; 15x17x14, 1600 orbitals: 150 and 126;
-// 12x12x24, 2048 orbitals: 171 and 158), with many projector values or atoms earlier (18^3, 26 000 values, 512
-// orbitals 120 and 147 us, 1024 235 and 200 us; 14 x 13 x 15, 86 000, 256 orbitals 148 and 172 us, 320 261 and
-// 182 us), and beyond one orbital per CU where no second block fits its LDS and 16 atoms fill the projections
-// (10 x 20 x 30, 320 orbitals 106 and 64 us).
+// More than six planes per thread in 768 threads: the registers spill.
+static bool small_spills(const SmallShape &s) { return kSmallClass[s.cls].bsmax == 768 && s.ppt > 6; }
+
+// Where the whole-orbital step is the faster one on such a grid. A block reads all projector values of its orbital
+// (kbval) in every term, k_proj and k_proj_scatter once for 16 or 64 orbitals, and the latter spread over more
+// blocks with more atoms. Up to one orbital per CU, and with few values for any number of orbitals, one block per
+// orbital won or tied wherever measured; else the line is drawn through 856 random cells (8 to 32 atoms of 1 to 16
+// projectors, 240 to 4500 orbitals), of which 15 end 4 to 20% behind the better form; orders 2 and 3, whose
+// orbitals are read and written for fewer terms, a little earlier (156 cells). Order 4, whole orbital against per
+// term: 16^3, 8 atoms of 9 projectors (18 000 values), 4096 orbitals 1369 and 1385 us; 18^3, 9 projectors (26
+// 000), 1024 orbitals 757 and 807 us, 2048 1573 and 1239 us; 12^3, 16 projectors (56 000), 512 orbitals 620 and
+// 794 us, 2048 2336 and 1320 us; 12 x 12 x 24, 16 atoms of 16 (112 000), 320 orbitals 1310 and 718 us, 2048 6485
+// and 2461 us.
+static bool small_step(const salmon_hip_ctx *c, int n_hamil) {
+  if (!small_fits(c)) return false;
+  const double f = std::min(1.0, 0.3 + 0.175 * n_hamil);
+  if (c->norb <= 256 || c->kbval <= 19e3 * f) return true;
+  const SmallShape s = small_shape(c);
+  return c->norb * std::sqrt(c->kbval * small_chain(c, s) * c->natom / 8) * (small_spills(s) ? 1.25 : 1.0) <= 1.44e6 * f;
+}
+
+// One application alone, whose three per-term launches are worth their cost above about a thousand orbitals
+// (16^3, 1024 orbitals: 93 us in one launch, 112 per term; 15x17x14, 1600 orbitals: 150 and 126; 12x12x24, 2048
+// orbitals: 171 and 158) and with many projector values or atoms earlier (18^3, 26 000 values, 512 orbitals 120
+// and 147 us, 1024 235 and 200 us; 14 x 13 x 15, 86 000, 256 orbitals 148 and 172 us, 320 261 and 182 us; 10 x 20 x
+// 30, 16 atoms, 320 orbitals 106 and 64 us).  Both forms' times in us, each within 10% (rms) of 538 random cells:
+// one block costs its points, its shared points' projectors and its chain, per orbital and CU or round of
+// resident blocks, and its projector values in the L2; the launches cost the points of all
+// orbitals, the rounds of k_proj's blocks (32 sphere points at a time) and the gathers.
 static bool small_hpsi(const salmon_hip_ctx *c) {
   if (c->norb > 1024 || !small_fits(c)) return false;
-  if (c->norb <= 256) return true;
-  if (small_one_per_cu(c)) return false;
-  return (double)c->norb * c->kbval * c->natom <= 196e6;
+  if (c->norb <= 256 || c->natom == 0) return true;
+  const SmallShape s = small_shape(c);
+  const int waves = s.bs / 64, percu = (c->norb + 255) / 256;
+  const int blocks = std::min(std::max(1, 4 * kSmallClass[s.cls].minw / waves), (int)std::max<size_t>(1, (160 * 1024) / s.lds));
+  const int rounds = (percu + blocks - 1) / blocks;
+  const double values = 1e-6 * c->norb * c->kbval, pts = c->kbval / c->nlma;
+  const double whole = 5.0 + percu * (4.1e-3 * c->ngrid + 1.4e-3 * c->ntp_shared * c->cmax +
+                                      (small_spills(s) ? 0.076 * waves * s.ppt : 0.0)) +
+                       0.32 * rounds * small_chain(c, s) + 1.9 * values;
+  const int pblk = c->natom * c->nk * ((c->nb + 63) / 64);
+  const double terms = 25.0 + 14e-6 * c->norb * c->ngrid + 3.6e-6 * c->norb * c->natom * pts + 1.2 * values +
+                       (c->cmax > 4 ? 4.9 * ((pblk + 511) / 512) * std::ceil(pts / 32) : 0.0);
+  return whole <= 1.08 * terms;
 }
 
 static SmallArgs small_args(salmon_hip_t c, const void *psi, void *out, void *h1) {
@@ -4064,14 +4090,19 @@ static bool small_current_args(salmon_hip_t c, const void *psi, const CurFinArgs
   return small_current_lds(c, a.nsub) <= kSmallLds;
 }
 
-// The whole-orbital current: alone on a CU it is bound by the local part's LDS reads and by an orbital's moments,
-// which the per-term kernels spread over the chip once the orbitals are many.  Measured, whole orbital
-// against per term: 16^3, 2048 orbitals of 4, 9 and 16 projectors per atom 81 and 83, 113 and 126, 146 and 159 us,
-// 4096 orbitals 166 and 146, 241 and 172, 319 and 208 us; 18^3, 1024 orbitals of 9 103 and 133 us, 2048 225 and
-// 194 us; up to 3456 points with up to 4 projectors it stays ahead (12^3, 4096 orbitals 77 and 101 us).
+// Where the whole-orbital current is the faster one: a block walks its orbital's points and its atoms' spheres (two
+// projectors at a time), which the per-term kernels spread over the chip once the orbitals are many.  The line is
+// drawn through 828 random cells (5 of them left more than 5% slower).  Whole orbital against per term: 16^3, 2048
+// orbitals of 4, 9 and 16 projectors per atom 81 and 83, 113 and 126, 146 and 159 us, 4096 166 and 146, 241 and 172,
+// 319 and 208 us; 18^3, 16 projectors, 1024 orbitals 136 and 172 us, 4096 647 and 335 us; 12^3, 4 projectors, 4096
+// orbitals 77 and 101 us.
 static bool small_current(const salmon_hip_ctx *c) {
   if (!small_fits(c)) return false;
-  return (double)c->norb * c->ngrid <= 8.5e6 || (c->cmax <= 4 && c->ngrid <= 3500);
+  if (c->natom == 0) return true;
+  const int nsub = std::max(1, kSmallCurBs / 64 / c->natom), ngroup = kSmallCurBs / 64 / nsub;
+  const int pts = (int)std::ceil(c->kbval / c->nlma);
+  const double chain = (double)((c->natom + ngroup - 1) / ngroup) * ((pts + 64 * nsub - 1) / (64 * nsub)) * ((c->cmax + 1) / 2);
+  return c->norb * std::sqrt(chain) * c->ngrid * c->natom / 8 <= 1e8;
 }
 
 static int launch_current_small(salmon_hip_t c, const SmallCurArgs &a) {

@@ -22,7 +22,7 @@ def _step(h, s, psi):
 @pytest.mark.parametrize("kw,whole", [
     (dict(n=(12, 11, 13), no=3), True),                                # an orbital per block
     (dict(n=(26, 20, 31), no=3), False),                               # too large for that
-    (dict(n=10, lmax=3, rcut=5.3, no=41, nkgrid=(1, 4, 4)), False),    # fits, but too many orbitals
+    (dict(n=10, lmax=3, rcut=5.3, no=64, nkgrid=(1, 4, 4)), False),    # fits, but too many orbitals
 ])
 def test_autotune_then_step(oracle_lib, kw, whole):
     import torch
