@@ -233,8 +233,9 @@ int salmon_hip_current(salmon_hip_t h, const double *vec_Ac, const void *psi, do
  * orbitals twice).  The next salmon_hip_update_kvector whose field equals vec_Ac_next bit
  * for bit takes that table instead of building it, and the next salmon_hip_taylor /
  * salmon_hip_hpsi of psi takes that projection instead of forming it; any other
- * update_kvector, projection or fused KB pass on the handle discards them.  psi must not
- * change in between.  Results equal the unfused sequence bit for bit.  Not for handles of
+ * update_kvector, projection or fused KB pass on the handle discards them.  Where the step or
+ * the current of a small grid runs one orbital per block, no projection is prepared and the
+ * step forms its own.  psi must not change in between.  Results equal the unfused sequence bit for bit.  Not for handles of
  * a batch (SALMON_HIP_ESTATE).
  */
 int salmon_hip_current_next(salmon_hip_t h, const double *vec_Ac, const void *psi, double *curr_dev,

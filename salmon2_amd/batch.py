@@ -2,7 +2,7 @@
 
 Each system has its own Handle (grid, orbitals, projectors, fixed V_local) and its
 own pulse; the batch runs the fixed-potential RT step for all of them with one
-persistent stencil kernel per halo class and per Taylor term, one packed launch
+stencil launch per halo class and per Taylor term, one packed launch
 per phase for all systems (phase table, projections, fused KB passes, scatter,
 density, current, dipole), and A(t) tables and the step counter on the device.
 Launches are eager: the library's graph capture of the batched step is switched

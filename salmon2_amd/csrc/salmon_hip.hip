@@ -255,7 +255,8 @@ __device__ __forceinline__ int xcd_order(int b, int nblk) {
 // 512 orbitals at 96 x 14 x 12: 79 us split, 57 us not; s+p projectors, 1024 orbitals at 32^3: 187 us split
 // and 202 us not for the fused pass, 128 orbitals there 14 us and 21 us for the projection).  Handles of
 // the mixed precision keep the points in one sequence (fused pass of 216 atoms, 1728 orbitals 985 us, 953 us
-// split): what is rounded to FP32 after it must not depend on how the sum is grouped.  One handle's
+// split), for reproducibility: what is rounded to FP32 after the sum then stays bit for bit what it was before
+// the split (either way 5e-8 from FP64 on that case).  One handle's
 // forms all sum a projection in one order (the chunks of S = 4 are of one length).
 constexpr int proj_split(int lm, bool mixed) { return lm <= 4 && !mixed ? 4 : 1; }
 constexpr int proj_orb(int split) { return split == 4 ? 16 : kProjOrb; }
@@ -4646,18 +4647,11 @@ void batch_buffers(salmon_hip_batch *b, int i, int p, void **hh, void **out) {
 // (re)build tile lists and descriptor tables for the current z_chunks / grid_mult
 int batch_tables(salmon_hip_batch *b) {
   for (auto &g : b->groups) {
-    // the terms without the Taylor sum run on the delayed-z tiles when every member's rows fit
-    // their slots (nx <= 64; the group takes its largest member's chunk count) and its z extent
-    // is a multiple of 4; z chunks are then rounded up to whole multiples of 4 planes
-    int zch = 0;
-    bool zok = g.hc <= 2;
-    for (int i : g.mem) {
-      const salmon_hip_t c = b->h[i];
-      zok = zok && c->nx <= 64 && c->TY * c->nx <= kTile &&
-            (c->TY + 8) * c->nx <= 3 * kTile;
-      zch = std::max(zch, tilez_chunks(c->TY, c->nx));
-    }
-    g.zch = zok ? zch : 0;
+    // rows of up to 64 points (hc <= 2) run on the delayed-z tiles, whose slots they fit, with any number of
+    // planes (the last term up to order 4); the group takes its largest member's chunk count
+    g.zch = 0;
+    if (g.hc <= 2)
+      for (int i : g.mem) g.zch = std::max(g.zch, tilez_chunks(b->h[i]->TY, b->h[i]->nx));
     // the members' common number of z chunks by tilez_zchunks' measure of the whole group
     int gz = 1;
     double tbest = 0.0;

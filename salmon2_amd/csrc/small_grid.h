@@ -1,16 +1,19 @@
 // Whole-orbital kernels for small grids (included by salmon_hip.hip inside its namespace).
 //
-// An orbital block of up to ~9000 points (one 8-atom cell: 12^3 .. 18^3) fits the 160 KB of LDS of
-// one CU, so the complete Taylor step of an orbital -- every stencil application, KB projection,
+// An orbital block of up to 7680 points (one 8-atom cell: 12^3 .. 18^3; the most that the launch classes' threads
+// and planes cover) fits the 160 KB of LDS of one CU, so the complete Taylor step of an orbital -- every stencil application, KB projection,
 // KB scatter and the Taylor sum -- runs in ONE workgroup without leaving the CU: the orbital is read
 // once and written once (plus H psi), instead of one stencil, one projection and one scatter launch
 // per term.  Orbitals do not couple inside a Taylor step, so no block waits for another.
 //
-// Bound by the CU's LDS reads in the stencil (17 per point: 11 to 13 cycles per wave read against the 8
-// of 128 bytes a cycle) and by the latency of the KB tables between the barriers.  Measured, one Taylor
-// step of order 4 (per-term kernels -> here): 16^3 x 16 orbitals 145 -> 51 us, 12^3 x 1024 225 -> 94 us,
-// 16^3 x 1024 446 -> 229 us, 18^3 x 1024 700 -> 428 us; the current: 16^3 x 16 118 -> 13 us, 12^3 x 1024
-// 85 -> 24 us.
+// Half of it is the stencil (17 LDS reads per point, 11 to 13 cycles per wave read against the 8 of 128 bytes a
+// cycle, beside the FP64 sums), a third the latency of the KB tables between the barriers, the rest loads and
+// stores: 12^3 x 1024 orbitals 90 us = 48 for the four applications + 26 for the KB passes + 16; 16^3 x 16
+// 52 us = 27 + 19 + 6 (orders 1 to 4 with and without projectors).  Measured, one Taylor
+// step of order 4 (per-term kernels -> here): 16^3 x 16 orbitals 145 -> 52 us, 12^3 x 1024 225 -> 90 us,
+// 16^3 x 1024 446 -> 223 us, 18^3 x 1024 700 -> 428 us; the current: 16^3 x 16 118 -> 13 us, 12^3 x 1024
+// 85 -> 24 us.  Where many orbitals carry many projector values the per-term kernels are the faster ones
+// (small_step, small_hpsi, small_current).
 
 // ---------------------------------------------------------------------------
 // Work split: thread t owns the column (x, y) = t % (nx ny) over PPT consecutive planes from
